@@ -297,6 +297,25 @@ int qq_quest_forward_decode_phase(const void* q, int q_dtype, int64_t q_batch_st
                                   int64_t workspace_bytes, void* sync, int64_t sync_bytes, int phase,
                                   void* stream);
 
+/* Replaces AttentionBackend.forward_extend's per-request loop (src/qwenquest/attention/
+ * base.py:65-93, attention/ops.py:18-45) for one layer, the new K/V being in the pool:
+ * request i's extend_lens[i] new tokens (q [n, H, 128] bf16, request after request)
+ * attend positions 0 .. prefix_lens[i] + t of req_to_token[req_pool_indices[i],
+ * 0 .. seq_lens[i]) -> out [n, H*128] bf16.  The lengths are read on the device only.
+ * bf16, head_dim 128, H divisible by KV, scale > 0 (QQ_EINVAL otherwise); scores,
+ * weights and sums in fp32.  A request whose index or a row of which lies outside its
+ * table gets NaN, as do rows of q past the requests' tokens.  workspace >=
+ * qq_extend_attention_workspace_bytes(n, bs, H, KV, req_to_token_stride): (m, l, o)
+ * partials, when few query rows meet a wide table. */
+int qq_extend_attention(const void* q, int num_q_heads, const void* k_layer, const void* v_layer,
+                        int64_t kv_rows, int kv_heads, int head_dim, const int32_t* req_to_token,
+                        int64_t req_to_token_stride, int64_t req_to_token_rows,
+                        const int64_t* req_pool_indices, const int64_t* seq_lens,
+                        const int64_t* prefix_lens, const int64_t* extend_lens, int bs, int64_t n,
+                        float scale, void* out, void* workspace, int64_t workspace_bytes, void* stream);
+int64_t qq_extend_attention_workspace_bytes(int64_t n, int bs, int num_q_heads, int kv_heads,
+                                            int64_t max_rows);
+
 /* Replaces DenseBackend.forward_decode (src/qwenquest/attention/dense.py:26-42) for
  * one layer: the new tokens' K/V (k_new/v_new [bs, KV, D]; NULL: none) go to rows
  * out_cache_loc (memory.py:114-120), then request i attends

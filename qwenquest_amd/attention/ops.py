@@ -1,8 +1,9 @@
 """Attention math (reference ``src/qwenquest/attention/ops.py``).
 
 ``decode_attention`` runs the HIP split-K kernel over an explicit row list;
-``extend_attention`` (dense causal prefill) is outside the accelerated path and
-uses torch's SDPA on the device, in float32.
+``extend_attention_batch`` runs a whole prefill batch (bf16, head_dim 128) in the HIP
+prefill kernel; ``extend_attention``, one request of any shape, uses torch's SDPA on the
+device, in float32.
 """
 
 from __future__ import annotations
@@ -12,7 +13,7 @@ import torch.nn.functional as F
 
 from qwenquest_amd import _lib
 
-__all__ = ["decode_attention", "extend_attention", "AttentionWorkspace"]
+__all__ = ["decode_attention", "extend_attention", "extend_attention_batch", "AttentionWorkspace"]
 
 
 class AttentionWorkspace:
@@ -100,3 +101,37 @@ def extend_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, prefix_l
     mask = torch.arange(kv_len, device=q.device).unsqueeze(0) <= q_pos.unsqueeze(1)
     out = F.scaled_dot_product_attention(qh.contiguous(), kh, vh, attn_mask=mask, scale=scaling)
     return out[0].transpose(0, 1).reshape(n, num_heads * head_dim).to(q.dtype)
+
+
+def extend_attention_batch(
+    q: torch.Tensor,
+    k_buf: torch.Tensor,
+    v_buf: torch.Tensor,
+    req_to_token: torch.Tensor,
+    req_pool_indices: torch.Tensor,
+    seq_lens: torch.Tensor,
+    prefix_lens: torch.Tensor,
+    extend_lens: torch.Tensor,
+    scaling: float,
+) -> torch.Tensor:
+    """Dense causal prefill of a batch (the loop of base.py:65-93): ``q [n, H, 128]`` holds the
+    requests' new tokens one request after the other, ``k_buf``/``v_buf [rows, KV, 128]`` the
+    pool with the new K/V in it.  bf16; returns ``[n, H*128]``.  No host synchronisation."""
+    n, heads, dim = q.shape
+    kv, bs, dev = k_buf.shape[1], int(req_pool_indices.shape[0]), q.device
+    q = q.contiguous()
+
+    def lens(t: torch.Tensor) -> torch.Tensor:
+        return t.to(device=dev, dtype=torch.int64).contiguous()
+
+    rpi, seq, prefix, ext = lens(req_pool_indices), lens(seq_lens), lens(prefix_lens), lens(extend_lens)
+    need = int(_lib.load().qq_extend_attention_workspace_bytes(n, bs, heads, kv, req_to_token.shape[1]))
+    ws = torch.empty(need, dtype=torch.uint8, device=dev) if need else None
+    out = torch.empty((n, heads * dim), dtype=q.dtype, device=dev)
+    _lib.call(
+        "qq_extend_attention", _lib.ptr(q), heads, _lib.ptr(k_buf), _lib.ptr(v_buf), k_buf.shape[0], kv, dim,
+        _lib.ptr(req_to_token), req_to_token.stride(0), req_to_token.shape[0], _lib.ptr(rpi), _lib.ptr(seq),
+        _lib.ptr(prefix), _lib.ptr(ext), bs, n, float(scaling), _lib.ptr(out), _lib.ptr(ws), need,
+        _lib.stream(dev),
+    )
+    return out

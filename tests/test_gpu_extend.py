@@ -1,0 +1,151 @@
+"""Batched prefill attention (reference ``src/qwenquest/attention/base.py:65-93``, ops.py:18-45):
+the HIP kernel against float64 and against the request-by-request path."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DEV = torch.device("cuda", 0)
+
+
+class Layer:
+    def __init__(self, d):
+        self.layer_id, self.scaling = 0, d**-0.5
+
+
+def make(new, prefix, H, KV, seed, width=None, qscale=1.0):
+    from qwenquest_amd.attention.dense import DenseBackend
+    from qwenquest_amd.batch import ForwardBatch, ForwardMode
+    from qwenquest_amd.memory import MHATokenToKVPool, ReqToTokenPool
+
+    total = [n + p for n, p in zip(new, prefix)]
+    bs, D = len(new), 128
+    rtp = ReqToTokenPool(bs + 1, width or max(total) + 5, DEV)
+    kvp = MHATokenToKVPool(sum(total), 1, KV, D, torch.bfloat16, DEV)
+    gen = torch.Generator(device=DEV).manual_seed(seed)
+    kvp.k_all.normal_(generator=gen)
+    kvp.v_all.normal_(generator=gen)
+    perm = torch.from_numpy(np.random.default_rng(seed).permutation(sum(total)).astype(np.int32) + 1).to(DEV)
+    slots = list(range(1, bs + 1))[::-1]  # request i in table row bs - i
+    at = 0
+    for i, n in enumerate(total):
+        rtp.req_to_token[slots[i], :n] = perm[at : at + n]
+        at += n
+    be = DenseBackend(rtp, kvp)
+    loc = torch.cat([rtp.req_to_token[slots[i], p : p + n] for i, (n, p) in enumerate(zip(new, prefix))]).long()
+    n = sum(new)
+    mk = lambda h: torch.empty((n, h, D), device=DEV).normal_(generator=gen).to(torch.bfloat16)  # noqa: E731
+    q, k, v = mk(H) * qscale, mk(KV), mk(KV)
+    t = lambda x: torch.tensor(x, dtype=torch.int64, device=DEV)  # noqa: E731
+    batch = ForwardBatch(ForwardMode.EXTEND, None, None, t(slots), t(total), loc, rtp, kvp, be,
+                         extend_prefix_lens=t(prefix), extend_seq_lens=t(new))
+    return be, q, k, v, batch, Layer(D), slots
+
+
+def exact(batch, slots, q, new, prefix, KV):
+    """float64 causal attention over the pool's rows."""
+    kvp, r2t = batch.token_to_kv_pool, batch.req_to_token_pool.req_to_token
+    H, D = q.shape[1:]
+    outs, at = [], 0
+    for i, (n, p) in enumerate(zip(new, prefix)):
+        rows = r2t[slots[i], : n + p].long()
+        k, v = kvp.k_all[0][rows].double(), kvp.v_all[0][rows].double()
+        mask = torch.arange(n + p, device=DEV)[None] <= (p + torch.arange(n, device=DEV))[:, None]
+        o = torch.empty((n, H, D), dtype=torch.float64, device=DEV)
+        for h in range(H):
+            s = (q[at : at + n, h].double() @ k[:, h // (H // KV)].T.contiguous()) * D**-0.5
+            o[:, h] = torch.softmax(s.masked_fill(~mask, -float("inf")), -1) @ v[:, h // (H // KV)].contiguous()
+        outs.append(o.view(n, H * D))
+        at += n
+    return torch.cat(outs)
+
+
+def close(got, ref):
+    """Half a bf16 ulp of the result (2^-8 of it) and the fp32 sums' own error."""
+    err = (got.double() - ref).abs()
+    assert bool((err <= 2.0**-8 * ref.abs() + 1e-5).all()), float((err - 2.0**-8 * ref.abs()).max())
+
+
+@pytest.mark.parametrize("H,KV,new,prefix", [
+    (32, 4, [1], [0]),
+    (32, 4, [16], [0]),  # one block's rows
+    (32, 4, [17, 15, 1, 64], [0, 63, 64, 65]),  # edges of the query and of the K/V tile
+    (32, 4, [600], [0]),
+    (20, 4, [77, 130], [5, 0]),  # groups of 5: a tile ends inside a token
+    (28, 4, [33, 200], [0, 129]),
+    (4, 4, [129, 1], [0, 300]),  # no grouping
+    (5, 1, [300], [40]),
+    (14, 2, [190, 31], [0, 12]),
+    (64, 8, [100, 9], [64, 1]),
+    (96, 2, [21], [7]),  # 48 heads per KV head
+    (32, 4, [5], [6000]),  # few rows, long prefix: K/V splits and the merge
+    (8, 2, [3, 40], [2047, 513]),  # splits for one request, none for the other
+    (32, 4, [2, 0, 3] + [1] * 66, [1, 4, 0] + [9] * 66),  # an empty request; more than 64 requests
+])
+def test_extend_batch_matches_float64_and_the_general_path(H, KV, new, prefix, monkeypatch):
+    be, q, k, v, batch, layer, slots = make(new, prefix, H, KV, 3, width=8192 if max(prefix) > 2000 else None)
+    got = be.forward_extend(q, k, v, layer, batch)
+    assert got.shape == (sum(new), H * 128) and got.dtype == torch.bfloat16
+    close(got, exact(batch, slots, q, new, prefix, KV))
+    again = be.forward_extend(q, k, v, layer, batch)
+    assert torch.equal(got, again)
+    monkeypatch.setattr(be, "_extend_fast", lambda *a: False)
+    ref = be.forward_extend(q, k, v, layer, batch).double()
+    err = (got.double() - ref).abs()  # one rounding each, of sums 1e-5 apart
+    assert bool((err <= 2.0**-7 * ref.abs() + 2e-5).all())
+
+
+def test_extend_batch_sharp_scores_and_other_forms():
+    """Scores up to hundreds (one weight near 1, the rest tiny); lengths as CPU and int32 tensors,
+    q as a view with gaps; a captured call replays."""
+    new, prefix = [70, 130], [0, 100]
+    be, q, k, v, batch, layer, slots = make(new, prefix, 32, 4, 9, qscale=40.0)
+    got = be.forward_extend(q, k, v, layer, batch)
+    ref = exact(batch, slots, q, new, prefix, 4)
+    # an fp32 score of 400 is off by up to 2e-5, and its weight by that share
+    assert bool(((got.double() - ref).abs() <= 2.0**-8 * ref.abs() + 4e-4).all())
+    wide = torch.zeros((q.shape[0], 40, 128), dtype=q.dtype, device=DEV)
+    wide[:, :32] = q
+    batch.seq_lens, batch.req_pool_indices = batch.seq_lens.cpu(), batch.req_pool_indices.to(torch.int32)
+    batch.extend_prefix_lens = batch.extend_prefix_lens.cpu()
+    assert torch.equal(be.forward_extend(wide[:, :32], k, v, layer, batch), got)
+    batch.seq_lens, batch.extend_prefix_lens = batch.seq_lens.to(DEV), batch.extend_prefix_lens.to(DEV)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = be.forward_extend(q, k, v, layer, batch)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, got)
+
+
+def test_extend_batch_rows_outside_their_tables():
+    """A request with a row past the pool, or past the table, gets NaN; the others their answer;
+    a context longer than the table is cut to it, as a slice is."""
+    new, prefix = [40, 50, 60], [0, 30, 0]
+    be, q, k, v, batch, layer, slots = make(new, prefix, 32, 4, 5)
+    want = be.forward_extend(q, k, v, layer, batch)
+    batch.req_pool_indices[2] = 99
+    got = be.forward_extend(q, k, v, layer, batch)
+    assert torch.equal(got[:90], want[:90]) and bool(got[90:].isnan().all())
+    batch.req_pool_indices[2] = slots[2]
+    r2t = batch.req_to_token_pool.req_to_token
+    keep = int(r2t[slots[1], 10])
+    r2t[slots[1], 10] = keep - batch.token_to_kv_pool.rows  # a negative row counts from the pool's end
+    assert torch.equal(be.forward_extend(q, k, v, layer, batch), want)
+    r2t[slots[1], 10] = 1 << 20
+    got = be.forward_extend(q, k, v, layer, batch)
+    assert torch.equal(got[:40], want[:40]) and torch.equal(got[90:], want[90:])
+    assert bool(got[40:90].isnan().all())
+    r2t[slots[1], 10] = keep
+    batch.seq_lens[1] = 10_000
+    batch.extend_prefix_lens[1] = r2t.shape[1] - 50
+    r2t[slots[1], 80:] = 1
+    got = be.forward_extend(q, k, v, layer, batch)
+    batch.seq_lens[1] = r2t.shape[1]
+    assert torch.equal(be.forward_extend(q, k, v, layer, batch), got)
