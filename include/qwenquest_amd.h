@@ -198,11 +198,12 @@ int qq_quest_decode_attention(const void* q, int q_dtype, int64_t q_batch_stride
  * qq_quest_decode_attention but rows come directly from `rows` [bs, rows_stride]
  * int64 (the hot-buffer rows returned by the swap-in).  With `sync` (>=
  * qq_quest_layer_step_sync_bytes(bs, kv_heads), zeroed before the first call),
- * bf16, KV*D = 4*128, G <= 16 and rows_stride <= 4096 slots, it runs the
+ * bf16, D = 128, KV of 1, 2, 4 or 8, G <= 16 and rows_stride <= 4096 slots, it runs the
  * attention kernel of qq_quest_forward_decode's fused path over the given rows
  * (same arithmetic in the same slot order: pass `sync` exactly when
- * qq_quest_fused_step holds for the quest configuration, and quest_hisparse
- * matches quest bit for bit); otherwise chunked MFMA attention + merge, as
+ * the quest side runs its fused step - qq_quest_fused_step for
+ * qq_quest_forward_decode, qq_quest_layer_step_fused for qq_quest_layer_step -, and
+ * quest_hisparse matches quest bit for bit); otherwise chunked MFMA attention + merge, as
  * qq_quest_decode_attention. */
 int qq_decode_attention_rows(const void* q, int q_dtype, int64_t q_batch_stride, int num_q_heads,
                              const void* k_layer, const void* v_layer, int kv_dtype,
@@ -296,6 +297,24 @@ int qq_quest_forward_decode_phase(const void* q, int q_dtype, int64_t q_batch_st
                                   float* scores_ws, int32_t* positions, void* out, void* workspace,
                                   int64_t workspace_bytes, void* sync, int64_t sync_bytes, int phase,
                                   void* stream);
+
+/* qq_quest_forward_decode_phase with the two-launch step at 1, 2, 4 or 8 KV heads of
+ * 128 (qq_quest_layer_step_fused: the shapes of qq_quest_fused_step at any of these head
+ * counts); what QuestOnlyBackend runs. */
+int qq_quest_layer_step(const void* q, int q_dtype, int64_t q_batch_stride, int num_q_heads,
+                        const void* k_new, const void* v_new, int new_dtype,
+                        const int64_t* out_cache_loc, void* k_layer, void* v_layer,
+                        int kv_dtype, int64_t kv_rows, const uint16_t* page_k_bounds,
+                        int layer, const int64_t* req_pool_indices, const int64_t* seq_lens,
+                        const int32_t* candidate_limit, const int32_t* actual_lens, int bs,
+                        int max_reqs, int max_pages, int kv_heads, int head_dim,
+                        int page_size, int top_k, const int32_t* req_to_token,
+                        int64_t req_to_token_stride, int64_t req_to_token_rows, float scale,
+                        float* scores_ws, int32_t* positions, void* out, void* workspace,
+                        int64_t workspace_bytes, void* sync, int64_t sync_bytes, int phase,
+                        void* stream);
+int qq_quest_layer_step_fused(int q_dtype, int kv_dtype, int new_dtype, int num_q_heads, int kv_heads,
+                              int head_dim, int page_size, int top_k, int max_pages);
 
 /* Replaces AttentionBackend.forward_extend's per-request loop (src/qwenquest/attention/
  * base.py:65-93, attention/ops.py:18-45) for one layer, the new K/V being in the pool:

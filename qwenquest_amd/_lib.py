@@ -72,6 +72,12 @@ SIGNATURES: dict[str, tuple] = {
         [_P, _I, _L, _I, _P, _P, _I, _P, _P, _P, _I, _L, _P, _I, _P, _P, _P, _P, _I, _I, _I, _I,
          _I, _I, _I, _P, _L, _L, _F, _P, _P, _P, _P, _L, _P, _L, _I, _P],
     ),
+    "qq_quest_layer_step": (
+        _I,
+        [_P, _I, _L, _I, _P, _P, _I, _P, _P, _P, _I, _L, _P, _I, _P, _P, _P, _P, _I, _I, _I, _I,
+         _I, _I, _I, _P, _L, _L, _F, _P, _P, _P, _P, _L, _P, _L, _I, _P],
+    ),
+    "qq_quest_layer_step_fused": (_I, [_I, _I, _I, _I, _I, _I, _I, _I, _I]),
     "qq_quest_forward_decode_noalloc": (
         _I,
         [_P, _I, _L, _I, _P, _P, _I, _P, _P, _P, _I, _L, _P, _I, _P, _P, _P, _P, _I, _I, _I, _I,

@@ -56,9 +56,9 @@ def decode_attention_rows(
 
     ``rows`` ``[bs, >= max(actual_lens)]`` int64, ``k_buf``/``v_buf`` ``[rows, KV, D]``.
     Returns ``[bs, H*D]`` in q's dtype.  With ``sync`` (a zeroed uint8 buffer of at least
-    ``qq_quest_layer_step_sync_bytes`` bytes) the bf16 KV*D = 4*128 shapes run the attention
-    kernel of the fused Quest layer step, whose arithmetic QuestHiSparseBackend shares with
-    QuestOnlyBackend.
+    ``qq_quest_layer_step_sync_bytes`` bytes) the bf16 shapes with D = 128 and 1, 2, 4 or 8
+    KV heads run the attention kernel of the fused Quest layer step, whose arithmetic
+    QuestHiSparseBackend shares with QuestOnlyBackend.
     """
     bs, heads, dim = q.shape
     kv = k_buf.shape[1]

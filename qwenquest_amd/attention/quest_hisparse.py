@@ -115,7 +115,7 @@ class QuestHiSparseBackend(AttentionBackend):
         key = (q3.dtype, new_dtype, q3.shape[1])
         if key not in self._fused_cache:
             qa, pool = self.quest, self.token_to_kv_pool
-            self._fused_cache[key] = bool(_lib.load().qq_quest_fused_step(
+            self._fused_cache[key] = bool(_lib.load().qq_quest_layer_step_fused(
                 _lib.dtype_code(q3.dtype), _lib.dtype_code(pool_dtype), _lib.dtype_code(new_dtype), q3.shape[1],
                 pool.kv_heads, pool.head_dim, qa.page_size, qa.top_k, qa.max_pages_per_req))
         return self._fused_cache[key]

@@ -159,7 +159,7 @@ class QuestOnlyBackend(AttentionBackend):
         r2t = self.req_to_token
         sync = self._step_sync  # None: the four-launch path
         _lib.call(
-            "qq_quest_forward_decode_phase", _lib.ptr(q3), _lib.dtype_code(q3.dtype), q3.stride(0), heads,
+            "qq_quest_layer_step", _lib.ptr(q3), _lib.dtype_code(q3.dtype), q3.stride(0), heads,
             _lib.ptr(kn), _lib.ptr(vn), _lib.dtype_code(kn.dtype), _lib.ptr(loc), _lib.ptr(k_buf),
             _lib.ptr(v_buf), _lib.dtype_code(k_buf.dtype), k_buf.shape[0], _lib.ptr(quest.page_k_bounds),
             layer.layer_id - quest.start_layer, _lib.ptr(rpi), _lib.ptr(step.seq_lens),

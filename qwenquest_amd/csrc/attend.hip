@@ -373,8 +373,8 @@ extern "C" int qq_decode_attention_rows(const void* q, int q_dtype, int64_t q_ba
                        kv_rows, kv_heads, head_dim, actual_lens, scale, out, what);
   if (st != QQ_OK) return st;
   QQ_REQUIRE(rows && rows_stride > 0, "%s: null row list", what);
-  if (sync && q_dtype == QQ_DTYPE_BF16 && kv_dtype == QQ_DTYPE_BF16 && kv_heads == 4 && head_dim == kMfmaDim &&
-      attend_rows_fused(q, q_batch_stride, num_q_heads, k_layer, v_layer, kv_rows, rows, rows_stride, actual_lens, bs,
+  if (sync && q_dtype == QQ_DTYPE_BF16 && kv_dtype == QQ_DTYPE_BF16 && head_dim == kMfmaDim &&
+      attend_rows_fused(q, q_batch_stride, num_q_heads, k_layer, v_layer, kv_rows, kv_heads, rows, rows_stride, actual_lens, bs,
                         scale, out, workspace, workspace_bytes, sync, sync_bytes,
                         static_cast<hipStream_t>(stream)) == QQ_OK)
     return check_launch(what);

@@ -2,9 +2,9 @@
 // (reference src/qwenquest/attention/quest_only.py:132-159): store the new
 // token's K/V, select the positions, gather through req_to_token and attend.
 //
-// Fused path (bf16, KV*D = 4*128, page 64, at most 64 selected pages, at most
-// 8192 pages per request, top_k <= 4096, and a zeroed sync buffer from the
-// caller): two launches.
+// Fused path (bf16, D = 128, 4 KV heads - 1, 2, 4 or 8 through qq_quest_layer_step -,
+// page 64, at most 64 selected pages, at most 8192 pages per request, top_k <= 4096,
+// and a zeroed sync buffer from the caller): two launches.
 //   1. page scores of every long request (score_pages_fast_kernel in select.hip,
 //      one 256-thread block per (request, 32 candidate pages), all resident at
 //      once) and the new token's K/V (set_kv_buffer, memory.py:114-120).
@@ -40,7 +40,7 @@
 namespace qq {
 namespace {
 
-constexpr int kStepKV = 4;            // KV heads of the fused path (KV*D = 512)
+constexpr int kDenseKV = 4;           // KV heads of the dense decode kernel (KV*D = 512)
 constexpr int kStepMaxG = 16;
 constexpr int kMaxSelFused = 64;
 constexpr int kStepMaxTopK = 4096;
@@ -68,6 +68,7 @@ struct StepArgs {
   float* part_ml;          // [bs, KV, parts, G, 2] (m in log2 units, l)
   uint32_t* sync;
   int bs, G;
+  int kv_shift;            // log2 of the KV heads
   int parts, per_wave;     // attention blocks per (request, KV head); rows per wave
   const int64_t* rows_in;  // rows given [bs, rows_stride] (attention over given rows)
   int64_t rows_stride;
@@ -91,7 +92,7 @@ struct StepRegs {
 template <int T>
 __device__ inline void load_step(StepRegs<T>& r, const int32_t* rows, int t0, const uint16_t* kb, const uint16_t* vb,
                                  int lo, int hi) {
-  constexpr int kRow = kStepKV * kMfmaDim;
+  constexpr int kRow = kDenseKV * kMfmaDim;
 #pragma unroll
   for (int t = 0; t < T; ++t) {
     const uint16_t* kp = kb + (int64_t)rows[t0 + t * 16 + lo] * kRow + hi * 8;
@@ -194,7 +195,7 @@ __device__ inline void finish_block(const StepArgs& a, int bh, int part, float M
   const int wave = tid >> 6, lane = tid & 63;
   const int lo = lane & 15, hi = lane >> 4;
   const int parts = a.parts;
-  const int b = bh / kStepKV, h = bh - b * kStepKV;
+  const int b = bh >> a.kv_shift, h = bh - (b << a.kv_shift);
   const int G = a.G;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -354,7 +355,7 @@ __device__ inline void attend_item(const StepArgs& a, int bh, int part, unsigned
   const int tid = threadIdx.x;
   const int wave = tid >> 6, lane = tid & 63;
   const int lo = lane & 15, hi = lane >> 4;
-  const int b = bh / kStepKV, h = bh - b * kStepKV;
+  const int b = bh / kDenseKV, h = bh - b * kDenseKV;
   const int64_t s = sa.seq[b];
   const int64_t req = sa.rpi[b];
   const int top_k = sa.top_k;  // the table's width: every context fits
@@ -482,7 +483,7 @@ __global__ __launch_bounds__(64 * W, 8 / W) void quest_attend_unit_kernel(StepAr
   const int tid = threadIdx.x;
   const int wave = tid >> 6, lane = tid & 63;
   const int lo = lane & 15, hi = lane >> 4;
-  const int b = bh / kStepKV, h = bh - b * kStepKV;
+  const int b = bh >> a.kv_shift, h = bh - (b << a.kv_shift);
   const int64_t s = ROWS ? 0 : sa.seq[b];
   const int64_t req = ROWS ? 0 : sa.rpi[b];
   const int top_k = sa.top_k, k = sa.k_sel;
@@ -536,7 +537,7 @@ __global__ __launch_bounds__(64 * W, 8 / W) void quest_attend_unit_kernel(StepAr
   int32_t* pos_out = !ROWS && h == 0 && sa.positions ? sa.positions + (int64_t)b * top_k : nullptr;
   const uint16_t* kb = a.k + h * kMfmaDim;
   const uint16_t* vb = a.v + h * kMfmaDim;
-  constexpr int kRow = kStepKV * kMfmaDim;
+  const int row_shift = a.kv_shift + 7;  // KV * 128 channels per pool row
   float M = -INFINITY, L = 0.0f;
   float4_t o[8];
 #pragma unroll
@@ -569,7 +570,7 @@ __global__ __launch_bounds__(64 * W, 8 / W) void quest_attend_unit_kernel(StepAr
     uint4 vr[4][4];
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
-      const uint16_t* kp = kb + (int64_t)__shfl(r32, t * 16 + lo, 64) * kRow + hi * 8;
+      const uint16_t* kp = kb + ((int64_t)__shfl(r32, t * 16 + lo, 64) << row_shift) + hi * 8;
 #pragma unroll
       for (int ks = 0; ks < 4; ++ks) ka[t][ks] = *reinterpret_cast<const bf16x8_t*>(kp + ks * 32);
     }
@@ -577,7 +578,7 @@ __global__ __launch_bounds__(64 * W, 8 / W) void quest_attend_unit_kernel(StepAr
     for (int t = 0; t < 4; ++t)
 #pragma unroll
       for (int j = 0; j < 4; ++j)
-        vr[t][j] = *reinterpret_cast<const uint4*>(vb + (int64_t)__shfl(r32, t * 16 + hi * 4 + j, 64) * kRow + lo * 8);
+        vr[t][j] = *reinterpret_cast<const uint4*>(vb + ((int64_t)__shfl(r32, t * 16 + hi * 4 + j, 64) << row_shift) + lo * 8);
     __builtin_amdgcn_sched_barrier(0);  // all 32 loads go out before the first use of any
     // S^T[token 16t + 4hi + i][head lo] in acc[t][i]
     float4_t acc[4];
@@ -703,7 +704,7 @@ static size_t unit_smem_bytes() {
 
 template <bool ROWS, int KPT, int W>
 static void launch_unit(const StepArgs& a, hipStream_t s) {
-  const int blocks = a.bs * kStepKV * a.parts;
+  const int blocks = (a.bs << a.kv_shift) * a.parts;
   quest_attend_unit_kernel<ROWS, KPT, W><<<blocks, 64 * W, unit_smem_bytes<ROWS, KPT, W>(), s>>>(a);
 }
 
@@ -725,17 +726,37 @@ static void launch_attend_select(const StepArgs& a, int n_max, hipStream_t s) {
   else launch_unit<false, kMaxKpt, W>(a, s);  // contexts past 384K tokens at W = 4
 }
 
-// Shapes the fused layer step takes (bf16, KV*D = 4*128, G <= 16, page 64, at
-// most 64 selected pages, top_k <= 4096, at most 8192 pages per request).
+// log2 of the KV heads for the unit attention, -1 for counts it does not take: the
+// powers of two up to 8 (a pool row is KV * 128 channels, the page scores hold at
+// most 1024), so that the kernel splits (request, KV head) and addresses rows with
+// shifts.
+static int kv_shift_of(int kv_heads) {
+  return kv_heads == 1 ? 0 : kv_heads == 2 ? 1 : kv_heads == 4 ? 2 : kv_heads == 8 ? 3 : -1;
+}
+
+// Shapes the fused layer step takes (bf16, D = 128, 1, 2, 4 or 8 KV heads, G <= 16,
+// page 64, at most 64 selected pages, top_k <= 4096, at most 8192 pages per request).
 // new_dtype < 0: no new token.
-static bool fused_shape(int q_dtype, int kv_dtype, int new_dtype, int num_q_heads, int kv_heads, int head_dim,
-                        int page_size, int top_k, int max_pages) {
-  if (kv_heads != kStepKV || head_dim != kMfmaDim || num_q_heads % kv_heads != 0 || page_size != 64 ||
+// Per layer-step against the four launches: 8 KV heads at batch 8 x 32K 38.9 -> 29.3 us,
+// 2 KV heads at batch 16 x 64K 32.3 -> 23.5 us; 4 KV heads are as with constants in the
+// place of the shifts (35.5 us at batch 16 x 128K).
+static bool layer_step_shape(int q_dtype, int kv_dtype, int new_dtype, int num_q_heads, int kv_heads, int head_dim,
+                             int page_size, int top_k, int max_pages) {
+  if (kv_shift_of(kv_heads) < 0 || head_dim != kMfmaDim || num_q_heads % kv_heads != 0 || page_size != 64 ||
       top_k <= 0 || top_k % page_size != 0)
     return false;
   return q_dtype == QQ_DTYPE_BF16 && kv_dtype == QQ_DTYPE_BF16 && (new_dtype < 0 || new_dtype == QQ_DTYPE_BF16) &&
          num_q_heads / kv_heads <= kStepMaxG && top_k / page_size - 1 <= kMaxSelFused && top_k <= kStepMaxTopK &&
          max_pages <= 32 * 64 * kUnitMinWaves;
+}
+
+// Those of qq_quest_forward_decode and its variants: the same at 4 KV heads.  Their
+// callers pair them with qq_decode_attention_rows by qq_quest_fused_step, so the head
+// counts at which they fuse are fixed; qq_quest_layer_step takes the others.
+static bool fused_shape(int q_dtype, int kv_dtype, int new_dtype, int num_q_heads, int kv_heads, int head_dim,
+                        int page_size, int top_k, int max_pages) {
+  return kv_heads == 4 && layer_step_shape(q_dtype, kv_dtype, new_dtype, num_q_heads, kv_heads, head_dim, page_size,
+                                           top_k, max_pages);
 }
 
 // Launch shape of the unit attention: W waves per block, `parts` blocks per (request,
@@ -754,8 +775,8 @@ static bool fused_shape(int q_dtype, int kv_dtype, int new_dtype, int num_q_head
 struct UnitShape {
   int W, parts;
 };
-static UnitShape unit_shape(int bs, int top_k) {
-  const int64_t c = device_cu_count(), units = top_k / 64, pairs = (int64_t)bs * kStepKV;
+static UnitShape unit_shape(int bs, int kv_heads, int top_k) {
+  const int64_t c = device_cu_count(), units = top_k / 64, pairs = (int64_t)bs * kv_heads;
   const int cap8 = std::max(1, std::min(kUnitParts, ceil_div(units, 8)));
   const int cap4 = std::max(1, std::min(kUnitParts, ceil_div(units, 4)));
   if (pairs * units < 8 * c) return {4, cap4};
@@ -770,20 +791,29 @@ extern "C" int qq_quest_fused_step(int q_dtype, int kv_dtype, int new_dtype, int
              : 0;
 }
 
+extern "C" int qq_quest_layer_step_fused(int q_dtype, int kv_dtype, int new_dtype, int num_q_heads, int kv_heads,
+                                         int head_dim, int page_size, int top_k, int max_pages) {
+  if (kv_heads <= 0) return 0;
+  return layer_step_shape(q_dtype, kv_dtype, new_dtype, num_q_heads, kv_heads, head_dim, page_size, top_k, max_pages)
+             ? 1
+             : 0;
+}
+
 // The fused attention over given rows (one launch of quest_attend_unit_kernel in its rows mode);
 // QQ_OK when launched, 1 when the shape or the buffers do not allow it.
 int qq::attend_rows_fused(const void* q, int64_t q_bstride, int num_q_heads, const void* k_layer, const void* v_layer,
-                      int64_t kv_rows, const int64_t* rows, int64_t slots, const int32_t* actual, int bs, float scale,
+                      int64_t kv_rows, int kv_heads, const int64_t* rows, int64_t slots, const int32_t* actual, int bs, float scale,
                       void* out, void* workspace, int64_t workspace_bytes, void* sync, int64_t sync_bytes,
                       hipStream_t s) {
-  if (!sync || sync_bytes < qq_quest_layer_step_sync_bytes(bs, kStepKV) || slots <= 0 || slots > kStepMaxTopK ||
-      slots % 64 != 0 || num_q_heads % kStepKV != 0 || num_q_heads / kStepKV > kStepMaxG || !workspace)
+  if (kv_shift_of(kv_heads) < 0 || !sync || sync_bytes < qq_quest_layer_step_sync_bytes(bs, kv_heads) || slots <= 0 ||
+      slots > kStepMaxTopK || slots % 64 != 0 || num_q_heads % kv_heads != 0 || num_q_heads / kv_heads > kStepMaxG ||
+      !workspace)
     return 1;
   const int top_k = (int)slots;
-  const int G = num_q_heads / kStepKV;
-  const UnitShape us = unit_shape(bs, top_k);
+  const int G = num_q_heads / kv_heads;
+  const UnitShape us = unit_shape(bs, kv_heads, top_k);
   const int W = us.W, parts = us.parts;
-  const int64_t part_bytes = (int64_t)bs * kStepKV * parts * G * (kMfmaDim + 2) * (int64_t)sizeof(float);
+  const int64_t part_bytes = (int64_t)bs * kv_heads * parts * G * (kMfmaDim + 2) * (int64_t)sizeof(float);
   if (parts > 1 && workspace_bytes < part_bytes) return 1;
   StepArgs a{};
   a.s.q = q;
@@ -798,7 +828,8 @@ int qq::attend_rows_fused(const void* q, int64_t q_bstride, int num_q_heads, con
   a.sl2 = scale * kLog2e;
   a.out = static_cast<uint16_t*>(out);
   a.part_o = static_cast<float*>(workspace);
-  a.part_ml = a.part_o + (int64_t)bs * kStepKV * parts * G * kMfmaDim;
+  a.part_ml = a.part_o + (int64_t)bs * kv_heads * parts * G * kMfmaDim;
+  a.kv_shift = kv_shift_of(kv_heads);
   a.parts = parts;
   a.sync = static_cast<uint32_t*>(sync);
   a.bs = bs;
@@ -837,10 +868,10 @@ extern "C" int qq_dense_forward_decode(const void* q, int q_dtype, int64_t q_bat
                                        int64_t sync_bytes, void* stream) {
   const char* what = "qq_dense_forward_decode";
   QQ_REQUIRE(q_dtype == QQ_DTYPE_BF16 && kv_dtype == QQ_DTYPE_BF16 && (!k_new || new_dtype == QQ_DTYPE_BF16) &&
-                 kv_heads == kStepKV && head_dim == kMfmaDim && num_q_heads % kv_heads == 0 &&
+                 kv_heads == kDenseKV && head_dim == kMfmaDim && num_q_heads % kv_heads == 0 &&
                  num_q_heads / kv_heads <= kStepMaxG,
              "%s: the HIP dense decode takes bf16 queries and K/V, %d KV heads x %d, at most %d query heads "
-             "per KV head", what, kStepKV, kMfmaDim, kStepMaxG);
+             "per KV head", what, kDenseKV, kMfmaDim, kStepMaxG);
   QQ_REQUIRE(bs >= 0 && req_to_token_stride > 0 && req_to_token_stride <= (int64_t)1 << 30, "%s: bad sizes", what);
   QQ_REQUIRE(!k_new || (v_new && out_cache_loc), "%s: new K without V or locations", what);
   if (bs == 0) return QQ_OK;
@@ -877,13 +908,14 @@ extern "C" int qq_dense_forward_decode(const void* q, int q_dtype, int64_t q_bat
   a.sl2 = scale * kLog2e;
   a.out = static_cast<uint16_t*>(out);
   a.part_o = static_cast<float*>(workspace);
-  a.part_ml = a.part_o + (int64_t)bs * kStepKV * parts * G * kMfmaDim;
+  a.part_ml = a.part_o + (int64_t)bs * kDenseKV * parts * G * kMfmaDim;
   a.sync = static_cast<uint32_t*>(sync);
   a.bs = bs;
   a.G = G;
+  a.kv_shift = kv_shift_of(kDenseKV);
   a.parts = parts;
   a.per_wave = ceil_div(top_k, parts * kHeadWaves * 32) * 32;
-  quest_attend_part_kernel<<<bs * kStepKV * parts, 64 * kHeadWaves, head_smem_bytes(), s>>>(a);
+  quest_attend_part_kernel<<<bs * kDenseKV * parts, 64 * kHeadWaves, head_smem_bytes(), s>>>(a);
   return check_launch(what);
 }
 
@@ -895,7 +927,8 @@ static int forward_decode(
     const int32_t* actual_lens, int bs, int max_reqs, int max_pages, int kv_heads, int head_dim,
     int page_size, int top_k, const int32_t* req_to_token, int64_t req_to_token_stride,
     int64_t req_to_token_rows, float scale, float* scores_ws, int32_t* positions, void* out,
-    void* workspace, int64_t workspace_bytes, void* sync, int64_t sync_bytes, int phase, hipStream_t s, const char* what) {
+    void* workspace, int64_t workspace_bytes, void* sync, int64_t sync_bytes,
+    bool any_heads, int phase, hipStream_t s, const char* what) {
   QQ_REQUIRE(dtype_ok(q_dtype) && dtype_ok(kv_dtype) && dtype_ok(new_dtype), "%s: unsupported dtype",
              what);
   QQ_REQUIRE(kv_heads > 0 && head_dim > 0 && num_q_heads > 0 && num_q_heads % kv_heads == 0,
@@ -946,12 +979,12 @@ static int forward_decode(
   sa.pool_rows = kv_rows;
 
   const int G = num_q_heads / kv_heads;
-  const UnitShape us = unit_shape(bs, top_k);
+  const UnitShape us = unit_shape(bs, kv_heads, top_k);
   const int W = us.W, parts = us.parts;
   const int64_t part_bytes = (int64_t)bs * kv_heads * parts * G * (kMfmaDim + 2) * (int64_t)sizeof(float);
   const bool fused = sync && sync_bytes >= qq_quest_layer_step_sync_bytes(bs, kv_heads) &&
-                     fused_shape(q_dtype, kv_dtype, k_new ? new_dtype : -1, num_q_heads, kv_heads, head_dim,
-                                 page_size, top_k, max_pages) &&
+                     (any_heads ? layer_step_shape : fused_shape)(q_dtype, kv_dtype, k_new ? new_dtype : -1, num_q_heads,
+                                                                  kv_heads, head_dim, page_size, top_k, max_pages) &&
                      workspace && workspace_bytes >= (parts > 1 ? part_bytes : 0);
   if (fused) {
     // 1. scores of the candidate pages (+ the new token's K/V), all CUs
@@ -972,6 +1005,7 @@ static int forward_decode(
     a.out = static_cast<uint16_t*>(out);
     a.part_o = static_cast<float*>(workspace);
     a.part_ml = a.part_o + (int64_t)bs * kv_heads * parts * G * kMfmaDim;
+    a.kv_shift = kv_shift_of(kv_heads);
     a.parts = parts;
     a.sync = static_cast<uint32_t*>(sync);
     a.bs = bs;
@@ -1024,7 +1058,7 @@ extern "C" int qq_quest_forward_decode(
   return forward_decode(q, q_dtype, q_batch_stride, num_q_heads, k_new, v_new, new_dtype, out_cache_loc, k_layer, v_layer,
       kv_dtype, kv_rows, page_k_bounds, layer, req_pool_indices, seq_lens, candidate_limit, actual_lens, bs,
       max_reqs, max_pages, kv_heads, head_dim, page_size, top_k, req_to_token, req_to_token_stride,
-      req_to_token_rows, scale, scores_ws, positions, out, workspace, workspace_bytes, sync, sync_bytes, 3, static_cast<hipStream_t>(stream), "qq_quest_forward_decode");
+      req_to_token_rows, scale, scores_ws, positions, out, workspace, workspace_bytes, sync, sync_bytes, false, 3, static_cast<hipStream_t>(stream), "qq_quest_forward_decode");
 }
 
 extern "C" int qq_quest_forward_decode_phase(
@@ -1039,7 +1073,22 @@ extern "C" int qq_quest_forward_decode_phase(
   return forward_decode(q, q_dtype, q_batch_stride, num_q_heads, k_new, v_new, new_dtype, out_cache_loc, k_layer, v_layer,
       kv_dtype, kv_rows, page_k_bounds, layer, req_pool_indices, seq_lens, candidate_limit, actual_lens, bs,
       max_reqs, max_pages, kv_heads, head_dim, page_size, top_k, req_to_token, req_to_token_stride,
-      req_to_token_rows, scale, scores_ws, positions, out, workspace, workspace_bytes, sync, sync_bytes, phase, static_cast<hipStream_t>(stream), "qq_quest_forward_decode_phase");
+      req_to_token_rows, scale, scores_ws, positions, out, workspace, workspace_bytes, sync, sync_bytes, false, phase, static_cast<hipStream_t>(stream), "qq_quest_forward_decode_phase");
+}
+
+extern "C" int qq_quest_layer_step(
+    const void* q, int q_dtype, int64_t q_batch_stride, int num_q_heads, const void* k_new,
+    const void* v_new, int new_dtype, const int64_t* out_cache_loc, void* k_layer, void* v_layer,
+    int kv_dtype, int64_t kv_rows, const uint16_t* page_k_bounds, int layer,
+    const int64_t* req_pool_indices, const int64_t* seq_lens, const int32_t* candidate_limit,
+    const int32_t* actual_lens, int bs, int max_reqs, int max_pages, int kv_heads, int head_dim,
+    int page_size, int top_k, const int32_t* req_to_token, int64_t req_to_token_stride,
+    int64_t req_to_token_rows, float scale, float* scores_ws, int32_t* positions, void* out,
+    void* workspace, int64_t workspace_bytes, void* sync, int64_t sync_bytes, int phase, void* stream) {
+  return forward_decode(q, q_dtype, q_batch_stride, num_q_heads, k_new, v_new, new_dtype, out_cache_loc, k_layer, v_layer,
+      kv_dtype, kv_rows, page_k_bounds, layer, req_pool_indices, seq_lens, candidate_limit, actual_lens, bs,
+      max_reqs, max_pages, kv_heads, head_dim, page_size, top_k, req_to_token, req_to_token_stride,
+      req_to_token_rows, scale, scores_ws, positions, out, workspace, workspace_bytes, sync, sync_bytes, true, phase, static_cast<hipStream_t>(stream), "qq_quest_layer_step");
 }
 
 // ------------------------------------------------------------ no allocation
@@ -1125,5 +1174,5 @@ extern "C" int qq_quest_forward_decode_noalloc(
                         actual_lens, bs, max_reqs, max_pages, kv_heads, head_dim, page_size, top_k, req_to_token,
                         req_to_token_stride, req_to_token_rows, scale,
                         reinterpret_cast<float*>(base + kScratchSyncBytes), positions, out, base + kScratchWorkOffset,
-                        kScratchWorkBytes, base, kScratchSyncBytes, 3, s, what);
+                        kScratchWorkBytes, base, kScratchSyncBytes, false, 3, s, what);
 }
