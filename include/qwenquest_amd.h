@@ -343,9 +343,9 @@ int64_t qq_extend_attention_workspace_bytes(int64_t n, int bs, int num_q_heads, 
  * otherwise); seq_lens[i] <= req_to_token_stride.  sync as for
  * qq_quest_forward_decode (>= qq_quest_layer_step_sync_bytes(bs, 4), zeroed
  * once, left zeroed); workspace >= qq_dense_decode_workspace_bytes(bs,
- * req_to_token_stride, H, KV).  Two launches: the K/V store, then the
- * attention (per (request, KV head, part of at most 4096 rows), parts merged
- * inside the launch). */
+ * req_to_token_stride, H, KV).  Two launches: the K/V store with the division of
+ * the batch into parts that fill the chip (on the device, from seq_lens), then the
+ * attention, a block per part, parts merged inside the launch. */
 int qq_dense_forward_decode(const void* q, int q_dtype, int64_t q_batch_stride, int num_q_heads,
                             const void* k_new, const void* v_new, int new_dtype,
                             const int64_t* out_cache_loc, void* k_layer, void* v_layer, int kv_dtype,

@@ -74,13 +74,17 @@ class AttentionBackend(ABC):
         return torch.cat(outputs, dim=0)
 
     def _extend_fast(self, q: torch.Tensor, scaling: float, batch: ForwardBatch) -> bool:
-        """Whether the batched prefill kernel takes this call (its tile is 128 channels wide, and
-        a row's maximum is taken before the scale, which therefore has to be positive)."""
-        pool = self.token_to_kv_pool
+        """Whether the batched prefill kernel takes this call (its tile is 128 channels wide, a
+        row's maximum is taken before the scale, which therefore has to be positive, and it reads
+        the pool in 16-byte pieces; it records no gradient)."""
+        pool, r2t = self.token_to_kv_pool, self.req_to_token
         return (q.dim() == 3 and q.dtype == torch.bfloat16 and pool.dtype == torch.bfloat16
                 and pool.head_dim == 128 and q.shape[2] == 128 and q.shape[0] > 0 and q.shape[1] > 0
                 and q.shape[1] % pool.kv_heads == 0 and q.is_cuda and batch.batch_size > 0
-                and batch.extend_seq_lens is not None and float(scaling) > 0.0)
+                and batch.extend_seq_lens is not None and float(scaling) > 0.0
+                and r2t.dtype == torch.int32 and r2t.stride(1) == 1
+                and (pool.k_all.data_ptr() | pool.v_all.data_ptr()) % 16 == 0
+                and not (q.requires_grad and torch.is_grad_enabled()))
 
     @abstractmethod
     def forward_decode(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, layer: Any, batch: ForwardBatch) -> torch.Tensor:

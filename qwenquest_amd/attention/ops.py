@@ -120,6 +120,8 @@ def extend_attention_batch(
     n, heads, dim = q.shape
     kv, bs, dev = k_buf.shape[1], int(req_pool_indices.shape[0]), q.device
     q = q.contiguous()
+    if q.data_ptr() % 16:  # the kernel reads 16-byte pieces
+        q = q.clone()
 
     def lens(t: torch.Tensor) -> torch.Tensor:
         return t.to(device=dev, dtype=torch.int64).contiguous()

@@ -44,10 +44,12 @@ constexpr int kDenseKV = 4;           // KV heads of the dense decode kernel (KV
 constexpr int kStepMaxG = 16;
 constexpr int kMaxSelFused = 64;
 constexpr int kStepMaxTopK = 4096;
-constexpr int kHeadWaves = 8;        // dense decode: 8-wave blocks (two waves per SIMD)
-constexpr int kHeadTiles = 2;        // 16-row tiles per step (32 rows)
-constexpr int kHeadDepth = 2;        // steps in flight per wave
-constexpr int kMaxParts = 8;         // dense decode: parts merged in one pass
+constexpr int kDenseWaves = 8;       // dense decode: 8-wave blocks (two waves per SIMD)
+constexpr int kDenseBlocks = 256;    // one per CU, at most: all resident
+constexpr int kDenseParts = kDenseBlocks / kDenseKV;  // parts of a (request, KV head), at most
+constexpr int kDenseWhole = 8;       // units of a pair that is not split
+constexpr int kDenseMinLen = 2;      // units of a part, at least
+constexpr int kDensePlanReqs = 4096; // requests whose units the plan keeps in LDS
 // The Quest step's attention (quest_attend_unit_kernel): up to kUnitParts blocks
 // per (request, KV head), merged in one pass; the selection of a 4-wave block
 // holds up to 32 scores per thread (8192 pages; its LDS, 68 KiB, still lets two
@@ -69,7 +71,7 @@ struct StepArgs {
   uint32_t* sync;
   int bs, G;
   int kv_shift;            // log2 of the KV heads
-  int parts, per_wave;     // attention blocks per (request, KV head); rows per wave
+  int parts;               // attention blocks per (request, KV head)
   const int64_t* rows_in;  // rows given [bs, rows_stride] (attention over given rows)
   int64_t rows_stride;
   const int32_t* actual;   // [bs] attended slots (attention over given rows)
@@ -80,68 +82,61 @@ __device__ inline uint32_t* attn_count(const StepArgs& a, int bh) { return a.syn
 
 __device__ inline bool needs_selection(const SelectArgs& sa, int64_t s) { return s > sa.top_k && sa.k_sel > 0; }
 
-// One wave's step: the K and V slices of 16T layout rows of one KV head
-// (lane layouts of attn_wave64: K tile t = tokens 16t .. 16t+15, V k-step u =
-// tokens 16u .. 16u+15).
-template <int T>
-struct StepRegs {
-  bf16x8_t ka[T][4];
-  uint4 vr[T][4];
-};
-
-template <int T>
-__device__ inline void load_step(StepRegs<T>& r, const int32_t* rows, int t0, const uint16_t* kb, const uint16_t* vb,
-                                 int lo, int hi) {
-  constexpr int kRow = kDenseKV * kMfmaDim;
+// One wave's 64 rows of one KV head (lane l: the pool row of token l, the first
+// `valid` of them real), folded into its running softmax: M, L per head lo (log2
+// units), o[e][i] per (head 4hi + i, channel 8lo + e).
+__device__ inline void attend_unit(int r32, int valid, const uint16_t* kb, const uint16_t* vb, int row_shift,
+                                   const bf16x8_t (&qb)[4], float sl2, float& M, float& L, float4_t (&o)[8]) {
+  const int lane = threadIdx.x & 63;
+  const int lo = lane & 15, hi = lane >> 4;
+  // every K and V load of the unit in flight at once
+  bf16x8_t ka[4][4];
+  uint4 vr[4][4];
 #pragma unroll
-  for (int t = 0; t < T; ++t) {
-    const uint16_t* kp = kb + (int64_t)rows[t0 + t * 16 + lo] * kRow + hi * 8;
+  for (int t = 0; t < 4; ++t) {
+    const uint16_t* kp = kb + ((int64_t)__shfl(r32, t * 16 + lo, 64) << row_shift) + hi * 8;
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) r.ka[t][ks] = *reinterpret_cast<const bf16x8_t*>(kp + ks * 32);
+    for (int ks = 0; ks < 4; ++ks) ka[t][ks] = *reinterpret_cast<const bf16x8_t*>(kp + ks * 32);
   }
 #pragma unroll
-  for (int u = 0; u < T; ++u)
+  for (int t = 0; t < 4; ++t)
 #pragma unroll
     for (int j = 0; j < 4; ++j)
-      r.vr[u][j] = *reinterpret_cast<const uint4*>(vb + (int64_t)rows[t0 + u * 16 + hi * 4 + j] * kRow + lo * 8);
-}
-
-// Online-softmax update with one step (tokens t0 .. t0+16T-1, the first
-// `valid` of them real): M, L per head lo (log2 units), o[e][i] per (head
-// 4hi+i, channel 8lo+e).
-template <int T>
-__device__ inline void attend_step(const StepRegs<T>& r, const bf16x8_t (&qb)[4], int valid, float sl2, float& M,
-                                   float& L, float4_t (&o)[8], int lo, int hi) {
-  float4_t acc[T];
+      vr[t][j] = *reinterpret_cast<const uint4*>(vb + ((int64_t)__shfl(r32, t * 16 + hi * 4 + j, 64) << row_shift) + lo * 8);
+  __builtin_amdgcn_sched_barrier(0);  // all 32 loads go out before the first use of any
+  // S^T[token 16t + 4hi + i][head lo] in acc[t][i]
+  float4_t acc[4];
 #pragma unroll
-  for (int t = 0; t < T; ++t) {
+  for (int t = 0; t < 4; ++t) {
     acc[t] = float4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(r.ka[t][ks], qb[ks], acc[t], 0, 0, 0);
+    for (int ks = 0; ks < 4; ++ks) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[t][ks], qb[ks], acc[t], 0, 0, 0);
   }
   float mx = -INFINITY;
 #pragma unroll
-  for (int t = 0; t < T; ++t)
+  for (int t = 0; t < 4; ++t)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const float x = (t * 16 + hi * 4 + i) < valid ? acc[t][i] * sl2 : -INFINITY;
       acc[t][i] = x;
       mx = fmaxf(mx, x);
     }
-  const int lane = threadIdx.x & 63;
   mx = fmaxf(mx, lane_xor16(mx, lane));
   mx = fmaxf(mx, lane_xor32(mx, lane));
   const float Mn = fmaxf(M, mx);
   const float alpha = M == -INFINITY ? 0.0f : exp2f(M - Mn);  // rescale of the running sums
   float sum = 0.0f;
-  short4_t pa[T];
+  short4_t pa[4];
 #pragma unroll
-  for (int t = 0; t < T; ++t)
+  for (int t = 0; t < 4; ++t)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const uint16_t pb = Mn == -INFINITY ? (uint16_t)0 : f2bf(exp2f(acc[t][i] - Mn));
-      sum += bf2f(pb);
-      pa[t][i] = (short)pb;
+      // v_exp_f32 as it is (exp2f adds a rescale for results below 2^-126, which only
+      // the weights of rows 126 binary orders under the maximum reach) and the hardware's
+      // round-to-nearest-even bf16 conversion, equal to f2bf for every value that is not NaN
+      const uint16_t pbits = __builtin_bit_cast(uint16_t, (__bf16)__builtin_amdgcn_exp2f(acc[t][i] - Mn));
+      sum += bf2f(pbits);
+      pa[t][i] = (short)pbits;
     }
   sum += lane_xor16(sum, lane);
   sum += lane_xor32(sum, lane);
@@ -155,11 +150,11 @@ __device__ inline void attend_step(const StepRegs<T>& r, const bf16x8_t (&qb)[4]
     for (int e = 0; e < 8; ++e) o[e][i] *= ai;
   }
 #pragma unroll
-  for (int u = 0; u < T; ++u) {
+  for (int t = 0; t < 4; ++t) {
     short4_t vbv[8];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const uint4 w = r.vr[u][j];
+      const uint4 w = vr[t][j];
       const uint32_t wv[4] = {w.x, w.y, w.z, w.w};
 #pragma unroll
       for (int x = 0; x < 4; ++x) {
@@ -168,33 +163,29 @@ __device__ inline void attend_step(const StepRegs<T>& r, const bf16x8_t (&qb)[4]
       }
     }
 #pragma unroll
-    for (int e = 0; e < 8; ++e) o[e] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(pa[u], vbv[e], o[e], 0, 0, 0);
+    for (int e = 0; e < 8; ++e) o[e] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(pa[t], vbv[e], o[e], 0, 0, 0);
   }
 }
 
-template <int W, int ROWCAP>
-struct HeadSmem {
-  int32_t rows[ROWCAP];  // this block's layout slots -> pool rows
+template <int W>
+struct CombineSmem {
   float m[W][kStepMaxG];
   float l[W][kStepMaxG];
   float o[W][kStepMaxG][kMfmaDim];
 };
 
 // The end of an attention block: its W waves' (M, L, o) (o[e][i]: head 4hi + i,
-// channel 8lo + e) combined in LDS; with one part the block writes the output,
-// else an (m, l, o) partial (agent scope) and the block that completes the
-// (request, KV head) count merges the parts (up to MG at once; GROUPED: more in
-// groups of MG, maximum first).  poison: the output becomes NaN.
-template <int W, int MG, bool GROUPED>
-__device__ inline void finish_block(const StepArgs& a, int bh, int part, float M, float L, const float4_t (&o)[8],
-                                    bool poison, float (*sm_m)[kStepMaxG], float (*sm_l)[kStepMaxG],
-                                    float (*sm_o)[kStepMaxG][kMfmaDim], uint32_t* s_last) {
-  const SelectArgs& sa = a.s;
+// channel 8lo + e) combined in LDS, and either the output (`single`: nothing else
+// attends for this (request, KV head)) or the (m, l, o) partial part_idx (agent
+// scope).  poison: the output becomes NaN.
+template <int W>
+__device__ inline void combine_block(const StepArgs& a, int bh, bool single, int64_t part_idx, float M, float L,
+                                     const float4_t (&o)[8], bool poison, float (*sm_m)[kStepMaxG],
+                                     float (*sm_l)[kStepMaxG], float (*sm_o)[kStepMaxG][kMfmaDim]) {
   constexpr int kThreads = 64 * W;
   const int tid = threadIdx.x;
   const int wave = tid >> 6, lane = tid & 63;
   const int lo = lane & 15, hi = lane >> 4;
-  const int parts = a.parts;
   const int b = bh >> a.kv_shift, h = bh - (b << a.kv_shift);
   const int G = a.G;
 #pragma unroll
@@ -211,8 +202,7 @@ __device__ inline void finish_block(const StepArgs& a, int bh, int part, float M
     sm_l[wave][lo] = poison ? __builtin_nanf("") : L;  // NaN survives every weight of the merge
   }
   __syncthreads();
-  uint16_t* outp = a.out + (int64_t)b * sa.H * kMfmaDim + (int64_t)h * G * kMfmaDim;
-  const int64_t part_idx = (int64_t)bh * parts + part;
+  uint16_t* outp = a.out + (int64_t)b * a.s.H * kMfmaDim + (int64_t)h * G * kMfmaDim;
   const __amdgpu_buffer_rsrc_t po =
       agent_rsrc(a.part_o + part_idx * G * kMfmaDim, (uint32_t)(G * kMfmaDim * sizeof(float)));
   // each thread one head x 4 channels: the waves' (m, l, o) weighted in wave order
@@ -241,7 +231,7 @@ __device__ inline void finish_block(const StepArgs& a, int bh, int part, float M
       Os.z += wgt * ov[w].z;
       Os.w += wgt * ov[w].w;
     }
-    if (parts == 1) {
+    if (single) {
       const bool any = !(Ls <= 0.0f);  // NaN (a poisoned part) stays NaN
       const uint32_t lo2 = (uint32_t)f2bf(any ? Os.x / Ls : 0.0f) | ((uint32_t)f2bf(any ? Os.y / Ls : 0.0f) << 16);
       const uint32_t hi2 = (uint32_t)f2bf(any ? Os.z / Ls : 0.0f) | ((uint32_t)f2bf(any ? Os.w / Ls : 0.0f) << 16);
@@ -254,16 +244,34 @@ __device__ inline void finish_block(const StepArgs& a, int bh, int part, float M
       }
     }
   }
-  if (parts == 1) return;
+}
+
+// Counts this block's partial of a (request, KV head); true, in every thread, for the
+// block that completes `parts` of them (the counter is then 0 again).
+__device__ inline bool last_part(const StepArgs& a, int bh, int parts, uint32_t* s_last) {
   wait_memory();
   __syncthreads();
-  if (tid == 0) *s_last = add_agent(attn_count(a, bh), 1u) == (uint32_t)(parts - 1);
+  if (threadIdx.x == 0) *s_last = add_agent(attn_count(a, bh), 1u) == (uint32_t)(parts - 1);
   __syncthreads();
-  if (!*s_last) return;
-  if (tid == 0) st_agent(attn_count(a, bh), 0u);
-  // merge the parts (in part order: the maximum of the parts' m first, then the
-  // weighted sums): each thread one head x 4 channels; up to MG parts all loads
-  // in flight at once, more parts (dense decode) in two passes of groups
+  if (!*s_last) return false;
+  if (threadIdx.x == 0) st_agent(attn_count(a, bh), 0u);
+  return true;
+}
+
+// combine_block, then the merge of a.parts <= MG parts by the block that completes
+// them (in part order: the maximum of the parts' m first, then the weighted sums),
+// each thread one head x 4 channels, all loads in flight at once.
+template <int W, int MG>
+__device__ inline void finish_block(const StepArgs& a, int bh, int part, float M, float L, const float4_t (&o)[8],
+                                    bool poison, float (*sm_m)[kStepMaxG], float (*sm_l)[kStepMaxG],
+                                    float (*sm_o)[kStepMaxG][kMfmaDim], uint32_t* s_last) {
+  constexpr int kThreads = 64 * W;
+  const int tid = threadIdx.x;
+  const int parts = a.parts, G = a.G;
+  combine_block<W>(a, bh, parts == 1, (int64_t)bh * parts + part, M, L, o, poison, sm_m, sm_l, sm_o);
+  if (parts == 1 || !last_part(a, bh, parts, s_last)) return;
+  const int b = bh >> a.kv_shift, h = bh - (b << a.kv_shift);
+  uint16_t* outp = a.out + (int64_t)b * a.s.H * kMfmaDim + (int64_t)h * G * kMfmaDim;
   const int64_t part0 = (int64_t)bh * parts;
   const __amdgpu_buffer_rsrc_t ro =
       agent_rsrc(a.part_o + part0 * G * kMfmaDim, (uint32_t)(parts * G * kMfmaDim * sizeof(float)));
@@ -273,63 +281,28 @@ __device__ inline void finish_block(const StepArgs& a, int bh, int part, float M
     float Mx = -INFINITY;
     float Ls = 0.0f;
     float4 Os = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (!GROUPED || parts <= MG) {
-      float4 ov[MG];
-      uint64_t mlv[MG];
+    float4 ov[MG];
+    uint64_t mlv[MG];
 #pragma unroll
-      for (int j = 0; j < MG; ++j) {
-        if (j < parts) {
-          ov[j] = ld_agent_x4(ro, (uint32_t)(((j * G + head) * kMfmaDim + d4) * sizeof(float)));
-          mlv[j] = ld_agent(ml64 + j * G + head);
-        }
+    for (int j = 0; j < MG; ++j) {
+      if (j < parts) {
+        ov[j] = ld_agent_x4(ro, (uint32_t)(((j * G + head) * kMfmaDim + d4) * sizeof(float)));
+        mlv[j] = ld_agent(ml64 + j * G + head);
       }
+    }
 #pragma unroll
-      for (int j = 0; j < MG; ++j)
-        if (j < parts) Mx = fmaxf(Mx, __uint_as_float((uint32_t)mlv[j]));
+    for (int j = 0; j < MG; ++j)
+      if (j < parts) Mx = fmaxf(Mx, __uint_as_float((uint32_t)mlv[j]));
 #pragma unroll
-      for (int j = 0; j < MG; ++j) {
-        if (j < parts) {
-          const float mj = __uint_as_float((uint32_t)mlv[j]);
-          const float wgt = mj == -INFINITY ? 0.0f : exp2f(mj - Mx);
-          Ls += wgt * __uint_as_float((uint32_t)(mlv[j] >> 32));
-          Os.x += wgt * ov[j].x;
-          Os.y += wgt * ov[j].y;
-          Os.z += wgt * ov[j].z;
-          Os.w += wgt * ov[j].w;
-        }
-      }
-    } else {
-      for (int j0 = 0; j0 < parts; j0 += MG) {
-        uint64_t mlv[MG];
-#pragma unroll
-        for (int j = 0; j < MG; ++j)
-          if (j0 + j < parts) mlv[j] = ld_agent(ml64 + (j0 + j) * G + head);
-#pragma unroll
-        for (int j = 0; j < MG; ++j)
-          if (j0 + j < parts) Mx = fmaxf(Mx, __uint_as_float((uint32_t)mlv[j]));
-      }
-      for (int j0 = 0; j0 < parts; j0 += MG) {
-        float4 ov[MG];
-        uint64_t mlv[MG];
-#pragma unroll
-        for (int j = 0; j < MG; ++j) {
-          if (j0 + j < parts) {
-            ov[j] = ld_agent_x4(ro, (uint32_t)((((j0 + j) * G + head) * kMfmaDim + d4) * sizeof(float)));
-            mlv[j] = ld_agent(ml64 + (j0 + j) * G + head);
-          }
-        }
-#pragma unroll
-        for (int j = 0; j < MG; ++j) {
-          if (j0 + j < parts) {
-            const float mj = __uint_as_float((uint32_t)mlv[j]);
-            const float wgt = mj == -INFINITY ? 0.0f : exp2f(mj - Mx);
-            Ls += wgt * __uint_as_float((uint32_t)(mlv[j] >> 32));
-            Os.x += wgt * ov[j].x;
-            Os.y += wgt * ov[j].y;
-            Os.z += wgt * ov[j].z;
-            Os.w += wgt * ov[j].w;
-          }
-        }
+    for (int j = 0; j < MG; ++j) {
+      if (j < parts) {
+        const float mj = __uint_as_float((uint32_t)mlv[j]);
+        const float wgt = mj == -INFINITY ? 0.0f : exp2f(mj - Mx);
+        Ls += wgt * __uint_as_float((uint32_t)(mlv[j] >> 32));
+        Os.x += wgt * ov[j].x;
+        Os.y += wgt * ov[j].y;
+        Os.z += wgt * ov[j].z;
+        Os.w += wgt * ov[j].w;
       }
     }
     const bool any = !(Ls <= 0.0f);  // NaN (a poisoned part) stays NaN
@@ -339,54 +312,286 @@ __device__ inline void finish_block(const StepArgs& a, int bh, int part, float M
   }
 }
 
-// Dense decode's attention of one (request, KV head, part) by a block of W
-// waves: the block's share of the dense layout's slots (positions 0 .. s - 1,
-// attention/dense.py:26-42), per_wave rows per wave in steps of 16T rows
-// (DEPTH steps in flight), the waves combined in LDS.  With one part the
-// block writes the output; else it stores an (m, l, o) partial (agent scope)
-// and the block that completes the (request, KV head) count merges the parts
-// (up to MG at once; GROUPED: more in groups).
-template <int W, int T, int DEPTH, int MG, bool GROUPED, int ROWCAP>
-__device__ inline void attend_item(const StepArgs& a, int bh, int part, unsigned char* smem_raw, uint32_t* s_last) {
-  using Smem = HeadSmem<W, ROWCAP>;
-  Smem& sm = *reinterpret_cast<Smem*>(smem_raw);
-  const SelectArgs& sa = a.s;
-  constexpr int kThreads = 64 * W;
-  const int tid = threadIdx.x;
-  const int wave = tid >> 6, lane = tid & 63;
-  const int lo = lane & 15, hi = lane >> 4;
-  const int b = bh / kDenseKV, h = bh - b * kDenseKV;
-  const int64_t s = sa.seq[b];
-  const int64_t req = sa.rpi[b];
-  const int top_k = sa.top_k;  // the table's width: every context fits
-  const int n = (int)min(max(s, (int64_t)0), (int64_t)top_k);
-  const bool r2t_ok = req >= 0 && req < a.r2t_rows;
-  // slots [slot_base, slot_base + per_block): per_wave rows per wave, a multiple of
-  // the 32-row step; the row table is filled over the whole range (row 0 past n),
-  // so every row a step reads is initialised and in range
-  const int per_wave = a.per_wave;
-  const int per_block = W * per_wave;  // <= ROWCAP
-  const int slot_base = part * per_block;
-  for (int i0 = 0; i0 < per_block; i0 += kThreads * 4) {
-    int64_t rv[4];
+// ------------------------------------------------------------- dense decode
+// Every request attends its whole context (attention/dense.py:26-42).  A (request, KV
+// head) pair's 64-row units are split into equal parts, one to a block.  The parts are
+// as long as they have to be for all pairs' parts to fit the blocks that are resident
+// at once: one long request or many ragged ones keep the same number of CUs busy, and
+// the table's width costs nothing.  The lengths are on the device, so the division is
+// made there, by one more block of the launch that stores the new tokens (it hides
+// behind that launch, and the attention's blocks each read one entry instead of the
+// batch's lengths).
+struct DenseItem {
+  int bh;           // pair, or -1: no work for this block
+  int u0, u1;       // its units
+  int part, parts;  // of the pair; its parts are consecutive blocks
+  int rows;         // context
+  int req;          // table row, or -1: outside the table
+  int pad;
+};
+
+struct DenseSmem {
+  union {
+    CombineSmem<kDenseWaves> comb;
+    struct {
+      float w[kStepMaxG][kDenseParts];  // weight of each part
+      float l[kStepMaxG];
+      float4 red[64 * kDenseWaves];
+    } merge;
+  };
+  uint32_t last;
+};
+
+__device__ inline int dense_rows(const StepArgs& a, int b) {
+  return (int)min(max(a.s.seq[b], (int64_t)0), (int64_t)a.s.top_k);
+}
+// A request without rows has one unit, which writes its zeros.
+__device__ inline int dense_units(int rows) { return max((rows + 63) / 64, 1); }
+
+// Parts of a pair for parts of `len` units.  A pair of up to a unit per wave stays
+// whole, which saves its merge (one request of 500 rows: 12.9 us against 15.3 in two
+// parts); longer ones may go down to two units a part (four of 1000 rows: 16.5 us, at
+// four units 17.4, at eight 19.6; one of 8000: 18.0, 17.8 and 19.9).
+__device__ inline int dense_parts(int units, int len) {
+  return units <= kDenseWhole ? 1 : (units + len - 1) / len;
+}
+
+// Sum of v over a 256-thread block (tmp: 4 ints).
+__device__ inline int block_sum_256(int v, int* tmp) {
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int slot = slot_base + i0 + tid + kThreads * u;
-      const bool mine = i0 + tid + kThreads * u < per_block;  // only this block's share is read
-      const int64_t p = min((int64_t)slot, max(s - 1, (int64_t)0));
-      rv[u] = (mine && slot < n && r2t_ok && p < a.r2t_stride) ? a.r2t[req * a.r2t_stride + p] : 0;
+  for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d, 64);
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) tmp[threadIdx.x >> 6] = v;
+  __syncthreads();
+  return tmp[0] + tmp[1] + tmp[2] + tmp[3];
+}
+
+// Block 0: the division of the batch into `blocks` parts; blocks 1 .. bs: the new
+// tokens (memory.py:114-120).  The part length is the smallest of 64 candidates,
+// between the one that would divide the batch without remainders and one that surely
+// fits, with which all parts fit; each lane tries one, the waves share the requests.
+// A batch of more requests than the LDS keeps gets one part per pair.
+__global__ __launch_bounds__(256) void dense_store_plan_kernel(StepArgs a, DenseItem* plan, int blocks) {
+  const int bs = a.bs, tid = threadIdx.x;
+  if (blockIdx.x > 0) {
+    store_new_token(a.s, blockIdx.x - 1);
+    return;
+  }
+  __shared__ uint16_t s_first[kDensePlanReqs + 1];  // parts (per KV head) before each request
+  __shared__ int s_units[kDensePlanReqs];
+  __shared__ int s_tmp[4], s_count[4][64], s_len;
+  const bool kept = bs <= kDensePlanReqs;
+  int sum = 0, most = 1;
+  for (int b = tid; kept && b < bs; b += 256) {
+    const int u = dense_units(dense_rows(a, b));
+    s_units[b] = u;
+    sum += u;
+    most = max(most, u);
+  }
+  const int wave = tid >> 6, lane = tid & 63;
+  const int fit = blocks / kDenseKV;  // parts per KV head that fit; at least bs
+  int len = 1 << 30;                  // units per part
+  if (kept && fit > bs) {
+    const int total = block_sum_256(sum, s_tmp);
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) most = max(most, __shfl_xor(most, d, 64));
+    __syncthreads();
+    if (lane == 0) s_tmp[wave] = most;
+    __syncthreads();
+    most = max(max(s_tmp[0], s_tmp[1]), max(s_tmp[2], s_tmp[3]));
+    const int lo = max((total + fit - 1) / fit, kDenseMinLen);
+    const int hi = max(lo, min(most, (total + fit - bs - 1) / (fit - bs)));  // sum of ceil(u / hi) <= total / hi + bs
+    const int cand = lo + (int)(((int64_t)(hi - lo) * lane) / 63);
+    int count = 0;
+    for (int b = wave; b < bs; b += 4) count += dense_parts(s_units[b], cand);
+    s_count[wave][lane] = count;
+    __syncthreads();
+    count = s_count[0][lane] + s_count[1][lane] + s_count[2][lane] + s_count[3][lane];
+    const uint64_t ok = __ballot(count <= fit);
+    len = __shfl(cand, ok ? __builtin_ctzll(ok) : 63, 64);
+  }
+  if (!kept || fit <= bs) {  // one part per pair
+    for (int e = tid; e < blocks; e += 256) {
+      DenseItem it = {-1, 0, 0, 0, 1, 0, -1, 0};
+      if (e < bs * kDenseKV) {
+        const int b = e / kDenseKV;
+        const int64_t req = a.s.rpi[b];
+        it.bh = e;
+        it.rows = dense_rows(a, b);
+        it.u1 = dense_units(it.rows);
+        it.req = req >= 0 && req < a.r2t_rows ? (int)req : -1;
+      }
+      plan[e] = it;
+    }
+    return;
+  }
+  // parts before each request: a prefix sum, 256 requests at a time
+  int base = 0;
+  for (int b0 = 0; b0 < bs; b0 += 256) {
+    const int b = b0 + tid;
+    const int mine = b < bs ? dense_parts(s_units[b], len) : 0;
+    int x = mine;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int y = __shfl_up(x, d, 64);
+      if (lane >= d) x += y;
+    }
+    __syncthreads();
+    if (lane == 63) s_tmp[wave] = x;
+    __syncthreads();
+    int before = base;
+    for (int w = 0; w < wave; ++w) before += s_tmp[w];
+    if (b < bs) s_first[b] = (uint16_t)(before + x - mine);
+    base += s_tmp[0] + s_tmp[1] + s_tmp[2] + s_tmp[3];
+  }
+  if (tid == 0) s_first[bs] = (uint16_t)base;
+  __syncthreads();
+  for (int e = tid; e < blocks; e += 256) {
+    DenseItem it = {-1, 0, 0, 0, 1, 0, -1, 0};
+    // blocks of a request: its parts of KV head 0, then of head 1, ...
+    if (e < base * kDenseKV) {
+      int b = 0, b_end = bs;  // the last request whose first block is <= e
+      while (b_end - b > 1) {
+        const int mid = (b + b_end) >> 1;
+        if (s_first[mid] * kDenseKV <= e) b = mid;
+        else b_end = mid;
+      }
+      const int parts = s_first[b + 1] - s_first[b];
+      const int at = e - s_first[b] * kDenseKV;
+      const int h = at / parts, part = at - h * parts;
+      const int units = s_units[b];
+      const int64_t req = a.s.rpi[b];
+      it.bh = b * kDenseKV + h;
+      it.u0 = (int)(((int64_t)units * part) / parts);
+      it.u1 = (int)(((int64_t)units * (part + 1)) / parts);
+      it.part = part;
+      it.parts = parts;
+      it.rows = dense_rows(a, b);
+      it.req = req >= 0 && req < a.r2t_rows ? (int)req : -1;
+    }
+    plan[e] = it;
+  }
+}
+
+// The parts of a pair added up by a whole block: the weights e^(m - max) of every
+// part in LDS, a wave per head and a lane per part, then each thread one head x 4
+// channels of every ng-th part, 32 loads in flight.
+__device__ inline void merge_dense(const StepArgs& a, int bh, int64_t part0, int parts, DenseSmem& sm) {
+  constexpr int kThreads = 64 * kDenseWaves;
+  constexpr int kPer = (kDenseParts + 63) / 64;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int G = a.G;
+  const uint64_t* ml64 = reinterpret_cast<const uint64_t*>(a.part_ml) + part0 * G;
+  const __amdgpu_buffer_rsrc_t ro =
+      agent_rsrc(a.part_o + part0 * G * kMfmaDim, (uint32_t)((int64_t)parts * G * kMfmaDim * sizeof(float)));
+  const int items = G * (kMfmaDim / 4);  // (head, 4 channels): up to 512
+  const int ng = max(kThreads / items, 1);
+  const int grp = items <= kThreads ? tid / items : 0;
+  // the first kBatch parts' sums go out before the weights are known; past the last
+  // part they are zeros, from beyond the resource
+  constexpr int kBatch = 32;
+  float4 ov[kBatch];
+  auto load_parts = [&](int at, int p0) {
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u)
+      ov[u] = ld_agent_x4(ro, (uint32_t)(((p0 + u * ng) * G * kMfmaDim + at * 4) * (int)sizeof(float)));
+  };
+  load_parts(tid - grp * items, grp);
+  for (int head = wave; head < G; head += kDenseWaves) {
+    uint64_t ml[kPer];
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      const int p = lane + 64 * i;
+      ml[i] = p < parts ? ld_agent(ml64 + (int64_t)p * G + head) : (uint64_t)0xFF800000u;  // (-inf, 0)
+    }
+    float Mx = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) Mx = fmaxf(Mx, __uint_as_float((uint32_t)ml[i]));
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) Mx = fmaxf(Mx, __shfl_xor(Mx, d, 64));
+    float Ls = 0.0f;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      const float m = __uint_as_float((uint32_t)ml[i]);
+      const float w = m == -INFINITY ? 0.0f : exp2f(m - Mx);
+      if (lane + 64 * i < parts) sm.merge.w[head][lane + 64 * i] = w;
+      Ls += w * __uint_as_float((uint32_t)(ml[i] >> 32));
     }
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int i = i0 + tid + kThreads * u;
-      const int slot = slot_base + i;
-      if (i < per_block) {
-        const int64_t row = rv[u];
-        sm.rows[i] = (slot < n && row >= 0 && row < a.kv_rows) ? (int32_t)row : 0;
+    for (int d = 32; d >= 1; d >>= 1) Ls += __shfl_xor(Ls, d, 64);
+    if (lane == 0) sm.merge.l[head] = Ls;
+  }
+  __syncthreads();
+  if (ng == 1 && grp > 0) return;  // threads past the items
+  const int b = bh / kDenseKV, h = bh - b * kDenseKV;
+  uint16_t* outp = a.out + (int64_t)b * a.s.H * kMfmaDim + (int64_t)h * G * kMfmaDim;
+  const int at0 = tid - grp * items;
+  for (int at = at0; at < items; at += kThreads) {  // once, for every thread, where ng > 1
+    const int head = at >> 5, d4 = (at & 31) * 4;
+    float4 Os = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (grp < ng) {
+      for (int p0 = grp; p0 < parts; p0 += kBatch * ng) {
+        if (at != at0 || p0 != grp) load_parts(at, p0);
+#pragma unroll
+        for (int u = 0; u < kBatch; ++u) {
+          const float w = sm.merge.w[head][min(p0 + u * ng, parts - 1)];
+          Os.x += w * ov[u].x;
+          Os.y += w * ov[u].y;
+          Os.z += w * ov[u].z;
+          Os.w += w * ov[u].w;
+        }
       }
     }
+    if (ng > 1) {  // block-uniform
+      sm.merge.red[tid] = Os;
+      __syncthreads();
+      if (grp != 0) return;
+      for (int g = 1; g < ng; ++g) {
+        const float4 x = sm.merge.red[tid + g * items];
+        Os.x += x.x;
+        Os.y += x.y;
+        Os.z += x.z;
+        Os.w += x.w;
+      }
+    }
+    const float Ls = sm.merge.l[head];
+    const bool any = !(Ls <= 0.0f);
+    const uint32_t lo2 = (uint32_t)f2bf(any ? Os.x / Ls : 0.0f) | ((uint32_t)f2bf(any ? Os.y / Ls : 0.0f) << 16);
+    const uint32_t hi2 = (uint32_t)f2bf(any ? Os.z / Ls : 0.0f) | ((uint32_t)f2bf(any ? Os.w / Ls : 0.0f) << 16);
+    *reinterpret_cast<uint2*>(outp + head * kMfmaDim + d4) = make_uint2(lo2, hi2);
   }
-  const int G = a.G;
+}
+
+// One part of a pair: wave w takes units u0 + w, u0 + w + 8, ..., each with all of its
+// 32 KiB of K and V in flight at once; one block per CU.
+//
+// Bound: HBM.  Attention and store, per layer at 32 / 4 heads, against blocks of 4096
+// rows each, as many per pair as the table's width holds: one request of 8000 rows
+// 49 -> 18 us, of 100000 83 -> 52; 16 ragged requests of 2000 .. 65000 in a
+// 131072-wide table 480 -> 106 (4.6 TB/s); 16 of 131000 785 -> 745 (5.8 TB/s); 64 of
+// 3000 84 -> 76.  4-wave blocks, two per CU: 64 of 3000 87 us, one of 100000 63 (twice
+// the parts to merge), one of 8000 16.9.
+__global__ __launch_bounds__(64 * kDenseWaves, 2) void dense_attend_kernel(StepArgs a, const DenseItem* plan) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  DenseSmem& sm = *reinterpret_cast<DenseSmem*>(smem_raw);
+  const SelectArgs& sa = a.s;
+  const DenseItem it = plan[blockIdx.x];
+  if (it.bh < 0) return;
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int lo = lane & 15, hi = lane >> 4;
+  const int G = a.G, n = it.rows;
+  const int b = it.bh / kDenseKV, h = it.bh - b * kDenseKV;
+  const int32_t* rt = a.r2t + (int64_t)max(it.req, 0) * a.r2t_stride;
+  // units with rows: a request without any has one unit and no rows
+  const int u_end = min(it.u1, (n + 63) / 64);
+  // lane l: the pool row of token l of a unit, as the table has it (row 0 past the
+  // context); looked at a unit later, so that it is loaded under the unit before
+  auto table_row = [&](int j) -> int {
+    const int slot = j * 64 + lane;
+    return (j < u_end && slot < n && it.req >= 0) ? rt[slot] : 0;
+  };
+  int row = table_row(it.u0 + wave);
   bf16x8_t qb[4];
   {
     const uint16_t* qp = static_cast<const uint16_t*>(sa.q) + (int64_t)b * sa.q_bstride +
@@ -400,44 +605,23 @@ __device__ inline void attend_item(const StepArgs& a, int bh, int part, unsigned
       }
     }
   }
-  lds_barrier();  // the row table is in LDS; the query loads stay in flight
-  // this wave's rows: local [r0, r0 + per_wave), real up to slot n
-  constexpr int kStep = 16 * T;
-  const int r0 = wave * per_wave;
-  const int r_end = max(r0, min(r0 + per_wave, n - slot_base));
-  const int nsteps = (r_end - r0 + kStep - 1) / kStep;
   const uint16_t* kb = a.k + h * kMfmaDim;
   const uint16_t* vb = a.v + h * kMfmaDim;
   float M = -INFINITY, L = 0.0f;
   float4_t o[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) o[e] = float4_t{0.f, 0.f, 0.f, 0.f};
-  StepRegs<T> ring[DEPTH];
-#pragma unroll
-  for (int j = 0; j < DEPTH - 1; ++j)
-    if (j < nsteps) load_step<T>(ring[j], sm.rows, r0 + kStep * j, kb, vb, lo, hi);
-  for (int i0 = 0; i0 < nsteps; i0 += DEPTH) {
-#pragma unroll
-    for (int j = 0; j < DEPTH; ++j) {
-      const int i = i0 + j;
-      if (i >= nsteps) break;
-      const int ahead = i + DEPTH - 1;
-      if (ahead < nsteps) load_step<T>(ring[(j + DEPTH - 1) % DEPTH], sm.rows, r0 + kStep * ahead, kb, vb, lo, hi);
-      attend_step<T>(ring[j], qb, r_end - (r0 + kStep * i), a.sl2, M, L, o, lo, hi);
-    }
+  // the row and the query are in; the compiler then knows that a unit's row, loaded
+  // under the unit before, needs no wait, which would be one for the next row too
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+  for (int j = it.u0 + wave; j < u_end; j += kDenseWaves) {
+    const int next = table_row(j + kDenseWaves);
+    attend_unit(row >= 0 && row < a.kv_rows ? row : 0, min(n - j * 64, 64), kb, vb, 9, qb, a.sl2, M, L, o);
+    row = next;
   }
-  finish_block<W, MG, GROUPED>(a, bh, part, M, L, o, false, sm.m, sm.l, sm.o, s_last);
-}
-
-using HeadSmemLaunch = HeadSmem<kHeadWaves, kStepMaxTopK>;
-
-// Dense decode's attention launch: one 8-wave block per (request, KV head,
-// part), blockIdx = (request, KV head) * parts + part.
-__global__ __launch_bounds__(64 * kHeadWaves, 1) void quest_attend_part_kernel(StepArgs a) {
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  __shared__ uint32_t s_last;
-  const int bh = blockIdx.x / a.parts, part = blockIdx.x - bh * a.parts;
-  attend_item<kHeadWaves, kHeadTiles, kHeadDepth, kMaxParts, true, kStepMaxTopK>(a, bh, part, smem_raw, &s_last);
+  combine_block<kDenseWaves>(a, it.bh, it.parts == 1, blockIdx.x, M, L, o, false, sm.comb.m, sm.comb.l, sm.comb.o);
+  if (it.parts > 1 && last_part(a, it.bh, it.parts, &sm.last))
+    merge_dense(a, it.bh, (int64_t)blockIdx.x - it.part, it.parts, sm);
 }
 
 // ------------------------------------------------------- per-page-unit attention
@@ -459,11 +643,7 @@ template <int KPT, int W>
 struct UnitSmem {
   union {
     RankSelectSmem<(KPT > 0 ? KPT : 1), 64 * W> sel;
-    struct {
-      float m[W][kStepMaxG];
-      float l[W][kStepMaxG];
-      float o[W][kStepMaxG][kMfmaDim];
-    } comb;
+    CombineSmem<W> comb;
   };
 };
 
@@ -565,87 +745,12 @@ __global__ __launch_bounds__(64 * W, 8 / W) void quest_attend_unit_kernel(StepAr
     }
     if (valid <= 0) continue;
     const int r32 = (row >= 0 && row < a.kv_rows) ? (int)row : 0;
-    // every K and V load of the unit in flight at once
-    bf16x8_t ka[4][4];
-    uint4 vr[4][4];
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const uint16_t* kp = kb + ((int64_t)__shfl(r32, t * 16 + lo, 64) << row_shift) + hi * 8;
-#pragma unroll
-      for (int ks = 0; ks < 4; ++ks) ka[t][ks] = *reinterpret_cast<const bf16x8_t*>(kp + ks * 32);
-    }
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        vr[t][j] = *reinterpret_cast<const uint4*>(vb + ((int64_t)__shfl(r32, t * 16 + hi * 4 + j, 64) << row_shift) + lo * 8);
-    __builtin_amdgcn_sched_barrier(0);  // all 32 loads go out before the first use of any
-    // S^T[token 16t + 4hi + i][head lo] in acc[t][i]
-    float4_t acc[4];
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      acc[t] = float4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int ks = 0; ks < 4; ++ks) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[t][ks], qb[ks], acc[t], 0, 0, 0);
-    }
-    float mx = -INFINITY;
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float x = (t * 16 + hi * 4 + i) < valid ? acc[t][i] * a.sl2 : -INFINITY;
-        acc[t][i] = x;
-        mx = fmaxf(mx, x);
-      }
-    mx = fmaxf(mx, lane_xor16(mx, lane));
-    mx = fmaxf(mx, lane_xor32(mx, lane));
-    const float Mn = fmaxf(M, mx);
-    const float alpha = M == -INFINITY ? 0.0f : exp2f(M - Mn);  // rescale of the running sums
-    float sum = 0.0f;
-    short4_t pa[4];
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        // v_exp_f32 as it is (exp2f adds a rescale for results below 2^-126, which only
-        // the weights of rows 126 binary orders under the maximum reach) and the hardware's
-        // round-to-nearest-even bf16 conversion, equal to f2bf for every value that is not NaN
-        const uint16_t pbits = __builtin_bit_cast(uint16_t, (__bf16)__builtin_amdgcn_exp2f(acc[t][i] - Mn));
-        sum += bf2f(pbits);
-        pa[t][i] = (short)pbits;
-      }
-    sum += lane_xor16(sum, lane);
-    sum += lane_xor32(sum, lane);
-    L = L * alpha + sum;
-    M = Mn;
-    // o rows are heads 4hi + i: their scale factors live in lanes 4hi + i
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float ai = __shfl(alpha, hi * 4 + i, 64);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) o[e][i] *= ai;
-    }
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      short4_t vbv[8];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const uint4 w = vr[t][j];
-        const uint32_t wv[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-        for (int x = 0; x < 4; ++x) {
-          vbv[2 * x][j] = (short)(wv[x] & 0xFFFFu);
-          vbv[2 * x + 1][j] = (short)(wv[x] >> 16);
-        }
-      }
-#pragma unroll
-      for (int e = 0; e < 8; ++e) o[e] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(pa[t], vbv[e], o[e], 0, 0, 0);
-    }
+    attend_unit(r32, valid, kb, vb, row_shift, qb, a.sl2, M, L, o);
   }
   bool poison = false;
   if constexpr (ROWS) poison = __syncthreads_or(bad ? 1 : 0) != 0;  // a failed swap-in: NaN output
   else lds_barrier();  // the selection's LDS is free before the combine reuses it
-  finish_block<W, kUnitParts, false>(a, bh, part, M, L, o, poison, sm.comb.m, sm.comb.l, sm.comb.o, &s_last);
+  finish_block<W, kUnitParts>(a, bh, part, M, L, o, poison, sm.comb.m, sm.comb.l, sm.comb.o, &s_last);
 }
 
 }  // namespace
@@ -673,15 +778,15 @@ static int device_cu_count() {
 
 // LDS of the dense attention kernel (above the 64 KiB default: opted in once per
 // device).
-static size_t head_smem_bytes() {
+static size_t dense_smem_bytes() {
   static bool opted[64] = {false};
   int dev = 0;
   if (hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < 64 && !opted[dev]) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&quest_attend_part_kernel),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(HeadSmemLaunch));
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&dense_attend_kernel),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(DenseSmem));
     opted[dev] = true;
   }
-  return sizeof(HeadSmemLaunch);
+  return sizeof(DenseSmem);
 }
 
 // LDS of a unit-attention instance: the wave combine, or the selection that
@@ -844,18 +949,18 @@ int qq::attend_rows_fused(const void* q, int64_t q_bstride, int num_q_heads, con
   return QQ_OK;
 }
 
-// Dense decode (attention/dense.py:26-42): every request attends
-// req_to_token[req, 0 .. seq_len) - the fused attention kernel without a
-// selection (its dense layout), at most kStepMaxTopK rows per block and as
-// many parts per (request, KV head) as the longest context of the table needs.
-static int dense_parts(int64_t max_rows) { return max(1, ceil_div(max_rows, kStepMaxTopK)); }
+// Dense decode: one block per CU, or as many as the table's width can use; at least
+// one per (request, KV head).
+static int64_t dense_blocks(int bs, int64_t max_rows) {
+  const int64_t pairs = (int64_t)bs * kDenseKV, units = pairs * ((max_rows + 63) / 64);
+  return std::max(pairs, std::min<int64_t>(std::min(device_cu_count(), kDenseBlocks), units));
+}
 
 extern "C" int64_t qq_dense_decode_workspace_bytes(int bs, int64_t max_rows, int num_q_heads, int kv_heads) {
   if (bs <= 0 || max_rows <= 0 || kv_heads <= 0 || num_q_heads <= 0) return 0;
-  const int parts = dense_parts(max_rows);
-  return parts > 1 ? (int64_t)bs * kv_heads * parts * (num_q_heads / kv_heads) * (kMfmaDim + 2) *
-                         (int64_t)sizeof(float)
-                   : 0;
+  // the division of the batch, then the parts' (m, l, o)
+  return dense_blocks(bs, max_rows) *
+         (int64_t)(sizeof(DenseItem) + (num_q_heads / kv_heads) * (kMfmaDim + 2) * sizeof(float));
 }
 
 extern "C" int qq_dense_forward_decode(const void* q, int q_dtype, int64_t q_batch_stride, int num_q_heads,
@@ -881,14 +986,10 @@ extern "C" int qq_dense_forward_decode(const void* q, int q_dtype, int64_t q_bat
   QQ_REQUIRE(need == 0 || (workspace && workspace_bytes >= need), "%s: workspace %lld bytes < %lld needed", what,
              (long long)workspace_bytes, (long long)need);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (k_new) {  // set_kv_buffer (memory.py:114-120) before the attention reads the pool
-    const int st = qq_kv_scatter(k_layer, v_layer, kv_dtype, kv_rows, k_new, v_new, new_dtype, out_cache_loc, bs,
-                                 (int64_t)kv_heads * head_dim, stream);
-    if (st != QQ_OK) return st;
-  }
   const int top_k = (int)req_to_token_stride;  // every context fits: seq_len <= the table's width
   const int G = num_q_heads / kv_heads;
-  const int parts = dense_parts(top_k);
+  const int64_t blocks = dense_blocks(bs, top_k);
+  QQ_REQUIRE(blocks < (int64_t)1 << 31 && req_to_token_rows < (int64_t)1 << 31, "%s: bad sizes", what);
   StepArgs a{};
   a.s.q = q;
   a.s.q_dtype = QQ_DTYPE_BF16;
@@ -907,15 +1008,34 @@ extern "C" int qq_dense_forward_decode(const void* q, int q_dtype, int64_t q_bat
   a.r2t_rows = req_to_token_rows;
   a.sl2 = scale * kLog2e;
   a.out = static_cast<uint16_t*>(out);
-  a.part_o = static_cast<float*>(workspace);
-  a.part_ml = a.part_o + (int64_t)bs * kDenseKV * parts * G * kMfmaDim;
+  DenseItem* plan = static_cast<DenseItem*>(workspace);
+  a.part_o = reinterpret_cast<float*>(plan + blocks);
+  a.part_ml = a.part_o + blocks * G * kMfmaDim;
   a.sync = static_cast<uint32_t*>(sync);
   a.bs = bs;
   a.G = G;
   a.kv_shift = kv_shift_of(kDenseKV);
-  a.parts = parts;
-  a.per_wave = ceil_div(top_k, parts * kHeadWaves * 32) * 32;
-  quest_attend_part_kernel<<<bs * kDenseKV * parts, 64 * kHeadWaves, head_smem_bytes(), s>>>(a);
+  // set_kv_buffer (memory.py:114-120) before the attention reads the pool: in 16-byte
+  // pieces by the plan's launch, else by the general scatter
+  const uintptr_t align = reinterpret_cast<uintptr_t>(k_new) | reinterpret_cast<uintptr_t>(v_new) |
+                          reinterpret_cast<uintptr_t>(k_layer) | reinterpret_cast<uintptr_t>(v_layer);
+  const bool store = k_new && align % 16 == 0;
+  if (k_new && !store) {
+    const int st = qq_kv_scatter(k_layer, v_layer, kv_dtype, kv_rows, k_new, v_new, new_dtype, out_cache_loc, bs,
+                                 (int64_t)kv_heads * head_dim, stream);
+    if (st != QQ_OK) return st;
+  }
+  a.s.C = kDenseKV * kMfmaDim;
+  a.s.new_k = k_new;
+  a.s.new_v = v_new;
+  a.s.new_dtype = QQ_DTYPE_BF16;
+  a.s.new_locs = out_cache_loc;
+  a.s.k_pool = k_layer;
+  a.s.v_pool = v_layer;
+  a.s.pool_dtype = QQ_DTYPE_BF16;
+  a.s.pool_rows = kv_rows;
+  dense_store_plan_kernel<<<store ? bs + 1 : 1, 256, 0, s>>>(a, plan, (int)blocks);
+  dense_attend_kernel<<<(int)blocks, 64 * kDenseWaves, dense_smem_bytes(), s>>>(a, plan);
   return check_launch(what);
 }
 

@@ -1,0 +1,70 @@
+"""Dense decode's division of a batch into equal runs (reference
+``src/qwenquest/attention/dense.py:26-42``): runs that end inside a request, inside a KV head's
+rows or cover many requests, merges over one and several thread groups, against float64."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DEV = torch.device("cuda", 0)
+KV, D = 4, 128
+
+
+class Layer:
+    layer_id, scaling = 0, D**-0.5
+
+
+@pytest.mark.parametrize("heads,ctx,width", [
+    (32, [8000], 8064),  # one request over 125 blocks
+    (16, [4097, 63], 4200),  # groups of 4: two thread groups merge
+    (20, [2500, 1, 64, 65], 2600),  # groups of 5: threads past the merge's items
+    (28, [700] * 3 + [3001], 3100),
+    (4, [5000, 256], 5100),  # no grouping: eight thread groups merge
+    (64, [3000, 17], 3100),  # groups of 16: two items per thread
+    (8, [130, 0, 64], 200),  # a request without rows: zeros
+    (32, [1 + 37 * i for i in range(70)], 2700),  # more requests than lanes
+    (32, [20000, 300, 9000], 131072),  # several units per wave; a table far wider than the contexts
+])
+def test_dense_decode_matches_float64(heads, ctx, width):
+    from qwenquest_amd.attention.dense import DenseBackend
+    from qwenquest_amd.batch import ForwardBatch, ForwardMode
+    from qwenquest_amd.memory import MHATokenToKVPool, ReqToTokenPool
+
+    bs, G = len(ctx), heads // KV
+    rtp = ReqToTokenPool(bs, width, DEV)
+    kvp = MHATokenToKVPool(sum(ctx) + 1, 1, KV, D, torch.bfloat16, DEV)
+    gen = torch.Generator(device=DEV).manual_seed(2)
+    kvp.k_all.normal_(generator=gen)
+    kvp.v_all.normal_(generator=gen)
+    perm = (torch.randperm(sum(ctx), generator=torch.Generator().manual_seed(3)) + 1).to(torch.int32).to(DEV)
+    at = 0
+    for i, n in enumerate(ctx):
+        rtp.req_to_token[i, :n] = perm[at : at + n]
+        at += n
+    be = DenseBackend(rtp, kvp)
+    rpi, seq = torch.arange(bs, device=DEV), torch.tensor(ctx, device=DEV)
+    loc = rtp.req_to_token[rpi, (seq - 1).clamp(min=0)].long()
+    loc = torch.where(seq > 0, loc, sum(ctx) + 1)
+    mk = lambda h: torch.empty((bs, h, D), device=DEV).normal_(generator=gen).to(torch.bfloat16)  # noqa: E731
+    q, k, v = mk(heads), mk(KV), mk(KV)
+    batch = ForwardBatch(ForwardMode.DECODE, None, None, rpi, seq, loc, rtp, kvp, be)
+    out = be.forward_decode(q, k, v, Layer(), batch)
+    assert torch.equal(be.forward_decode(q, k, v, Layer(), batch), out)
+    assert not be._sync.any()
+    for i, n in enumerate(ctx):
+        if n == 0:
+            assert not out[i].any()
+            continue
+        rows = rtp.req_to_token[i, :n].long()
+        kk, vv = kvp.k_all[0][rows].double(), kvp.v_all[0][rows].double()
+        got = out[i].view(heads, D).double()
+        for h in range(heads):
+            p = torch.softmax((kk[:, h // G] @ q[i, h].double()) * D**-0.5, 0)
+            ref = p @ vv[:, h // G]
+            # half a bf16 ulp of the output, and of every weight (2^-9 each, at random signs
+            # over the weights: their root sum of squares bounds it well)
+            bound = 2.0**-8 * ref.abs() + 2.0**-8 * 3 * float((p * p).sum().sqrt()) + 1e-5
+            assert bool(((got[h] - ref).abs() <= bound).all()), (i, h)
