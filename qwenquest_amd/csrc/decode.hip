@@ -630,7 +630,7 @@ __global__ __launch_bounds__(64 * kDenseWaves, 2) void dense_attend_kernel(StepA
 // one 4-wave block per (request, KV head, part), blockIdx = (request, KV head) *
 // parts + part.  The layout's slots come in units of 64 (a selected page, or the
 // recent window, or 64 slots of the dense layout); wave w of part p takes units
-// p*4 + w, p*4 + w + 4*parts, ...  (one unit per wave at top_k 2048).  Per unit a
+// w*parts + p, w*parts + p + W*parts, ...  (unit_shape).  Per unit a
 // wave resolves its 64 rows itself (lane l: slot 64u + l -> position ->
 // req_to_token), shuffles them into the MFMA lane layouts and issues all 32
 // loads of the unit's K and V slices (32 KiB per wave) at once, then
@@ -723,7 +723,7 @@ __global__ __launch_bounds__(64 * W, 8 / W) void quest_attend_unit_kernel(StepAr
 #pragma unroll
   for (int e = 0; e < 8; ++e) o[e] = float4_t{0.f, 0.f, 0.f, 0.f};
   bool bad = false;
-  for (int u = part * W + wave; u < units; u += stride_units) {  // wave-uniform
+  for (int u = wave * parts + part; u < units; u += stride_units) {  // wave-uniform
     const int slot = u * P + lane;
     const int valid = min(n - u * P, P);  // real slots of this unit
     int64_t row = 0;
@@ -865,18 +865,23 @@ static bool fused_shape(int q_dtype, int kv_dtype, int new_dtype, int num_q_head
 }
 
 // Launch shape of the unit attention: W waves per block, `parts` blocks per (request,
-// KV head); a wave takes the units p*W + w, p*W + w + W*parts, ... one after the other.
-// The grid is sized to one round of resident blocks, since each block pays its own
-// selection, row lookups and merge before and after its streaming:
-//  * fewer units than one 8-wave block per CU could take: 4-wave blocks, one unit per
-//    wave (as many parts as that needs, up to kUnitParts);
-//  * up to one (request, KV head) pair per CU: 8-wave blocks (one per CU), parts =
-//    CUs / pairs (batch 16 x 2048 slots: 4 parts, one unit per wave; batch 32: 2 parts);
-//  * more pairs: 4-wave blocks (two per CU), parts = ceil(2 CUs / pairs) (1 from 2 pairs
-//    per CU on).
-// Measured at 48 layers: batch 32 x 64K 51.3 -> 45.2 us per layer-step, batch 64 x 32K
-// 83.5 -> 67.1, batch 96 x 21.8K 101.4 -> 93.0, batch 128 x 16K 147.6 -> 111.0 against
-// one unit per wave throughout.
+// KV head); wave w of part p takes the units w * parts + p, + W * parts, ... one after
+// the other.  The grid is sized to one round of resident blocks, since each block pays
+// its own selection, row lookups and merge before and after its streaming (us per
+// layer-step, top_k 2048 at 4 KV heads unless said):
+//  * a unit per wave in 4-wave blocks that leave each CU at most one: those (batch 8:
+//    16.4, 18.2 in 8-wave blocks; batch 9, where they would be more than the CUs: 19.9
+//    against 18.7);
+//  * up to one pair per CU: 8-wave blocks (one per CU), parts = CUs / pairs, unless two
+//    4-wave blocks per CU, parts = 2 CUs / pairs, leave a wave fewer units in a row
+//    (batch 34: 42.3 in 4-wave blocks, three parts, against 47.6; batch 40: 45.5 and
+//    48.1, at top_k 4096 75.9 and 83.9; batch 48, where the rows are as long: 51.7
+//    and 50.5);
+//  * more pairs: 4-wave blocks, 3 parts up to 4/3 pairs per CU, then 2, past 8/5 1
+//    (batch 72: 74.3 in 3, 77.1 in 2; batch 84: 81.4 and 83.0; batch 96: 94.7 and 89.6;
+//    batch 104: 102.2 in 2, 96.3 in 1).
+// A second round of units in a part is dealt over all parts, not to the first ones
+// (batch 20, 32 units over 24 waves: 32.0 -> 28.5).
 struct UnitShape {
   int W, parts;
 };
@@ -884,9 +889,14 @@ static UnitShape unit_shape(int bs, int kv_heads, int top_k) {
   const int64_t c = device_cu_count(), units = top_k / 64, pairs = (int64_t)bs * kv_heads;
   const int cap8 = std::max(1, std::min(kUnitParts, ceil_div(units, 8)));
   const int cap4 = std::max(1, std::min(kUnitParts, ceil_div(units, 4)));
-  if (pairs * units < 8 * c) return {4, cap4};
-  if (pairs <= c) return {8, (int)std::max<int64_t>(1, std::min<int64_t>(cap8, c / pairs))};
-  return {4, std::max(1, std::min(cap4, ceil_div(2 * c, pairs)))};
+  if (units <= 4 * cap4 && pairs * cap4 <= c) return {4, cap4};
+  if (pairs <= c) {
+    const int p8 = (int)std::max<int64_t>(1, std::min<int64_t>(cap8, c / pairs));
+    const int p4 = (int)std::max<int64_t>(1, std::min<int64_t>(cap4, 2 * c / pairs));
+    if (ceil_div(units, 4 * p4) < ceil_div(units, 8 * p8)) return {4, p4};
+    return {8, p8};
+  }
+  return {4, std::min(cap4, 3 * pairs <= 4 * c ? 3 : 5 * pairs <= 8 * c ? 2 : 1)};
 }
 
 extern "C" int qq_quest_fused_step(int q_dtype, int kv_dtype, int new_dtype, int num_q_heads, int kv_heads,
