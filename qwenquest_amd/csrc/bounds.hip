@@ -259,34 +259,51 @@ __device__ inline uint32_t u16x2_min(uint32_t a, uint32_t b) {
 __device__ inline uint32_t u16x2_max(uint32_t a, uint32_t b) {
   return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2_t, a), __builtin_bit_cast(u16x2_t, b)));
 }
-// max over the halves of (|x| - 1) mod 2^16: >= 0x7F80 exactly when a half is a NaN or a zero
-__device__ inline uint32_t bf16x2_special(uint32_t w) {
-  return __builtin_bit_cast(uint32_t, __builtin_bit_cast(u16x2_t, w & 0x7FFF7FFFu) - (u16x2_t){1, 1});
+// A fold's result as keys is exact unless one of its extremes is a NaN or a zero.  A NaN
+// among the values shows in them: its key lies above +inf's (0xFF80) or below -inf's
+// (0x007F).  A zero that is neither the minimum nor the maximum leaves no trace, so only
+// an extreme that is a zero (0x7FFF, 0x8000) needs the order of the values.
+__device__ inline bool keys_need_order(const uint32_t (&kmn)[4], const uint32_t (&kmx)[4]) {
+  uint32_t nan = 0xFFFFFFFFu, zero = 0xFFFFFFFFu;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const u16x2_t mn = __builtin_bit_cast(u16x2_t, kmn[q]), mx = __builtin_bit_cast(u16x2_t, kmx[q]);
+    nan = u16x2_min(nan, u16x2_min(kmn[q], __builtin_bit_cast(uint32_t, mx - (u16x2_t){0xFF81, 0xFF81})));
+    zero = u16x2_min(zero, u16x2_min(__builtin_bit_cast(uint32_t, mn - (u16x2_t){0x7FFF, 0x7FFF}),
+                                     __builtin_bit_cast(uint32_t, mx - (u16x2_t){0x7FFF, 0x7FFF})));
+  }
+  return min(nan & 0xFFFFu, nan >> 16) <= 0x7Eu || min(zero & 0xFFFFu, zero >> 16) <= 1u;
 }
 
-// The wide fold for C = 512 (KV*D = 4 x 128, bf16): one wave per PPW consecutive pages
-// of one layer, 4 waves per block, no LDS and no barrier.  Lane l holds channels 8l ..
+// The wide fold for C = 512 SL (KV*D = 4 x 128 and 8 x 128, bf16): one wave per PPW
+// consecutive pages of one layer (and, at SL = 2, half of the channels: blockIdx.z),
+// no LDS and no barrier.  Lane l holds channels 8l ..
 // 8l + 7 of every row (one 1 KiB row per load instruction); a page's row indices come in
 // with one load (lane r: row r of a 64-row chunk; the first chunk of every page of the
 // wave is loaded up front) and reach the row loads through readlane, and the rows fold
-// in order in batches of B loads in flight, so ties and NaNs resolve as in a sequential
-// fold: a batch without NaNs and zeros folds as unsigned min / max of monotone 16-bit
-// keys (two channels per instruction), any other batch element by element with
-// torch.minimum / maximum semantics.  A row outside the buffer is not folded (its load
+// in order in batches of B loads in flight, as unsigned min / max of monotone 16-bit keys
+// (two channels per instruction); a batch after which an extreme is a NaN or a zero is
+// folded again from the state before it, element by element with torch.minimum / maximum
+// semantics, so ties and NaNs resolve as in a sequential fold.  (Looking for NaNs and
+// zeros in every element instead cost as much as the fold, and one zero in a page - one
+// in a million of normally distributed keys - sent it through the slow fold, 20 us of a
+// wave: 64 rows of 24 layers at KV*D = 512 32 -> 10 us, 16384 rows of 48 layers 173 ->
+// 159 (5.2 TB/s); at KV*D = 1024, against a block per page, 374 -> 317.)  A row outside the buffer is not folded (its load
 // reads row 0).
-template <int B, int PPW>
+template <int SL, int B, int PPW>
 __global__ __launch_bounds__(kPfThreads) void prefill_bounds_wave_kernel(PrefillArgs a) {
-  constexpr int C = 512;
+  constexpr int C = 512 * SL;
+  const int slice = SL > 1 ? blockIdx.z : 0;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int64_t page0 = ((int64_t)blockIdx.x * (kPfThreads / 64) + wave) * PPW;
   const int li = blockIdx.y;
   const int layer = a.layer_begin + li;
-  if (a.set_counters && page0 == 0 && li == a.n_layers - 1 && lane == 0) {
+  if (a.set_counters && page0 == 0 && slice == 0 && li == a.n_layers - 1 && lane == 0) {
     a.count[a.req] = (int32_t)(a.n - a.full_pages * a.P);
     a.page_idx[a.req] = (int32_t)a.full_pages;
   }
   if (page0 * a.P >= a.n) return;  // wave-uniform
-  const uint4* kl = reinterpret_cast<const uint4*>(a.k_base + (int64_t)li * a.k_layer_stride_bytes);
+  const uint4* kl = reinterpret_cast<const uint4*>(a.k_base + (int64_t)li * a.k_layer_stride_bytes) + slice * 64;
   auto chunk_row = [&](int64_t t0, int cnt) -> int32_t {  // lane r: row t0 + r (-1: none)
     int64_t r = lane < cnt ? load_index(a.idx, a.idx64, t0 + lane) : -1;
     return (int32_t)((r >= 0 && r < a.k_rows) ? r : -1);  // rows < 2^31 (checked by the host)
@@ -323,29 +340,28 @@ __global__ __launch_bounds__(kPfThreads) void prefill_bounds_wave_kernel(Prefill
           ok[i] = r >= 0;
           v[i] = kl[(int64_t)(ok[i] ? r : 0) * (C / 8) + lane];
         }
-        uint32_t sp = 0;  // a NaN or a zero in the batch, or a NaN already folded (it must stay)
+        uint32_t nmn[4], nmx[4];
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-          sp = u16x2_max(sp, u16x2_max(bf16x2_special(bf16x2_unkey(kmn[q])), bf16x2_special(bf16x2_unkey(kmx[q]))));
+        for (int q = 0; q < 4; ++q) {
+          nmn[q] = kmn[q];
+          nmx[q] = kmx[q];
+        }
 #pragma unroll
         for (int i = 0; i < B; ++i) {
           if (!ok[i]) continue;  // wave-uniform
-          sp = u16x2_max(sp, u16x2_max(u16x2_max(bf16x2_special(v[i].x), bf16x2_special(v[i].y)),
-                                       u16x2_max(bf16x2_special(v[i].z), bf16x2_special(v[i].w))));
+          const uint32_t w[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const uint32_t kw = bf16x2_key(w[q]);
+            nmn[q] = u16x2_min(nmn[q], kw);
+            nmx[q] = u16x2_max(nmx[q], kw);
+          }
         }
-        const bool special = (sp & 0xFFFFu) >= 0x7F80u || (sp >> 16) >= 0x7F80u;
-        if (!__builtin_amdgcn_ballot_w64(special)) {
-          // no NaN and no zero in the batch or the fold so far: unsigned min / max of the keys
+        if (!__builtin_amdgcn_ballot_w64(keys_need_order(nmn, nmx))) {
 #pragma unroll
-          for (int i = 0; i < B; ++i) {
-            if (!ok[i]) continue;
-            const uint32_t w[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              const uint32_t kw = bf16x2_key(w[q]);
-              kmn[q] = u16x2_min(kmn[q], kw);
-              kmx[q] = u16x2_max(kmx[q], kw);
-            }
+          for (int q = 0; q < 4; ++q) {
+            kmn[q] = nmn[q];
+            kmx[q] = nmx[q];
           }
         } else {
           // NaNs or zeros: torch.minimum / maximum element by element, in row order
@@ -378,7 +394,7 @@ __global__ __launch_bounds__(kPfThreads) void prefill_bounds_wave_kernel(Prefill
       mx[2 * q] = (uint16_t)bmx;
       mx[2 * q + 1] = (uint16_t)(bmx >> 16);
     }
-    const int c0 = lane * 8;
+    const int c0 = slice * 512 + lane * 8;
     if (page < a.full_pages) {
       if (page < a.MP) {
         uint32_t* dst = a.bounds + (((int64_t)layer * a.R + a.req) * a.MP + page) * C + c0;
@@ -401,6 +417,159 @@ __global__ __launch_bounds__(kPfThreads) void prefill_bounds_wave_kernel(Prefill
         a.rmin[rc + e] = mn[e];
         a.rmax[rc + e] = mx[e];
       }
+    }
+  }
+}
+
+// The wide fold for C = 8 L < 512 (KV*D = 2 x 128 and 1 x 128, bf16): one wave per page
+// of one layer, no LDS and no barrier.  A load instruction reads one row in each of the
+// wave's 64 / L lane groups; group g takes the g-th run of consecutive rows of a chunk of
+// 16 rows per group, all of its loads in flight at once.  The chunk folds as keys, whatever the
+// order; where that does not do (keys_need_order) element by element in each group, and
+// the groups' results fold in group order, which is the rows' order.
+//
+// Bound: HBM.  16384 rows over 48 layers, against a block per page that folds every
+// element by itself: KV*D = 256 121 -> 76 us (5.4 TB/s), 128 94 -> 36 (5.8 TB/s); 32-row
+// runs at KV*D = 256 take 256 VGPRs and 81 us.
+template <int L>
+__global__ __launch_bounds__(kPfThreads) void prefill_bounds_groups_kernel(PrefillArgs a) {
+  constexpr int C = 8 * L, GR = 64 / L, B = 16, CH = B * GR;
+  static_assert(L == 16 || L == 32, "two or four rows per load");
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int sub = lane % L, grp = lane / L;
+  const int64_t page = (int64_t)blockIdx.x * (kPfThreads / 64) + wave;
+  const int li = blockIdx.y;
+  const int layer = a.layer_begin + li;
+  if (a.set_counters && page == 0 && li == a.n_layers - 1 && lane == 0) {
+    a.count[a.req] = (int32_t)(a.n - a.full_pages * a.P);
+    a.page_idx[a.req] = (int32_t)a.full_pages;
+  }
+  const int64_t begin = page * a.P;
+  if (begin >= a.n) return;  // wave-uniform
+  const int64_t end = min(begin + (int64_t)a.P, a.n);
+  const uint4* kl = reinterpret_cast<const uint4*>(a.k_base + (int64_t)li * a.k_layer_stride_bytes) + sub;
+  // the fold so far (the same in every group) as keys of channel pairs (8 sub + 2q, + 1)
+  uint32_t kmn[4], kmx[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    kmn[q] = 0xFF80FF80u;
+    kmx[q] = 0x007F007Fu;
+  }
+  for (int64_t t0 = begin; t0 < end && a.k_rows > 0; t0 += CH) {  // no rows: sentinels
+    const int cnt = (int)min((int64_t)CH, end - t0);
+    const int64_t idx = lane < cnt ? load_index(a.idx, a.idx64, t0 + lane) : -1;
+    const int32_t row32 = (int32_t)((idx >= 0 && idx < a.k_rows) ? idx : -1);  // rows < 2^31 (checked by the host)
+    const int per = (cnt + GR - 1) / GR;
+    uint4 v[B];
+    int r[B];  // -1: no row (its load reads row 0)
+#pragma unroll
+    for (int i = 0; i < B; ++i) {
+      const int t = grp * per + i;
+      const int x = __shfl(row32, t & (CH - 1), 64);
+      r[i] = i < per && t < cnt ? x : -1;
+      v[i] = kl[(int64_t)max(r[i], 0) * L];
+    }
+    bool whole = true;
+#pragma unroll
+    for (int i = 0; i < B; ++i) whole &= r[i] >= 0;
+    uint32_t nmn[4], nmx[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      nmn[q] = kmn[q];
+      nmx[q] = kmx[q];
+    }
+    if (!__builtin_amdgcn_ballot_w64(!whole)) {
+#pragma unroll
+      for (int i = 0; i < B; ++i) {
+        const uint32_t w[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const uint32_t kw = bf16x2_key(w[q]);
+          nmn[q] = u16x2_min(nmn[q], kw);
+          nmx[q] = u16x2_max(nmx[q], kw);
+        }
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < B; ++i) {
+        const uint32_t w[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
+        const uint32_t none = r[i] < 0 ? 0xFFFFFFFFu : 0u;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const uint32_t kw = bf16x2_key(w[q]);
+          nmn[q] = u16x2_min(nmn[q], kw | none);
+          nmx[q] = u16x2_max(nmx[q], kw & ~none);
+        }
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+#pragma unroll
+      for (int d = L; d < 64; d <<= 1) {
+        nmn[q] = u16x2_min(nmn[q], (uint32_t)__shfl_xor((int)nmn[q], d, 64));
+        nmx[q] = u16x2_max(nmx[q], (uint32_t)__shfl_xor((int)nmx[q], d, 64));
+      }
+    }
+    if (!__builtin_amdgcn_ballot_w64(keys_need_order(nmn, nmx))) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        kmn[q] = nmn[q];
+        kmx[q] = nmx[q];
+      }
+    } else {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        uint16_t gmn[2] = {0x7F80, 0x7F80}, gmx[2] = {0xFF80, 0xFF80};  // this group's rows
+#pragma unroll
+        for (int i = 0; i < B; ++i) {
+          if (r[i] < 0) continue;
+          const uint32_t w = q == 0 ? v[i].x : q == 1 ? v[i].y : q == 2 ? v[i].z : v[i].w;
+          gmn[0] = bmin(gmn[0], (uint16_t)w);
+          gmn[1] = bmin(gmn[1], (uint16_t)(w >> 16));
+          gmx[0] = bmax(gmx[0], (uint16_t)w);
+          gmx[1] = bmax(gmx[1], (uint16_t)(w >> 16));
+        }
+        const uint32_t bmn = bf16x2_unkey(kmn[q]), bmx = bf16x2_unkey(kmx[q]);
+        uint16_t mn0 = (uint16_t)bmn, mn1 = (uint16_t)(bmn >> 16);
+        uint16_t mx0 = (uint16_t)bmx, mx1 = (uint16_t)(bmx >> 16);
+        const int pmn = (int)(gmn[0] | ((uint32_t)gmn[1] << 16)), pmx = (int)(gmx[0] | ((uint32_t)gmx[1] << 16));
+#pragma unroll
+        for (int g = 0; g < GR; ++g) {
+          const uint32_t um = (uint32_t)__shfl(pmn, g * L + sub, 64), ux = (uint32_t)__shfl(pmx, g * L + sub, 64);
+          mn0 = bmin(mn0, (uint16_t)um);
+          mn1 = bmin(mn1, (uint16_t)(um >> 16));
+          mx0 = bmax(mx0, (uint16_t)ux);
+          mx1 = bmax(mx1, (uint16_t)(ux >> 16));
+        }
+        kmn[q] = bf16x2_key((uint32_t)mn0 | ((uint32_t)mn1 << 16));
+        kmx[q] = bf16x2_key((uint32_t)mx0 | ((uint32_t)mx1 << 16));
+      }
+    }
+  }
+  if (grp != 0) return;
+  const int c0 = sub * 8;
+  if (page < a.full_pages) {
+    if (page < a.MP) {
+      uint32_t w[8];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const uint32_t bmn = bf16x2_unkey(kmn[q]), bmx = bf16x2_unkey(kmx[q]);
+        w[2 * q] = pack_pair((uint16_t)bmn, (uint16_t)bmx);
+        w[2 * q + 1] = pack_pair((uint16_t)(bmn >> 16), (uint16_t)(bmx >> 16));
+      }
+      uint4* dst = reinterpret_cast<uint4*>(a.bounds + (((int64_t)layer * a.R + a.req) * a.MP + page) * C + c0);
+      dst[0] = make_uint4(w[0], w[1], w[2], w[3]);
+      dst[1] = make_uint4(w[4], w[5], w[6], w[7]);
+    }
+  } else {
+    const int64_t rc = ((int64_t)layer * a.R + a.req) * C + c0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const uint32_t bmn = bf16x2_unkey(kmn[q]), bmx = bf16x2_unkey(kmx[q]);
+      a.rmin[rc + 2 * q] = (uint16_t)bmn;
+      a.rmin[rc + 2 * q + 1] = (uint16_t)(bmn >> 16);
+      a.rmax[rc + 2 * q] = (uint16_t)bmx;
+      a.rmax[rc + 2 * q + 1] = (uint16_t)(bmx >> 16);
     }
   }
 }
@@ -706,8 +875,15 @@ extern "C" int qq_quest_prefill_bounds(const void* k_base, int64_t k_layer_strid
   if (!wide)
     prefill_bounds_kernel<<<grid, kThreads, 0, s>>>(a);
   else if (C == 512 && k_rows <= INT32_MAX)
-    prefill_bounds_wave_kernel<kWaveFoldBatch, kWavePages>
+    prefill_bounds_wave_kernel<1, kWaveFoldBatch, kWavePages>
         <<<dim3(ceil_div(pages, kPfThreads / 64 * kWavePages), n_layers), kPfThreads, 0, s>>>(a);
+  else if (C == 1024 && k_rows <= INT32_MAX)
+    prefill_bounds_wave_kernel<2, kWaveFoldBatch, kWavePages>
+        <<<dim3(ceil_div(pages, kPfThreads / 64 * kWavePages), n_layers, 2), kPfThreads, 0, s>>>(a);
+  else if (C == 256 && k_rows <= INT32_MAX)
+    prefill_bounds_groups_kernel<32><<<dim3(ceil_div(pages, kPfThreads / 64), n_layers), kPfThreads, 0, s>>>(a);
+  else if (C == 128 && k_rows <= INT32_MAX)
+    prefill_bounds_groups_kernel<16><<<dim3(ceil_div(pages, kPfThreads / 64), n_layers), kPfThreads, 0, s>>>(a);
   else if (C == 512)
     prefill_bounds_wide_kernel<64><<<grid, kThreads, 0, s>>>(a);
   else if (C == 1024)

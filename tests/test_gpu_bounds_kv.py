@@ -1,0 +1,35 @@
+"""Prefill page bounds at KV*D = 128, 256 and 1024 (1, 2 and 8 KV heads x 128): the wave-per-page
+folds against the per-element fold of the same keys as fp32 (reference quest.py:231-280)."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from tests.test_gpu_quest import DEV, new_quest, rand_bf16
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("kv", [1, 2, 8])
+@pytest.mark.parametrize("page,n", [(64, 0), (64, 1), (64, 63), (64, 777), (16, 100), (32, 65), (128, 333), (200, 777)])
+@pytest.mark.parametrize("kind", ["plain", "special", "bad_rows"])
+def test_prefill_bounds_match_the_per_element_fold(kv, page, n, kind):
+    pool = rand_bf16((1100, kv, 128), seed=n + page)
+    gen = torch.Generator().manual_seed(kv)
+    if kind == "special":  # NaN, both zeros and both infinities, several to a page
+        bits = pool.view(torch.int16).view(-1)
+        for val in (0x7FC0, 0x0000, -0x8000, 0x7F80, 0xFF80 - 65536):
+            bits[torch.randint(0, bits.numel(), (60 * kv,), generator=gen)] = val
+    idx = torch.randperm(1100, generator=gen)[:n].to(torch.int32 if page != 128 else torch.int64)
+    if kind == "bad_rows" and n > 3:
+        idx[[0, n // 2, n - 1]] = torch.tensor([-1, 5000, 1100], dtype=idx.dtype)
+    qb, _ = new_quest(page * 4, page, 2, 4, 1024, kv, 128)
+    qf, _ = new_quest(page * 4, page, 2, 4, 1024, kv, 128)
+    for layer in range(2):
+        qb.update_prefill_representations(layer, 2, pool.to(DEV), idx.to(DEV))
+        qf.update_prefill_representations(layer, 2, pool.float().to(DEV), idx.to(DEV))
+    for name in ("page_k_bounds", "running_k_min", "running_k_max"):
+        assert torch.equal(getattr(qb, name).view(torch.int16), getattr(qf, name).view(torch.int16)), name
+    for name in ("running_token_count", "running_page_idx"):
+        assert torch.equal(getattr(qb, name), getattr(qf, name)), name
