@@ -218,33 +218,71 @@ __device__ inline float reduce8_pages(float (&acc)[8], int lane) {
   return v;
 }
 
-// Bounds words of 8 pages for KV*D == 64*M (M a multiple of 4): lane l holds
-// channels [l*M, l*M + M) as M/4 16-byte loads; pages at or past `lim` re-read
+// Lane partials of N = 2, 4 or 8 pages at once: the first log2(N) levels keep half of
+// the pages each, as in reduce8_pages, the others run on one value.  Lane l ends with
+// page l / (64 / N); only the first lane of each page's 64 / N returns the result.
+template <int N>
+__device__ inline float reduce_pages(float (&acc)[N], int lane) {
+  static_assert(N == 2 || N == 4 || N == 8, "pages per wave");
+  if constexpr (N == 8) {
+    return reduce8_pages(acc, lane);
+  } else {
+    const bool up32 = lane & 32, up16 = lane & 16;
+    float v2[N / 2];
+#pragma unroll
+    for (int j = 0; j < N / 2; ++j) {
+      const float send = up32 ? acc[j] : acc[N / 2 + j];
+      const float keep = up32 ? acc[N / 2 + j] : acc[j];
+      v2[j] = __fadd_rn(keep, lane_xor32(send, lane));
+    }
+    float v;
+    if constexpr (N == 4) {
+      const float send = up16 ? v2[0] : v2[1];
+      const float keep = up16 ? v2[1] : v2[0];
+      v = __fadd_rn(keep, lane_xor16(send, lane));
+    } else {
+      v = __fadd_rn(v2[0], lane_xor16(v2[0], lane));
+    }
+    v = __fadd_rn(v, lane_xor8(v));
+    v = __fadd_rn(v, lane_up4(v));
+    v = __fadd_rn(v, lane_xor2(v));
+    return __fadd_rn(v, lane_xor1(v));
+  }
+}
+
+// Bounds words of N pages for KV*D == 64*M (M = 2 or a multiple of 4): lane l holds
+// channels [l*M, l*M + M) as 8- or 16-byte loads; pages at or past `lim` re-read
 // page lim - 1 (their scores are not stored), so every load is unconditional.
-template <int M>
-__device__ inline void load_8pages(uint32_t (&w)[8][M], const uint32_t* req_bounds, int pw, int lim, int lane) {
-  static_assert(M % 4 == 0, "16-byte lane loads");
+template <int M, int N>
+__device__ inline void load_pages(uint32_t (&w)[N][M], const uint32_t* req_bounds, int pw, int lim, int lane) {
+  static_assert(M == 2 || M % 4 == 0, "8- or 16-byte lane loads");
   constexpr int C = 64 * M;
   const uint32_t lane_bytes = (uint32_t)lane * (M * 4);
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
+  for (int i = 0; i < N; ++i) {
     const char* page = reinterpret_cast<const char*>(req_bounds + (int64_t)min(pw + i, lim - 1) * C);
+    if constexpr (M == 2) {
+      const uint2 v = *reinterpret_cast<const uint2*>(page + lane_bytes);
+      w[i][0] = v.x;
+      w[i][1] = v.y;
+    } else {
 #pragma unroll
-    for (int j = 0; j < M / 4; ++j) {
-      const uint4 v = *reinterpret_cast<const uint4*>(page + lane_bytes + 16 * j);
-      w[i][4 * j] = v.x;
-      w[i][4 * j + 1] = v.y;
-      w[i][4 * j + 2] = v.z;
-      w[i][4 * j + 3] = v.w;
+      for (int j = 0; j < M / 4; ++j) {
+        const uint4 v = *reinterpret_cast<const uint4*>(page + lane_bytes + 16 * j);
+        w[i][4 * j] = v.x;
+        w[i][4 * j + 1] = v.y;
+        w[i][4 * j + 2] = v.z;
+        w[i][4 * j + 3] = v.w;
+      }
     }
   }
 }
 
-// Scores of the 8 pages in w (quest.py:393-405): min or max picked by q-bar's
+// Scores of the N pages in w (quest.py:393-405): min or max picked by q-bar's
 // sign with one byte permute per channel, fp32 products summed in channel
-// order, then the halving tree.  Lane l returns page l >> 3.
-template <int M>
-__device__ inline float score_8pages(const uint32_t (&w)[8][M], const float* s_q, int lane) {
+// order, then the halving tree.  Lane l returns page l / (64 / N).
+template <int M, int N>
+__device__ inline float score_pages(const uint32_t (&w)[N][M], const float* s_q, int lane) {
   float qreg[M];
   uint32_t sel[M];  // v_perm selector: max (high half) for q >= 0, else min, into bits 31:16
 #pragma unroll
@@ -252,16 +290,16 @@ __device__ inline float score_8pages(const uint32_t (&w)[8][M], const float* s_q
     qreg[j] = s_q[lane * M + j];
     sel[j] = qreg[j] >= 0.0f ? 0x03020C0Cu : 0x01000C0Cu;
   }
-  float acc[8];
+  float acc[N];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
+  for (int i = 0; i < N; ++i) {
     float t = __fmul_rn(qreg[0], __uint_as_float(__builtin_amdgcn_perm(w[i][0], w[i][0], sel[0])));
 #pragma unroll
     for (int j = 1; j < M; ++j)
       t = __fadd_rn(t, __fmul_rn(qreg[j], __uint_as_float(__builtin_amdgcn_perm(w[i][j], w[i][j], sel[j]))));
     acc[i] = t;
   }
-  return reduce8_pages(acc, lane);
+  return reduce_pages<N>(acc, lane);
 }
 
 // ----------------------------------------------------------------- selection

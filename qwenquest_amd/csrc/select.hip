@@ -138,25 +138,25 @@ __global__ __launch_bounds__(kThreads) void score_candidates_kernel(SelectArgs a
   if ((lane & 7) == 0 && p < lim) a.scores[(int64_t)b * a.MP + p] = v;
 }
 
-// score_candidates_kernel for KV*D == 64*M (M a multiple of 4): lane l holds
-// channels [l*M, l*M + M) as M/4 16-byte loads.  The page addresses are wave
-// uniform (scalar base + the lane's offset), min-or-max is one byte permute per
-// channel picked by q-bar's sign, and the products and sums are the same fp32
-// operations in the same order as lane_partial.  Pages past the candidate limit
+// score_candidates_kernel for KV*D == 64*M (M = 2 or a multiple of 4), N pages per
+// wave: lane l holds channels [l*M, l*M + M) as 8- or 16-byte loads.  The page
+// addresses are wave uniform (scalar base + the lane's offset), min-or-max is one byte
+// permute per channel picked by q-bar's sign, and the products and sums are the same
+// fp32 operations in the same order as lane_partial.  Pages past the candidate limit
 // re-read the limit's last page and are not stored, so every load is issued
 // unconditionally.
 //
 // Tile 0 of a request also stores the new token's K/V (set_kv_buffer); its
 // loads go out with the page loads and its stores after the scores, so that
 // the block's pages are not held back by the copy's round trips.
-template <int M>
+template <int M, int N>
 __global__ __launch_bounds__(kThreads) void score_pages_fast_kernel(SelectArgs a, int store_new) {
   constexpr int C = 64 * M;
   const int b = blockIdx.y;
   const int64_t s = a.seq[b];
   const int lim = min(a.limit[b], a.MP);
   const int64_t req = a.rpi[b];
-  const int p0 = blockIdx.x * a.ppb;
+  const int p0 = blockIdx.x * (kBlockWaves * N);
   const bool copy_new = store_new && blockIdx.x == 0;
   if (s <= a.top_k || a.k_sel == 0 || p0 >= lim || req < 0 || req >= a.R) {
     if (copy_new) store_new_token(a, b);
@@ -195,9 +195,9 @@ __global__ __launch_bounds__(kThreads) void score_pages_fast_kernel(SelectArgs a
   }
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  const int pw = p0 + wave * 8;  // this wave's 8 pages
-  uint32_t w[8][M];
-  load_8pages<M>(w, a.bounds_layer + req * a.MP * C, pw, lim, lane);
+  const int pw = p0 + wave * N;  // this wave's pages
+  uint32_t w[N][M];
+  load_pages<M, N>(w, a.bounds_layer + req * a.MP * C, pw, lim, lane);
   __shared__ float s_q[kMaxC];
   if (q_early) {
 #pragma unroll
@@ -221,9 +221,10 @@ __global__ __launch_bounds__(kThreads) void score_pages_fast_kernel(SelectArgs a
   }
   lds_barrier();  // s_q is written; the page loads stay in flight
   if (pw < lim) {
-    const float v = score_8pages<M>(w, s_q, lane);
-    const int p = pw + (lane >> 3);
-    if ((lane & 7) == 0 && p < lim) a.scores[(int64_t)b * a.MP + p] = v;
+    const float v = score_pages<M, N>(w, s_q, lane);
+    constexpr int kLanes = 64 / N;  // per page
+    const int p = pw + lane / kLanes;
+    if (lane % kLanes == 0 && p < lim) a.scores[(int64_t)b * a.MP + p] = v;
   }
   if (copy_fast) {
     if (threadIdx.x < C / 8 && loc >= 0 && loc < a.pool_rows) {
@@ -248,7 +249,7 @@ __global__ __launch_bounds__(kThreads) void score_pages_fast_kernel(SelectArgs a
 // (second half).  Their sum is the tree's first level; the levels 16 .. 1 pair
 // odd lanes 32, 16, 8, 4 and 2 apart, the 4 pages' trees interleaved as in
 // reduce8_pages.  Lane 16p + 1 ends with page p's score, bit-identical to
-// score_8pages.  The query words of the GQA mean are loaded unconditionally (heads
+// score_pages.  The query words of the GQA mean are loaded unconditionally (heads
 // past G re-read the last one and are not summed).  One extra block per request
 // (blockIdx.x == 0; page tiles follow it) stores the new token's K/V, so that its
 // registers are not held across the page loads.
@@ -576,6 +577,7 @@ void launch_select(const SelectArgs& a, int bs, int max_pages, int k_sel, hipStr
 
 int launch_score(const SelectArgs& a, int bs, bool store_new, hipStream_t s) {
   dim3 grid(max(1, ceil_div(a.MP, kPagesPerBlock)), bs);
+  auto pages_grid = [&](int n) { return dim3(max(1, ceil_div(a.MP, kBlockWaves * n)), bs); };
   const int M = (a.C + 63) / 64;
   const int st = store_new ? 1 : 0;
   const int G = a.KV > 0 ? a.H / a.KV : 0;
@@ -583,11 +585,18 @@ int launch_score(const SelectArgs& a, int bs, bool store_new, hipStream_t s) {
     const int tiles = max(1, ceil_div(a.MP, kPagesPerBlock4));
     score_pages_fast4_kernel<<<dim3(tiles + 1, bs), kThreads, 0, s>>>(a, st);
   } else if (a.C == 512)
-    score_pages_fast_kernel<8><<<grid, kThreads, 0, s>>>(a, st);
+    score_pages_fast_kernel<8, 8><<<grid, kThreads, 0, s>>>(a, st);
+  // pages per wave: few of the larger pages, so that a small batch still has waves on
+  // every CU (us per launch: 8 KV heads x 128 at batch 1 x 8K 5.6 with 8, 4.2 with 4, 3.8
+  // with 2, at batch 8 x 32K 7.0, 7.5, 6.6, at 48 x 16K 12.1, 12.5, 11.8; 2 heads at 16 x
+  // 64K 5.9 with 8, 5.6 with 4; 1 head at 60 x 30K 5.6 with 8, 6.4 with 4 and in the
+  // general kernel)
   else if (a.C == 1024)
-    score_pages_fast_kernel<16><<<grid, kThreads, 0, s>>>(a, st);
+    score_pages_fast_kernel<16, 2><<<pages_grid(2), kThreads, 0, s>>>(a, st);
   else if (a.C == 256)
-    score_pages_fast_kernel<4><<<grid, kThreads, 0, s>>>(a, st);
+    score_pages_fast_kernel<4, 4><<<pages_grid(4), kThreads, 0, s>>>(a, st);
+  else if (a.C == 128)
+    score_pages_fast_kernel<2, 8><<<pages_grid(8), kThreads, 0, s>>>(a, st);
   else if (M <= 1)
     score_candidates_kernel<1><<<grid, kThreads, 0, s>>>(a, st);
   else if (M <= 2)

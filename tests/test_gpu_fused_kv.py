@@ -75,3 +75,9 @@ def test_fused_and_four_launch_steps_agree(kv, heads, bs):
     assert torch.equal(be._positions[:bs], pos)
     err, scale = (out.double() - four.double()).abs(), four.double().abs().amax()
     assert float(err.max()) <= 2.0**-7 * float(scale) + 1e-4
+
+
+@pytest.mark.parametrize("kv,group", [(1, 8), (1, 1), (2, 5), (2, 16), (8, 8), (8, 1)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_scores_bit_exact_at_other_pages_per_wave(kv, group, dtype):
+    tq.test_retrieve_scores_bit_exact_in_canonical_order(kv, 128, group, dtype)
