@@ -630,7 +630,7 @@ __global__ __launch_bounds__(64 * kDenseWaves, 2) void dense_attend_kernel(StepA
 // one 4-wave block per (request, KV head, part), blockIdx = (request, KV head) *
 // parts + part.  The layout's slots come in units of 64 (a selected page, or the
 // recent window, or 64 slots of the dense layout); wave w of part p takes units
-// w*parts + p, w*parts + p + W*parts, ... (p*W + w where a wave has one; unit_shape).  Per unit a
+// w*parts + p, w*parts + p + W*parts, ...  (unit_shape).  Per unit a
 // wave resolves its 64 rows itself (lane l: slot 64u + l -> position ->
 // req_to_token), shuffles them into the MFMA lane layouts and issues all 32
 // loads of the unit's K and V slices (32 KiB per wave) at once, then
@@ -723,9 +723,7 @@ __global__ __launch_bounds__(64 * W, 8 / W) void quest_attend_unit_kernel(StepAr
 #pragma unroll
   for (int e = 0; e < 8; ++e) o[e] = float4_t{0.f, 0.f, 0.f, 0.f};
   bool bad = false;
-  // one unit per wave: a part's are consecutive; more: a second round goes over all parts
-  const int u_first = stride_units >= units ? part * W + wave : wave * parts + part;
-  for (int u = u_first; u < units; u += stride_units) {  // wave-uniform
+  for (int u = wave * parts + part; u < units; u += stride_units) {  // wave-uniform
     const int slot = u * P + lane;
     const int valid = min(n - u * P, P);  // real slots of this unit
     int64_t row = 0;
@@ -868,7 +866,7 @@ static bool fused_shape(int q_dtype, int kv_dtype, int new_dtype, int num_q_head
 
 // Launch shape of the unit attention: W waves per block, `parts` blocks per (request,
 // KV head); wave w of part p takes the units w * parts + p, + W * parts, ... one after
-// the other (p * W + w where a wave has one).  The grid is sized to one round of resident blocks, since each block pays
+// the other.  The grid is sized to one round of resident blocks, since each block pays
 // its own selection, row lookups and merge before and after its streaming (us per
 // layer-step, top_k 2048 at 4 KV heads unless said):
 //  * a unit per wave in 4-wave blocks that leave each CU at most one: those (batch 8:
@@ -883,7 +881,8 @@ static bool fused_shape(int q_dtype, int kv_dtype, int new_dtype, int num_q_head
 //    (batch 72: 74.3 in 3, 77.1 in 2; batch 84: 81.4 and 83.0; batch 96: 94.7 and 89.6;
 //    batch 104: 102.2 in 2, 96.3 in 1).
 // A second round of units in a part is dealt over all parts, not to the first ones
-// (batch 20, 32 units over 24 waves: 32.0 -> 28.5).
+// (batch 20, 32 units over 24 waves: 32.0 -> 28.5; choosing the order by whether there
+// is a second round costs batch 1 more, 0.04 us a layer, than the order does).
 struct UnitShape {
   int W, parts;
 };

@@ -36,8 +36,7 @@ def test_every_unit_belongs_to_one_wave(kv, top_k):
         taken = []
         for part in range(parts):
             for wave in range(W):
-                first = part * W + wave if parts * W >= units else wave * parts + part
-                taken += range(first, units, parts * W)
+                taken += range(wave * parts + part, units, parts * W)
         assert sorted(taken) == list(range(units))
         if bs * kv <= CUS:  # one round of resident blocks
             assert bs * kv * parts <= (2 * CUS if W == 4 else CUS)
