@@ -60,7 +60,7 @@ struct ExtendArgs {
   const int64_t* prefix;
   const int64_t* ext;
   int bs, n;
-  int tiles;   // query tiles the grid holds (an upper bound of the requests' tiles)
+  int tiles;   // query tiles the grid holds (an upper bound of the requests' tiles), one more at its end
   int splits;  // K/V splits the grid holds
   float sl2;   // scale * log2(e)
   uint16_t* out;
@@ -170,18 +170,24 @@ __global__ __launch_bounds__(64 * kExtWaves, 2) void extend_kernel(ExtendArgs a)
   // of the requests, which attend the most, first
   const int h = blockIdx.x % a.KV;
   const int rest = blockIdx.x / a.KV;
-  const int t_lin = a.tiles - 1 - rest % a.tiles;
-  const int split = rest / a.tiles;
+  const bool tail = rest >= a.tiles * a.splits;  // the grid's last tile, past every request's
+  const int t_lin = tail ? a.tiles : a.tiles - 1 - rest % a.tiles;
+  const int split = tail ? 0 : rest / a.tiles;
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int lo = lane & 31, hf = lane >> 5;
   const ExtendTile et = find_tile(a, t_lin);
   const int64_t row_out = (int64_t)a.H * kMfmaDim;
   if (et.b < 0) {
-    // rows of q past the requests' tokens have no answer; normally none
-    if (split == 0 && et.q0 < a.n && et.past == 0)
-      for (int64_t i = tid; i < (int64_t)(a.n - et.q0) * a.G * kMfmaDim; i += 64 * kExtWaves)
-        a.out[(et.q0 + i / (a.G * kMfmaDim)) * row_out + (int64_t)h * a.G * kMfmaDim + i % (a.G * kMfmaDim)] = 0x7FC0;
+    // rows of q past the requests' tokens have no answer (normally there are none): NaN, in
+    // 8-byte pieces, shared by the tiles past the requests' - the grid's last one always is
+    const int past_tiles = a.tiles + 1 - (t_lin - et.past);
+    const int pieces = a.G * kMfmaDim / 4;  // of a row, per KV head
+    if (split == 0)
+      for (int64_t i = et.past * 64 * kExtWaves + tid; i < (int64_t)(a.n - et.q0) * pieces;
+           i += (int64_t)past_tiles * 64 * kExtWaves)
+        *reinterpret_cast<uint2*>(a.out + (et.q0 + i / pieces) * row_out + ((int64_t)h * pieces + i % pieces) * 4) =
+            make_uint2(0x7FC07FC0u, 0x7FC07FC0u);
     return;
   }
   const int kv_len = et.kv_len, prefix = et.prefix;
@@ -506,7 +512,8 @@ extern "C" int qq_extend_attention(const void* q, int num_q_heads, const void* k
   a.n = (int)n;
   const int64_t tiles = extend_tiles(n, bs, a.G);
   a.splits = extend_splits(tiles, kv_heads, req_to_token_stride);
-  QQ_REQUIRE(tiles * kv_heads * a.splits < (int64_t)1 << 31, "%s: too many query rows", what);
+  const int64_t grid = (tiles * a.splits + 1) * kv_heads;
+  QQ_REQUIRE(grid < (int64_t)1 << 31, "%s: too many query rows", what);
   a.tiles = (int)tiles;
   a.sl2 = scale * kLog2e;
   a.out = static_cast<uint16_t*>(out);
@@ -514,7 +521,7 @@ extern "C" int qq_extend_attention(const void* q, int num_q_heads, const void* k
   a.part_ml = a.part_o ? a.part_o + a.splits * kv_heads * tiles * kExtRows * kMfmaDim : nullptr;
   hipStream_t s = static_cast<hipStream_t>(stream);
   constexpr size_t kSmem = 4 * kTileElems * sizeof(uint16_t);  // 64 KiB: two buffers of K and V
-  extend_kernel<<<(int)(tiles * kv_heads * a.splits), 64 * kExtWaves, kSmem, s>>>(a);
+  extend_kernel<<<(int)grid, 64 * kExtWaves, kSmem, s>>>(a);
   if (a.splits > 1)
     extend_merge_kernel<<<dim3(a.tiles, kv_heads, kExtRows / 8), 256, 0, s>>>(a);
   return check_launch(what);

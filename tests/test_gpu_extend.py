@@ -149,3 +149,34 @@ def test_extend_batch_rows_outside_their_tables():
     got = be.forward_extend(q, k, v, layer, batch)
     batch.seq_lens[1] = r2t.shape[1]
     assert torch.equal(be.forward_extend(q, k, v, layer, batch), got)
+
+
+@pytest.mark.parametrize("H,KV,n,ext", [
+    (32, 4, 6, [5]),  # the request's partial tile is the last one that the rows can fill
+    (32, 4, 31, [30]),
+    (4, 4, 255, [254]),
+    (8, 2, 63, [50, 12]),
+    (32, 4, 700, [33, 1, 17]),  # many tiles past the requests'
+    (20, 4, 40, [0, 0]),  # no tokens at all
+])
+def test_rows_past_the_requests_tokens_are_nan(H, KV, n, ext):
+    """q with more rows than the requests have tokens: the rows past them are written."""
+    from qwenquest_amd.attention.ops import extend_attention_batch
+
+    be, q, k, v, batch, layer, slots = make([max(e, 1) for e in ext], [3] * len(ext), H, KV, 7)
+    lens = torch.tensor(ext, device=DEV)
+    total = sum(ext)
+    k_buf, v_buf = batch.token_to_kv_pool.get_kv_buffer(0)
+    qp = torch.ones((n, H, 128), dtype=torch.bfloat16, device=DEV)
+    qp[:total] = q[:total]
+
+    def call(x):
+        stale = [torch.ones((n, H * 128), dtype=torch.bfloat16, device=DEV) for _ in range(4)]
+        del stale  # the output's memory holds numbers before the call
+        return extend_attention_batch(x, k_buf, v_buf, be.req_to_token, batch.req_pool_indices, lens + 3,
+                                      batch.extend_prefix_lens, lens, layer.scaling)
+
+    got = call(qp)
+    assert got.shape == (n, H * 128) and bool(got[total:].isnan().all())
+    if total:
+        assert torch.equal(got[:total], call(qp[:total].contiguous()))
