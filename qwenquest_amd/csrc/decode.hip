@@ -125,6 +125,7 @@ __device__ inline void attend_unit(int r32, int valid, const uint16_t* kb, const
   mx = fmaxf(mx, lane_xor32(mx, lane));
   const float Mn = fmaxf(M, mx);
   const float alpha = M == -INFINITY ? 0.0f : exp2f(M - Mn);  // rescale of the running sums
+  const float Mb = Mn == -INFINITY ? 0.0f : Mn;  // every score so far -inf: weights of 0, not of NaN
   float sum = 0.0f;
   short4_t pa[4];
 #pragma unroll
@@ -134,7 +135,7 @@ __device__ inline void attend_unit(int r32, int valid, const uint16_t* kb, const
       // v_exp_f32 as it is (exp2f adds a rescale for results below 2^-126, which only
       // the weights of rows 126 binary orders under the maximum reach) and the hardware's
       // round-to-nearest-even bf16 conversion, equal to f2bf for every value that is not NaN
-      const uint16_t pbits = __builtin_bit_cast(uint16_t, (__bf16)__builtin_amdgcn_exp2f(acc[t][i] - Mn));
+      const uint16_t pbits = __builtin_bit_cast(uint16_t, (__bf16)__builtin_amdgcn_exp2f(acc[t][i] - Mb));
       sum += bf2f(pbits);
       pa[t][i] = (short)pbits;
     }
