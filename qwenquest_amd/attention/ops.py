@@ -13,7 +13,7 @@ import torch.nn.functional as F
 
 from qwenquest_amd import _lib
 
-__all__ = ["decode_attention", "extend_attention", "extend_attention_batch", "AttentionWorkspace"]
+__all__ = ["decode_attention", "extend_attention", "extend_attention_batch", "AttentionWorkspace", "ExtendLengths"]
 
 
 class AttentionWorkspace:
@@ -103,6 +103,47 @@ def extend_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, prefix_l
     return out[0].transpose(0, 1).reshape(n, num_heads * head_dim).to(q.dtype)
 
 
+class ExtendLengths:
+    """The request indices and lengths of a prefill batch, on the device and on the host.
+
+    The host's copy is under way when the constructor returns and is waited for by ``rows``, so
+    that what is launched in between runs behind it: the wait is one for the work before the
+    constructor, and the device is not left idle.  Inside a graph capture there is none.
+    """
+
+    def __init__(self, req_pool_indices: torch.Tensor, seq_lens: torch.Tensor, prefix_lens: torch.Tensor,
+                 extend_lens: torch.Tensor, device: torch.device):
+        bs = req_pool_indices.shape[0]
+        words = [t[:bs] for t in (req_pool_indices, seq_lens, prefix_lens, extend_lens)]
+        self._ready = None
+        if torch.cuda.is_current_stream_capturing():
+            self.device = words
+            self._host = None
+        elif all(not t.is_cuda for t in words):
+            self._host = torch.stack([t.to(torch.int64) for t in words])
+            self.device = self._host.to(device).unbind(0)
+        else:
+            both = torch.stack([t.to(device=device, dtype=torch.int64) for t in words])
+            self._host = both.to("cpu", non_blocking=True)  # into pinned memory
+            self._ready = torch.cuda.Event()
+            self._ready.record(torch.cuda.current_stream(device))
+            self.device = both.unbind(0)
+
+    def rows(self, n: int, table_rows: int) -> int | None:
+        """How many of the ``n`` rows of q belong to the requests; None for a batch that the
+        request-by-request path treats in another way (or refuses)."""
+        if self._host is None:
+            return n
+        if self._ready is not None:
+            self._ready.synchronize()
+        total = 0
+        for req, seq, prefix, new in zip(*self._host.tolist(), strict=True):
+            if not -table_rows <= req < table_rows or new < 0 or (new > 0 and (seq < 1 or prefix < 0)):
+                return None
+            total += new
+        return min(total, n)
+
+
 def extend_attention_batch(
     q: torch.Tensor,
     k_buf: torch.Tensor,
@@ -116,7 +157,9 @@ def extend_attention_batch(
 ) -> torch.Tensor:
     """Dense causal prefill of a batch (the loop of base.py:65-93): ``q [n, H, 128]`` holds the
     requests' new tokens one request after the other, ``k_buf``/``v_buf [rows, KV, 128]`` the
-    pool with the new K/V in it.  bf16; returns ``[n, H*128]``.  No host synchronisation."""
+    pool with the new K/V in it.  bf16; returns ``[n, H*128]``.  The lengths (each ``[>= bs]``)
+    are read on the device only; a request whose index lies outside the table gets NaN, as do
+    rows of q past the requests' tokens."""
     n, heads, dim = q.shape
     kv, bs, dev = k_buf.shape[1], int(req_pool_indices.shape[0]), q.device
     q = q.contiguous()

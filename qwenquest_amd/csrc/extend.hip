@@ -90,7 +90,7 @@ __device__ inline ExtendTile find_tile(const ExtendArgs& a, int t) {
     const int b = b0 + lane;
     // the request's four words go out together
     const int64_t len = b < a.bs ? a.ext[b] : 0;
-    const int64_t req = b < a.bs ? a.rpi[b] : -1;
+    const int64_t req = b < a.bs ? a.rpi[b] : 0;
     const int64_t seq = b < a.bs ? a.seq[b] : 0;
     const int64_t prefix = b < a.bs ? a.prefix[b] : 0;
     int n = (int)min(max(len, (int64_t)0), (int64_t)a.n);
@@ -120,7 +120,8 @@ __device__ inline ExtendTile find_tile(const ExtendArgs& a, int t) {
       r.q0 = __shfl(first, src, 64);
       r.n = __shfl(n, src, 64);
       r.past = 0;
-      r.req = __shfl(req >= 0 && req < a.r2t_rows ? (int)req : -1, src, 64);
+      const int64_t row = req < 0 ? req + a.r2t_rows : req;  // a negative index counts from the table's end
+      r.req = __shfl(row >= 0 && row < a.r2t_rows ? (int)row : -1, src, 64);
       const int kv = (int)min(max(seq, (int64_t)0), a.r2t_stride);
       r.kv_len = r.req >= 0 ? __shfl(kv, src, 64) : 0;  // wave-uniform branch
       r.prefix = __shfl((int)min(max(prefix, -(int64_t)(1 << 30)), (int64_t)(1 << 30)), src, 64);

@@ -46,6 +46,15 @@ def make(new, prefix, H, KV, seed, width=None, qscale=1.0):
     return be, q, k, v, batch, Layer(D), slots
 
 
+def launch(be, q, batch, layer):
+    """The launch alone, as a captured call runs it: nothing is read on the host."""
+    from qwenquest_amd.attention.ops import extend_attention_batch
+
+    k_buf, v_buf = batch.token_to_kv_pool.get_kv_buffer(0)
+    return extend_attention_batch(q, k_buf, v_buf, be.req_to_token, batch.req_pool_indices, batch.seq_lens,
+                                  batch.extend_prefix_lens, batch.extend_seq_lens, layer.scaling)
+
+
 def exact(batch, slots, q, new, prefix, KV):
     """float64 causal attention over the pool's rows."""
     kvp, r2t = batch.token_to_kv_pool, batch.req_to_token_pool.req_to_token
@@ -125,14 +134,19 @@ def test_extend_batch_sharp_scores_and_other_forms():
 
 
 def test_extend_batch_rows_outside_their_tables():
-    """A request with a row past the pool, or past the table, gets NaN; the others their answer;
-    a context longer than the table is cut to it, as a slice is."""
+    """A request index past the table raises, a row past the pool gives NaN, the others get their
+    answer, and negative ones count from the end; a context longer than the table is cut to it, as a slice is."""
     new, prefix = [40, 50, 60], [0, 30, 0]
     be, q, k, v, batch, layer, slots = make(new, prefix, 32, 4, 5)
     want = be.forward_extend(q, k, v, layer, batch)
     batch.req_pool_indices[2] = 99
-    got = be.forward_extend(q, k, v, layer, batch)
+    with pytest.raises(IndexError):  # as the request-by-request path
+        be.forward_extend(q, k, v, layer, batch)
+    got = launch(be, q, batch, layer)
     assert torch.equal(got[:90], want[:90]) and bool(got[90:].isnan().all())
+    batch.req_pool_indices[2] = slots[2] - batch.req_to_token_pool.size  # counts from the table's end
+    assert torch.equal(be.forward_extend(q, k, v, layer, batch), want)
+    assert torch.equal(launch(be, q, batch, layer), want)
     batch.req_pool_indices[2] = slots[2]
     r2t = batch.req_to_token_pool.req_to_token
     keep = int(r2t[slots[1], 10])
@@ -180,3 +194,52 @@ def test_rows_past_the_requests_tokens_are_nan(H, KV, n, ext):
     assert got.shape == (n, H * 128) and bool(got[total:].isnan().all())
     if total:
         assert torch.equal(got[:total], call(qp[:total].contiguous()))
+
+
+@pytest.mark.parametrize("where", ["cuda", "cpu"])
+def test_calls_that_the_request_by_request_path_takes_or_refuses(where, monkeypatch):
+    """The batched path against the loop over the forms of a call: the same rows, values to one
+    rounding of each, and the same refusals."""
+    new, prefix = [40, 0, 30], [0, 5, 70]
+    be, q, k, v, batch, layer, slots = make(new, prefix, 8, 2, 11)
+    names = ("req_pool_indices", "seq_lens", "extend_prefix_lens", "extend_seq_lens")
+    for name in names:
+        setattr(batch, name, getattr(batch, name).to(where))
+    fields = {name: getattr(batch, name) for name in names}
+    fast = be._extend_fast
+
+    def both(q=q, **changed):
+        got = []
+        for loop in (False, True):
+            for name in names:
+                setattr(batch, name, changed.get(name, fields[name]))
+            monkeypatch.setattr(be, "_extend_fast", (lambda *a: False) if loop else fast)
+            try:
+                got.append(be.forward_extend(q, k, v, layer, batch))
+            except (IndexError, RuntimeError) as e:
+                got.append(type(e))
+        a, b = got
+        if isinstance(b, type):
+            assert a is b
+            return a
+        assert a.shape == b.shape
+        err = (a.double() - b.double()).abs()
+        assert bool((err <= 2.0**-7 * b.double().abs() + 2e-5).all())
+        return a
+
+    def t(*x):
+        return torch.tensor(x, device=where)
+
+    full = both()
+    padded = torch.cat([q, torch.ones_like(q[:9])])
+    assert torch.equal(both(q=padded), full)  # the requests' rows and no others
+    assert torch.equal(both(q=q[:60].contiguous()), full[:60])  # fewer: the last request has what is left
+    assert torch.equal(both(req_pool_indices=t(*(s - batch.req_to_token_pool.size for s in slots))), full)
+    assert both(req_pool_indices=t(slots[0], slots[1], batch.req_to_token_pool.size)) is IndexError
+    assert both(req_pool_indices=t(-batch.req_to_token_pool.size - 1, *slots[1:])) is IndexError
+    for name in names[1:]:  # fewer lengths than requests
+        assert both(**{name: fields[name][:2]}) is IndexError
+    for name in names[1:]:  # and more of them
+        assert torch.equal(both(**{name: torch.cat([fields[name], t(7)])}), full)
+    both(extend_seq_lens=t(0, 0, 0), q=q[:0])
+    both(seq_lens=t(40, 5, 10_000))  # longer than the table: cut to its width
