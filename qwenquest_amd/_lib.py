@@ -95,6 +95,11 @@ SIGNATURES: dict[str, tuple] = {
         _I,
         [_P, _I, _P, _P, _L, _I, _I, _P, _L, _L, _P, _P, _P, _P, _I, _L, _F, _P, _P, _L, _P],
     ),
+    "qq_extend_attention_checked": (
+        _I,
+        [_P, _I, _P, _P, _L, _I, _I, _P, _L, _L, _P, _P, _P, _P, _I, _L, _F, _P, _P, _L, _P, _P],
+    ),
+    "qq_extend_verdict_wait": (_I, [_P, _P]),
     "qq_extend_attention_workspace_bytes": (_L, [_L, _I, _I, _I, _L]),
     "qq_kv_scatter": (_I, [_P, _P, _I, _L, _P, _P, _I, _P, _I, _L, _P]),
     "qq_hisparse_swap_in": (

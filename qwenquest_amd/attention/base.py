@@ -12,7 +12,7 @@ from typing import TYPE_CHECKING, Any
 
 import torch
 
-from qwenquest_amd.attention.ops import ExtendLengths, extend_attention, extend_attention_batch
+from qwenquest_amd.attention.ops import extend_attention, extend_attention_batch, extend_attention_batch_checked
 
 if TYPE_CHECKING:
     from qwenquest_amd.batch import ForwardBatch
@@ -49,25 +49,22 @@ class AttentionBackend(ABC):
         """Dense causal prefill: save the new K/V, then attend per request (base.py:65-93).
 
         bf16 with head_dim 128 runs the whole batch in one launch, which reads the lengths
-        on the device; they are read on the host under it, and a batch that the launch does
-        not answer as the loop below does goes through the loop (which raises IndexError for
-        a request index outside the table).  Other shapes go request by request through
-        ``extend_attention``.  Inside a graph capture nothing is read on the host: a request
-        index outside the table gives NaN, and so do rows of ``q`` past the requests' tokens.
+        on the device; a batch that the launch does not answer as the loop below does goes
+        through the loop (which raises IndexError for a request index outside the table).  Other shapes go request by request through
+        ``extend_attention``.  Inside a graph capture, which the loop refuses, a
+        request index outside the table gives NaN, as do rows of ``q`` past the requests' tokens.
         """
         assert batch.out_cache_loc is not None and batch.extend_prefix_lens is not None
         pool = self.token_to_kv_pool
-        fast = self._extend_fast(q, layer.scaling, batch)
-        if fast:
-            lens = ExtendLengths(batch.req_pool_indices, batch.seq_lens, batch.extend_prefix_lens,
-                                 batch.extend_seq_lens, q.device)
         pool.set_kv_buffer(layer.layer_id, batch.out_cache_loc, k, v)
         k_buf, v_buf = pool.get_kv_buffer(layer.layer_id)
-        if fast:
-            out = extend_attention_batch(q, k_buf, v_buf, self.req_to_token, *lens.device, float(layer.scaling))
-            rows = lens.rows(q.shape[0], self.req_to_token.shape[0])
-            if rows is not None:
-                return out if rows == q.shape[0] else out[:rows]
+        if self._extend_fast(q, layer.scaling, batch):
+            attend = (extend_attention_batch if torch.cuda.is_current_stream_capturing()
+                      else extend_attention_batch_checked)
+            out = attend(q, k_buf, v_buf, self.req_to_token, batch.req_pool_indices, batch.seq_lens,
+                         batch.extend_prefix_lens, batch.extend_seq_lens, float(layer.scaling))
+            if out is not None:
+                return out
         offsets = batch.extend_token_offsets()
         outputs = []
         for i in range(batch.batch_size):

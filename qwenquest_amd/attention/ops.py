@@ -13,7 +13,7 @@ import torch.nn.functional as F
 
 from qwenquest_amd import _lib
 
-__all__ = ["decode_attention", "extend_attention", "extend_attention_batch", "AttentionWorkspace", "ExtendLengths"]
+__all__ = ["decode_attention", "extend_attention", "extend_attention_batch", "AttentionWorkspace"]
 
 
 class AttentionWorkspace:
@@ -103,45 +103,40 @@ def extend_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, prefix_l
     return out[0].transpose(0, 1).reshape(n, num_heads * head_dim).to(q.dtype)
 
 
-class ExtendLengths:
-    """The request indices and lengths of a prefill batch, on the device and on the host.
-
-    The host's copy is under way when the constructor returns and is waited for by ``rows``, so
-    that what is launched in between runs behind it: the wait is one for the work before the
-    constructor, and the device is not left idle.  Inside a graph capture there is none.
-    """
-
-    def __init__(self, req_pool_indices: torch.Tensor, seq_lens: torch.Tensor, prefix_lens: torch.Tensor,
-                 extend_lens: torch.Tensor, device: torch.device):
-        bs = req_pool_indices.shape[0]
-        words = [t[:bs] for t in (req_pool_indices, seq_lens, prefix_lens, extend_lens)]
-        self._ready = None
-        if torch.cuda.is_current_stream_capturing():
-            self.device = words
-            self._host = None
-        elif all(not t.is_cuda for t in words):
-            self._host = torch.stack([t.to(torch.int64) for t in words])
-            self.device = self._host.to(device).unbind(0)
-        else:
-            both = torch.stack([t.to(device=device, dtype=torch.int64) for t in words])
-            self._host = both.to("cpu", non_blocking=True)  # into pinned memory
-            self._ready = torch.cuda.Event()
-            self._ready.record(torch.cuda.current_stream(device))
-            self.device = both.unbind(0)
-
-    def rows(self, n: int, table_rows: int) -> int | None:
-        """How many of the ``n`` rows of q belong to the requests; None for a batch that the
-        request-by-request path treats in another way (or refuses)."""
-        if self._host is None:
-            return n
-        if self._ready is not None:
-            self._ready.synchronize()
-        total = 0
-        for req, seq, prefix, new in zip(*self._host.tolist(), strict=True):
-            if not -table_rows <= req < table_rows or new < 0 or (new > 0 and (seq < 1 or prefix < 0)):
-                return None
-            total += new
-        return min(total, n)
+def _extend_launch(
+    q: torch.Tensor,
+    k_buf: torch.Tensor,
+    v_buf: torch.Tensor,
+    req_to_token: torch.Tensor,
+    lens: tuple[torch.Tensor, ...],
+    scaling: float,
+    checked: bool,
+) -> tuple[torch.Tensor, list[int] | None]:
+    """qq_extend_attention; the output, and the verdict on the lengths if asked for."""
+    n, heads, dim = q.shape
+    kv, bs, dev = k_buf.shape[1], int(lens[0].shape[0]), q.device
+    q = q.contiguous()
+    if q.data_ptr() % 16:  # the kernel reads 16-byte pieces
+        q = q.clone()
+    rpi, seq, prefix, ext = (
+        t if t.dtype == torch.int64 and t.device == dev and t.is_contiguous()
+        else t.to(device=dev, dtype=torch.int64).contiguous() for t in lens)
+    need = int(_lib.load().qq_extend_attention_workspace_bytes(n, bs, heads, kv, req_to_token.shape[1]))
+    ws = torch.empty(need, dtype=torch.uint8, device=dev) if need else None
+    out = torch.empty((n, heads * dim), dtype=q.dtype, device=dev)
+    args = (
+        _lib.ptr(q), heads, _lib.ptr(k_buf), _lib.ptr(v_buf), k_buf.shape[0], kv, dim,
+        _lib.ptr(req_to_token), req_to_token.stride(0), req_to_token.shape[0], _lib.ptr(rpi), _lib.ptr(seq),
+        _lib.ptr(prefix), _lib.ptr(ext), bs, n, float(scaling), _lib.ptr(out), _lib.ptr(ws), need,
+    )
+    stream = _lib.stream(dev)
+    if not checked:
+        _lib.call("qq_extend_attention", *args, stream)
+        return out, None
+    verdict = torch.empty(2, dtype=torch.int64, pin_memory=True)
+    _lib.call("qq_extend_attention_checked", *args, verdict.data_ptr(), stream)
+    _lib.call("qq_extend_verdict_wait", verdict.data_ptr(), stream)  # before the words may be freed
+    return out, verdict.tolist()
 
 
 def extend_attention_batch(
@@ -160,23 +155,30 @@ def extend_attention_batch(
     pool with the new K/V in it.  bf16; returns ``[n, H*128]``.  The lengths (each ``[>= bs]``)
     are read on the device only; a request whose index lies outside the table gets NaN, as do
     rows of q past the requests' tokens."""
-    n, heads, dim = q.shape
-    kv, bs, dev = k_buf.shape[1], int(req_pool_indices.shape[0]), q.device
-    q = q.contiguous()
-    if q.data_ptr() % 16:  # the kernel reads 16-byte pieces
-        q = q.clone()
+    lens = (req_pool_indices, seq_lens, prefix_lens, extend_lens)
+    return _extend_launch(q, k_buf, v_buf, req_to_token, lens, scaling, False)[0]
 
-    def lens(t: torch.Tensor) -> torch.Tensor:
-        return t.to(device=dev, dtype=torch.int64).contiguous()
 
-    rpi, seq, prefix, ext = lens(req_pool_indices), lens(seq_lens), lens(prefix_lens), lens(extend_lens)
-    need = int(_lib.load().qq_extend_attention_workspace_bytes(n, bs, heads, kv, req_to_token.shape[1]))
-    ws = torch.empty(need, dtype=torch.uint8, device=dev) if need else None
-    out = torch.empty((n, heads * dim), dtype=q.dtype, device=dev)
-    _lib.call(
-        "qq_extend_attention", _lib.ptr(q), heads, _lib.ptr(k_buf), _lib.ptr(v_buf), k_buf.shape[0], kv, dim,
-        _lib.ptr(req_to_token), req_to_token.stride(0), req_to_token.shape[0], _lib.ptr(rpi), _lib.ptr(seq),
-        _lib.ptr(prefix), _lib.ptr(ext), bs, n, float(scaling), _lib.ptr(out), _lib.ptr(ws), need,
-        _lib.stream(dev),
-    )
-    return out
+def extend_attention_batch_checked(
+    q: torch.Tensor,
+    k_buf: torch.Tensor,
+    v_buf: torch.Tensor,
+    req_to_token: torch.Tensor,
+    req_pool_indices: torch.Tensor,
+    seq_lens: torch.Tensor,
+    prefix_lens: torch.Tensor,
+    extend_lens: torch.Tensor,
+    scaling: float,
+) -> torch.Tensor | None:
+    """``extend_attention_batch`` outside a graph capture: the requests' rows only, and None for a
+    batch that the loop treats in another way (or refuses).
+
+    The launch judges the lengths as it begins and the host waits for that, not for its end: the
+    device is not left idle, and no copy or event is queued (600 new tokens: a stack of the lengths
+    and its copy 52 us, a kernel of its own and an event 43)."""
+    lens = (req_pool_indices, seq_lens, prefix_lens, extend_lens)
+    out, verdict = _extend_launch(q, k_buf, v_buf, req_to_token, lens, scaling, True)
+    irregular, total = verdict
+    if irregular:
+        return None
+    return out if total >= out.shape[0] else out[:total]

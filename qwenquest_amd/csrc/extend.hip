@@ -66,6 +66,7 @@ struct ExtendArgs {
   uint16_t* out;
   float* part_o;   // [splits, KV, tiles, 128 rows, 128]
   float* part_ml;  // [splits, KV, tiles, 128 rows, 2]
+  int64_t* verdict;  // nullptr, or where the first block reports on the lengths
 };
 
 // What a block works on: request, first query row of its tile, the request's rows.
@@ -133,6 +134,25 @@ __device__ inline ExtendTile find_tile(const ExtendArgs& a, int t) {
   return {-1, 0, tok, 0, t - tile, -1, 0, 0};
 }
 
+// qq_extend_attention_checked's verdict, by one wave: host memory, so the words go out at
+// system scope, the one that the host waits for last.
+__device__ inline void report_lengths(const ExtendArgs& a) {
+  const int lane = threadIdx.x & 63;
+  int64_t total = 0;
+  bool irregular = false;
+  for (int b = lane; b < a.bs; b += 64) {
+    const int64_t req = a.rpi[b], n = a.ext[b], s = a.seq[b], p = a.prefix[b];
+    irregular |= req < -a.r2t_rows || req >= a.r2t_rows || n < 0 || (n > 0 && (s < 1 || p < 0));
+    total += n;
+  }
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1) total += __shfl_xor((long long)total, d, 64);
+  const bool any = __any(irregular);
+  if (lane != 0) return;
+  __hip_atomic_store(a.verdict + 1, total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  __hip_atomic_store(a.verdict, any ? 1 : 0, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // K/V tiles per split of a query tile that attends nt of them: equal parts, none
 // shorter than kExtMinChunk.
 __device__ inline int split_chunk(int nt, int splits) {
@@ -177,6 +197,7 @@ __global__ __launch_bounds__(64 * kExtWaves, 2) void extend_kernel(ExtendArgs a)
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int lo = lane & 31, hf = lane >> 5;
+  if (a.verdict && blockIdx.x == 0 && wave == 0) report_lengths(a);
   const ExtendTile et = find_tile(a, t_lin);
   const int64_t row_out = (int64_t)a.H * kMfmaDim;
   if (et.b < 0) {
@@ -478,6 +499,35 @@ extern "C" int qq_extend_attention(const void* q, int num_q_heads, const void* k
                                    const int64_t* req_pool_indices, const int64_t* seq_lens,
                                    const int64_t* prefix_lens, const int64_t* extend_lens, int bs, int64_t n,
                                    float scale, void* out, void* workspace, int64_t workspace_bytes, void* stream) {
+  return qq_extend_attention_checked(q, num_q_heads, k_layer, v_layer, kv_rows, kv_heads, head_dim, req_to_token,
+                                     req_to_token_stride, req_to_token_rows, req_pool_indices, seq_lens, prefix_lens,
+                                     extend_lens, bs, n, scale, out, workspace, workspace_bytes, nullptr, stream);
+}
+
+extern "C" int qq_extend_verdict_wait(const int64_t* verdict, void* stream) {
+  const char* what = "qq_extend_verdict_wait";
+  QQ_REQUIRE(verdict, "%s: null pointer", what);
+  for (;;) {
+    for (int spin = 0; spin < 4096; ++spin) {
+      if (__atomic_load_n(verdict, __ATOMIC_ACQUIRE) >= 0) return QQ_OK;
+      __builtin_ia32_pause();
+    }
+    // the launch reports as it begins; a stream that is done, or in error, has nothing to wait for
+    const hipError_t e = hipStreamQuery(static_cast<hipStream_t>(stream));
+    if (e == hipErrorNotReady) continue;
+    if (e == hipSuccess && __atomic_load_n(verdict, __ATOMIC_ACQUIRE) >= 0) return QQ_OK;
+    set_error(QQ_EHIP, "%s: no verdict: %s", what, hipGetErrorString(e));
+    return QQ_EHIP;
+  }
+}
+
+extern "C" int qq_extend_attention_checked(const void* q, int num_q_heads, const void* k_layer, const void* v_layer,
+                                           int64_t kv_rows, int kv_heads, int head_dim, const int32_t* req_to_token,
+                                           int64_t req_to_token_stride, int64_t req_to_token_rows,
+                                           const int64_t* req_pool_indices, const int64_t* seq_lens,
+                                           const int64_t* prefix_lens, const int64_t* extend_lens, int bs, int64_t n,
+                                           float scale, void* out, void* workspace, int64_t workspace_bytes,
+                                           int64_t* verdict, void* stream) {
   const char* what = "qq_extend_attention";
   QQ_REQUIRE(kv_heads > 0 && num_q_heads > 0 && num_q_heads % kv_heads == 0,
              "%s: q_heads %d not divisible by kv_heads %d", what, num_q_heads, kv_heads);
@@ -487,6 +537,7 @@ extern "C" int qq_extend_attention(const void* q, int num_q_heads, const void* k
                  req_to_token_stride < (int64_t)1 << 30 && kv_rows > 0 &&
                  req_to_token_rows < (int64_t)1 << 31,
              "%s: bad sizes", what);
+  if (verdict) verdict[0] = verdict[1] = bs == 0 || n == 0 ? 0 : -1;
   if (bs == 0 || n == 0) return QQ_OK;
   QQ_REQUIRE(q && k_layer && v_layer && req_to_token && req_pool_indices && seq_lens && prefix_lens &&
                  extend_lens && out, "%s: null pointer", what);
@@ -520,6 +571,7 @@ extern "C" int qq_extend_attention(const void* q, int num_q_heads, const void* k
   a.out = static_cast<uint16_t*>(out);
   a.part_o = static_cast<float*>(workspace);
   a.part_ml = a.part_o ? a.part_o + a.splits * kv_heads * tiles * kExtRows * kMfmaDim : nullptr;
+  a.verdict = verdict;
   hipStream_t s = static_cast<hipStream_t>(stream);
   constexpr size_t kSmem = 4 * kTileElems * sizeof(uint16_t);  // 64 KiB: two buffers of K and V
   extend_kernel<<<(int)grid, 64 * kExtWaves, kSmem, s>>>(a);
