@@ -88,7 +88,7 @@ class AttentionBackend(ABC):
                 and batch.extend_seq_lens is not None and float(scaling) > 0.0
                 and all(t.dim() == 1 and t.shape[0] >= batch.batch_size for t in (
                     batch.req_pool_indices, batch.seq_lens, batch.extend_prefix_lens, batch.extend_seq_lens))
-                and r2t.dtype == torch.int32 and r2t.stride(1) == 1
+                and r2t.dtype == torch.int32 and r2t.stride(1) == 1 and r2t.stride(0) >= r2t.shape[1]
                 and (pool.k_all.data_ptr() | pool.v_all.data_ptr()) % 16 == 0
                 and not (q.requires_grad and torch.is_grad_enabled()))
 

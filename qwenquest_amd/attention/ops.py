@@ -121,12 +121,15 @@ def _extend_launch(
     rpi, seq, prefix, ext = (
         t if t.dtype == torch.int64 and t.device == dev and t.is_contiguous()
         else t.to(device=dev, dtype=torch.int64).contiguous() for t in lens)
-    need = int(_lib.load().qq_extend_attention_workspace_bytes(n, bs, heads, kv, req_to_token.shape[1]))
+    width, stride = req_to_token.shape[1], req_to_token.stride(0)
+    if stride != width:  # columns of a wider table: the kernel cuts a context at the stride
+        seq = seq.clamp(max=width)
+    need = int(_lib.load().qq_extend_attention_workspace_bytes(n, bs, heads, kv, stride))
     ws = torch.empty(need, dtype=torch.uint8, device=dev) if need else None
     out = torch.empty((n, heads * dim), dtype=q.dtype, device=dev)
     args = (
         _lib.ptr(q), heads, _lib.ptr(k_buf), _lib.ptr(v_buf), k_buf.shape[0], kv, dim,
-        _lib.ptr(req_to_token), req_to_token.stride(0), req_to_token.shape[0], _lib.ptr(rpi), _lib.ptr(seq),
+        _lib.ptr(req_to_token), stride, req_to_token.shape[0], _lib.ptr(rpi), _lib.ptr(seq),
         _lib.ptr(prefix), _lib.ptr(ext), bs, n, float(scaling), _lib.ptr(out), _lib.ptr(ws), need,
     )
     stream = _lib.stream(dev)

@@ -243,3 +243,28 @@ def test_calls_that_the_request_by_request_path_takes_or_refuses(where, monkeypa
         assert torch.equal(both(**{name: torch.cat([fields[name], t(7)])}), full)
     both(extend_seq_lens=t(0, 0, 0), q=q[:0])
     both(seq_lens=t(40, 5, 10_000))  # longer than the table: cut to its width
+
+
+@pytest.mark.parametrize("new,prefix", [([5], [600]), ([70, 3], [0, 200])])
+def test_columns_of_a_wider_table(new, prefix):
+    """req_to_token as a slice of a table whose width asks for other K/V splits; a context longer
+    than the slice is cut to the slice, not to the table."""
+    be, q, k, v, batch, layer, slots = make(new, prefix, 8, 1, 13)
+    want = be.forward_extend(q, k, v, layer, batch)
+    narrow = be.req_to_token
+    wide = torch.full((narrow.shape[0], 9000), 1 << 20, dtype=torch.int32, device=DEV)  # rows past the pool
+    wide[:, 11 : 11 + narrow.shape[1]] = narrow
+    batch.req_to_token_pool.req_to_token = wide[:, 11 : 11 + narrow.shape[1]]
+    exact_err(be.forward_extend(q, k, v, layer, batch), want)
+    batch.seq_lens[0] = 9000
+    batch.extend_prefix_lens[0] = narrow.shape[1] - new[0]
+    got = be.forward_extend(q, k, v, layer, batch)
+    batch.req_to_token_pool.req_to_token = narrow
+    exact_err(got, be.forward_extend(q, k, v, layer, batch))
+
+
+def exact_err(got, want):
+    """Other splits of the same sums: one rounding of each."""
+    assert not bool(got.isnan().any())
+    err = (got.double() - want.double()).abs()
+    assert bool((err <= 2.0**-7 * want.double().abs() + 2e-5).all())
