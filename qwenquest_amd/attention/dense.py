@@ -67,7 +67,7 @@ class DenseBackend(AttentionBackend):
         kn = k.reshape(bs, pool.kv_heads * dim).to(torch.bfloat16).contiguous()
         vn = v.reshape(bs, pool.kv_heads * dim).to(torch.bfloat16).contiguous()
         loc = batch.out_cache_loc.to(device=q3.device, dtype=torch.int64).contiguous()
-        need = int(_lib.load().qq_dense_decode_workspace_bytes(bs, r2t.shape[1], heads, pool.kv_heads))
+        need = int(_lib.load().qq_dense_decode_workspace_bytes(bs, r2t.stride(0), heads, pool.kv_heads))
         if self._ws.numel() < need:
             self._ws = torch.empty(need, dtype=torch.uint8, device=q3.device)
         out = torch.empty((bs, heads * dim), dtype=q3.dtype, device=q3.device)

@@ -68,3 +68,32 @@ def test_dense_decode_matches_float64(heads, ctx, width):
             # over the weights: their root sum of squares bounds it well)
             bound = 2.0**-8 * ref.abs() + 2.0**-8 * 3 * float((p * p).sum().sqrt()) + 1e-5
             assert bool(((got[h] - ref).abs() <= bound).all()), (i, h)
+
+
+def test_columns_of_a_wider_table():
+    """req_to_token as a slice of a wider table, at widths that give another number of blocks."""
+    from qwenquest_amd.attention.dense import DenseBackend
+    from qwenquest_amd.batch import ForwardBatch, ForwardMode
+    from qwenquest_amd.memory import MHATokenToKVPool, ReqToTokenPool
+
+    ctx, width = [300, 77], 320
+    rtp = ReqToTokenPool(2, width, DEV)
+    kvp = MHATokenToKVPool(2 * width, 1, KV, D, torch.bfloat16, DEV)
+    gen = torch.Generator(device=DEV).manual_seed(8)
+    kvp.k_all.normal_(generator=gen)
+    kvp.v_all.normal_(generator=gen)
+    rtp.req_to_token.copy_(torch.arange(1, 2 * width + 1, dtype=torch.int32).view(2, width))
+    rpi, seq = torch.arange(2, device=DEV), torch.tensor(ctx, device=DEV)
+    loc = rtp.req_to_token[rpi, seq - 1].long()
+    mk = lambda h: torch.empty((2, h, D), device=DEV).normal_(generator=gen).to(torch.bfloat16)  # noqa: E731
+    q, k, v = mk(32), mk(KV), mk(KV)
+    out = []
+    for wide in (0, 2000):
+        if wide:
+            table = torch.zeros((2, wide), dtype=torch.int32, device=DEV)
+            table[:, 5 : 5 + width] = rtp.req_to_token
+            rtp.req_to_token = table[:, 5 : 5 + width]
+        be = DenseBackend(rtp, kvp)
+        batch = ForwardBatch(ForwardMode.DECODE, None, None, rpi, seq, loc, rtp, kvp, be)
+        out.append(be.forward_decode(q, k, v, Layer(), batch))
+    assert torch.equal(*out)
