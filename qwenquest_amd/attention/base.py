@@ -11,6 +11,7 @@ from abc import ABC, abstractmethod
 from typing import TYPE_CHECKING, Any
 
 import torch
+from torch.autograd import forward_ad
 
 from qwenquest_amd.attention.ops import extend_attention, extend_attention_batch, extend_attention_batch_checked
 
@@ -19,6 +20,13 @@ if TYPE_CHECKING:
     from qwenquest_amd.memory import MHATokenToKVPool, ReqToTokenPool
 
 __all__ = ["AttentionBackend"]
+
+
+def _plain(t: torch.Tensor) -> bool:
+    """Whether torch would only compute with ``t``: no gradient to record, no tangent to carry and
+    no subclass that sees the operations."""
+    return (type(t) in (torch.Tensor, torch.nn.Parameter) and not (t.requires_grad and torch.is_grad_enabled())
+            and forward_ad.unpack_dual(t).tangent is None)
 
 
 class AttentionBackend(ABC):
@@ -50,15 +58,16 @@ class AttentionBackend(ABC):
 
         bf16 with head_dim 128 runs the whole batch in one launch, which reads the lengths
         on the device; a batch that the launch does not answer as the loop below does goes
-        through the loop (which raises IndexError for a request index outside the table).  Other shapes go request by request through
-        ``extend_attention``.  Inside a graph capture, which the loop refuses, a
-        request index outside the table gives NaN, as do rows of ``q`` past the requests' tokens.
+        through the loop (which raises IndexError for a request index outside the table).
+        Other shapes go request by request through ``extend_attention``.  Inside a graph
+        capture, which the loop refuses, a request index outside the table gives NaN, as do
+        rows of ``q`` past the requests' tokens.
         """
         assert batch.out_cache_loc is not None and batch.extend_prefix_lens is not None
         pool = self.token_to_kv_pool
         pool.set_kv_buffer(layer.layer_id, batch.out_cache_loc, k, v)
         k_buf, v_buf = pool.get_kv_buffer(layer.layer_id)
-        if self._extend_fast(q, layer.scaling, batch):
+        if self._extend_fast(q, k_buf, v_buf, layer.scaling, batch):
             attend = (extend_attention_batch if torch.cuda.is_current_stream_capturing()
                       else extend_attention_batch_checked)
             out = attend(q, k_buf, v_buf, self.req_to_token, batch.req_pool_indices, batch.seq_lens,
@@ -77,20 +86,28 @@ class AttentionBackend(ABC):
             )
         return torch.cat(outputs, dim=0)
 
-    def _extend_fast(self, q: torch.Tensor, scaling: float, batch: ForwardBatch) -> bool:
-        """Whether the batched prefill kernel takes this call (its tile is 128 channels wide, a
-        row's maximum is taken before the scale, which therefore has to be positive, and it reads
-        the pool in 16-byte pieces; it records no gradient)."""
-        pool, r2t = self.token_to_kv_pool, self.req_to_token
-        return (q.dim() == 3 and q.dtype == torch.bfloat16 and pool.dtype == torch.bfloat16
-                and pool.head_dim == 128 and q.shape[2] == 128 and q.shape[0] > 0 and q.shape[1] > 0
-                and q.shape[1] % pool.kv_heads == 0 and q.is_cuda and batch.batch_size > 0
-                and batch.extend_seq_lens is not None and float(scaling) > 0.0
-                and all(t.dim() == 1 and t.shape[0] >= batch.batch_size for t in (
-                    batch.req_pool_indices, batch.seq_lens, batch.extend_prefix_lens, batch.extend_seq_lens))
-                and r2t.dtype == torch.int32 and r2t.stride(1) == 1 and r2t.stride(0) >= r2t.shape[1]
-                and (pool.k_all.data_ptr() | pool.v_all.data_ptr()) % 16 == 0
-                and not (q.requires_grad and torch.is_grad_enabled()))
+    def _extend_fast(self, q: torch.Tensor, k_buf: torch.Tensor, v_buf: torch.Tensor, scaling: float,
+                     batch: ForwardBatch) -> bool:
+        """Whether the batched prefill kernel takes this call: its tile is 128 channels wide, a
+        row's maximum is taken before the scale, which therefore has to be positive, it reads the
+        pool in 16-byte pieces, and it records and carries no derivative."""
+        pool, r2t, ext, bs = self.token_to_kv_pool, self.req_to_token, batch.extend_seq_lens, batch.batch_size
+        dev = q.device
+        if (q.dim() != 3 or q.dtype != torch.bfloat16 or pool.dtype != torch.bfloat16 or pool.head_dim != 128
+                or bs == 0 or ext is None or not float(scaling) > 0.0 or not q.is_cuda or not _plain(q)
+                or torch._C._get_tracing_state() is not None):
+            return False
+        n, heads, dim = q.shape
+        if n == 0 or heads == 0 or dim != 128 or heads % pool.kv_heads:
+            return False
+        for b in (k_buf, v_buf):
+            if b.device != dev or b.data_ptr() % 16 or not b.is_contiguous() or b.requires_grad:
+                return False
+        for t in (batch.req_pool_indices, batch.seq_lens, batch.extend_prefix_lens, ext):
+            if t.dim() != 1 or t.shape[0] < bs:
+                return False
+        row, col = r2t.stride()
+        return r2t.dtype == torch.int32 and col == 1 and row >= r2t.shape[1] and r2t.device == dev
 
     @abstractmethod
     def forward_decode(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, layer: Any, batch: ForwardBatch) -> torch.Tensor:

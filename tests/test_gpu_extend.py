@@ -268,3 +268,27 @@ def exact_err(got, want):
     assert not bool(got.isnan().any())
     err = (got.double() - want.double()).abs()
     assert bool((err <= 2.0**-7 * want.double().abs() + 2e-5).all())
+
+
+def test_derivatives_and_subclasses_go_through_torch():
+    """A gradient, a tangent or a subclass keeps what torch does with it."""
+    from torch.autograd import forward_ad as fwad
+    from torch.nn.attention import SDPBackend, sdpa_kernel
+
+    be, q, k, v, batch, layer, slots = make([20, 13], [0, 30], 4, 2, 17)
+    dq = torch.randn_like(q)
+    run = lambda x: be.forward_extend(x, k, v, layer, batch)  # noqa: E731
+    want = run(q)
+    x = q.clone().requires_grad_()
+    run(x).sum().backward()
+    assert bool(x.grad.abs().sum() > 0)
+    with sdpa_kernel(SDPBackend.MATH):  # the one form with forward derivatives
+        with fwad.dual_level():
+            out = fwad.unpack_dual(run(fwad.make_dual(q, dq)))
+        assert out.tangent is not None and bool(out.tangent.abs().sum() > 0)
+        exact_err(out.primal, want)
+
+    class Seen(torch.Tensor):
+        pass
+
+    assert type(run(q.as_subclass(Seen))) is Seen
