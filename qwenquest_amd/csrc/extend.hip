@@ -31,6 +31,8 @@
 // 600 new tokens, where a chain of ten K/V tiles per block is what counts: 25 us of
 // 430.  The products are ordered so that neighbours have different accumulators
 // (2.83 -> 2.78 ms).
+#include <type_traits>
+
 #include "qq_quest_dev.h"
 
 namespace qq {
@@ -165,6 +167,17 @@ __device__ inline uint32_t pack_hi16(float even, float odd) {  // the high halve
 }
 __device__ inline float trunc_bf(float x) { return __uint_as_float(__float_as_uint(x) & 0xFFFF0000u); }
 
+// The finite ones of eight bf16 values, 0 for the others.
+__device__ inline bf16x8_t finite_only(bf16x8_t v) {
+  u32x4_t w = __builtin_bit_cast(u32x4_t, v);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if ((w[i] & 0x7F80u) == 0x7F80u) w[i] &= 0xFFFF0000u;
+    if ((w[i] & 0x7F800000u) == 0x7F800000u) w[i] &= 0xFFFFu;
+  }
+  return __builtin_bit_cast(bf16x8_t, w);
+}
+
 // 64 lanes x 16 bytes from per-lane global addresses to LDS byte address `lds` + 16 *
 // lane.  In inline asm (it writes no register; tile_barrier waits for it), since the
 // compiler would wait for the builtin's pending LDS write before the other buffer's
@@ -263,11 +276,7 @@ __global__ __launch_bounds__(64 * kExtWaves, 2) void extend_kernel(ExtendArgs a)
     }
   };
   float16_t o[4];
-#pragma unroll
-  for (int c = 0; c < 4; ++c)
-#pragma unroll
-    for (int i = 0; i < 16; ++i) o[c][i] = 0.0f;
-  float M = -INFINITY, L = 0.0f;
+  float M, L;
 
   // K operand pieces 2 ks + hf of row lo (+ 32); V operand: token 4 hf + l16 / 4, channels 16 (g & 1) + 4 (l16 % 4)
   const int l16 = lane & 15;
@@ -279,114 +288,140 @@ __global__ __launch_bounds__(64 * kExtWaves, 2) void extend_kernel(ExtendArgs a)
   for (int c = 0; c < 4; ++c)
     v_off[c] = v_row * kMfmaDim + ((c ^ (l16 >> 2)) << 5) + ((lane >> 4) & 1) * 16 + (l16 & 3) * 4;
 
-  if (j_begin < j_end) {
-    load_rows(j_begin);
-    load_tile(0);
-    if (j_begin + 1 < j_end) load_rows(j_begin + 1);
-  }
-  int buf = 0;
-  for (int j = j_begin; j < j_end; ++j) {
-    tile_barrier();
-    if (j + 1 < j_end) {
-      load_tile(buf ^ 1);
-      if (j + 2 < j_end) load_rows(j + 2);
+  // the block's K/V tiles; finite: the lower pieces of a weight meet only finite values
+  auto attend = [&](auto finite) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) o[c][i] = 0.0f;
+    M = -INFINITY;
+    L = 0.0f;
+    if (j_begin < j_end) {
+      load_rows(j_begin);
+      load_tile(0);
+      if (j_begin + 1 < j_end) load_rows(j_begin + 1);
     }
-    const uint16_t* sk = sm + buf * 2 * kTileElems;
-    const uint16_t* sv = sk + kTileElems;
-    buf ^= 1;
-    // S^T[token 32 t + 8 (i / 4) + 4 hf + i % 4][row lo] in s[t][i]
-    float16_t s[2];
-    {
-      bf16x8_t ka[2][8];
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-#pragma unroll
-        for (int ks = 0; ks < 8; ++ks)
-          ka[t][ks] = *reinterpret_cast<const bf16x8_t*>(sk + t * 32 * kMfmaDim + k_off[ks]);
+    int buf = 0;
+    for (int j = j_begin; j < j_end; ++j) {
+      tile_barrier();
+      if (j + 1 < j_end) {
+        load_tile(buf ^ 1);
+        if (j + 2 < j_end) load_rows(j + 2);
       }
+      const uint16_t* sk = sm + buf * 2 * kTileElems;
+      const uint16_t* sv = sk + kTileElems;
+      buf ^= 1;
+      // S^T[token 32 t + 8 (i / 4) + 4 hf + i % 4][row lo] in s[t][i]
+      float16_t s[2];
+      {
+        bf16x8_t ka[2][8];
 #pragma unroll
-      for (int t = 0; t < 2; ++t) {
+        for (int t = 0; t < 2; ++t) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) s[t][i] = 0.0f;
+          for (int ks = 0; ks < 8; ++ks)
+            ka[t][ks] = *reinterpret_cast<const bf16x8_t*>(sk + t * 32 * kMfmaDim + k_off[ks]);
+        }
 #pragma unroll
-        for (int ks = 0; ks < 8; ++ks)
-          s[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ka[t][ks], qb[ks], s[t], 0, 0, 0);
+        for (int t = 0; t < 2; ++t) {
+#pragma unroll
+          for (int i = 0; i < 16; ++i) s[t][i] = 0.0f;
+#pragma unroll
+          for (int ks = 0; ks < 8; ++ks)
+            s[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ka[t][ks], qb[ks], s[t], 0, 0, 0);
+        }
+        // the first 32 tokens' reads, then the others' under their products
+        __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        }
+        __builtin_amdgcn_sched_group_barrier(0x8, 8, 0);
       }
-      // the first 32 tokens' reads, then the others' under their products
-      __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
+      if ((j + 1) * kExtTile > lim_full) {  // block-uniform: some row's limit is inside this tile
+        const int left = lim - j * kExtTile - 4 * hf;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int i = 0; i < 16; ++i)
+            s[t][i] = (t * 32 + 8 * (i / 4) + i % 4) < left ? s[t][i] : -INFINITY;
       }
-      __builtin_amdgcn_sched_group_barrier(0x8, 8, 0);
-    }
-    if ((j + 1) * kExtTile > lim_full) {  // block-uniform: some row's limit is inside this tile
-      const int left = lim - j * kExtTile - 4 * hf;
+      float mx = s[0][0];
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int i = 0; i < 16; ++i)
-          s[t][i] = (t * 32 + 8 * (i / 4) + i % 4) < left ? s[t][i] : -INFINITY;
-    }
-    float mx = s[0][0];
+        for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[t][i]);
+      mx = fmaxf(mx, lane_xor32(mx, lane));
+      if (__any(mx > M)) {
+        const float Mn = fmaxf(M, mx);
+        const float alpha = M == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((M - Mn) * a.sl2);
+        L *= alpha;
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+        for (int c = 0; c < 4; ++c)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[t][i]);
-    mx = fmaxf(mx, lane_xor32(mx, lane));
-    if (__any(mx > M)) {
-      const float Mn = fmaxf(M, mx);
-      const float alpha = M == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((M - Mn) * a.sl2);
-      L *= alpha;
-#pragma unroll
-      for (int c = 0; c < 4; ++c)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) o[c][i] *= alpha;
-      M = Mn;
-    }
-    const float mb = M == -INFINITY ? 0.0f : -M * a.sl2;  // nothing attended yet: weights of 0
-    float sum = 0.0f;
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[t][i], a.sl2, mb));
-        s[t][i] = p;
-        sum += p;
+          for (int i = 0; i < 16; ++i) o[c][i] *= alpha;
+        M = Mn;
       }
-    L += sum;
-    // O^T += V^T P^T, 16 tokens at a time, P in bf16 pieces
+      const float mb = M == -INFINITY ? 0.0f : -M * a.sl2;  // nothing attended yet: weights of 0
+      float sum = 0.0f;
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      u32x4_t pw[kPieces];
+      for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int x = 0; x < 4; ++x) {
-        float e = s[u >> 1][(u & 1) * 8 + 2 * x], f = s[u >> 1][(u & 1) * 8 + 2 * x + 1];
-#pragma unroll
-        for (int c = 0; c < kPieces; ++c) {
-          pw[c][x] = pack_hi16(e, f);
-          e -= trunc_bf(e);
-          f -= trunc_bf(f);
+        for (int i = 0; i < 16; ++i) {
+          const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[t][i], a.sl2, mb));
+          s[t][i] = p;
+          sum += p;
         }
+      L += sum;
+      // O^T += V^T P^T, 16 tokens at a time, P in bf16 pieces
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        u32x4_t pw[kPieces];
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+          float e = s[u >> 1][(u & 1) * 8 + 2 * x], f = s[u >> 1][(u & 1) * 8 + 2 * x + 1];
+#pragma unroll
+          for (int c = 0; c < kPieces; ++c) {
+            pw[c][x] = pack_hi16(e, f);
+            e -= trunc_bf(e);
+            f -= trunc_bf(f);
+          }
+        }
+        bf16x8_t va[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          uint16_t* vp = const_cast<uint16_t*>(sv) + v_off[c] + u * 16 * kMfmaDim;
+          const short4_t v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_t*)vp);
+          const short4_t v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_t*)(vp + 8 * kMfmaDim));
+          va[c] = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
+        }
+        bf16x8_t vl[4];  // for the weights' lower pieces
+#pragma unroll
+        for (int c = 0; c < 4; ++c) vl[c] = decltype(finite)::value ? finite_only(va[c]) : va[c];
+#pragma unroll
+        for (int x = 0; x < kPieces; ++x)
+#pragma unroll
+          for (int c = 0; c < 4; ++c)  // independent accumulators one after the other
+            o[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x == 0 ? va[c] : vl[c],
+                                                           __builtin_bit_cast(bf16x8_t, pw[x]), o[c], 0, 0, 0);
       }
-      bf16x8_t va[4];
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        uint16_t* vp = const_cast<uint16_t*>(sv) + v_off[c] + u * 16 * kMfmaDim;
-        const short4_t v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_t*)vp);
-        const short4_t v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_t*)(vp + 8 * kMfmaDim));
-        va[c] = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
-      }
-#pragma unroll
-      for (int x = 0; x < kPieces; ++x)
-#pragma unroll
-        for (int c = 0; c < 4; ++c)  // independent accumulators one after the other
-          o[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va[c], __builtin_bit_cast(bf16x8_t, pw[x]), o[c], 0, 0, 0);
     }
+    L += lane_xor32(L, lane);
+  };
+  attend(std::false_type{});
+  // An infinite value times a weight is infinite (or NaN, for a weight of 0), but times a
+  // lower piece that happens to be 0 it is NaN: where a sum is NaN and its weights are not,
+  // the block goes over its tiles again with the infinities left to the upper pieces.
+  bool again = false;
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) again |= o[c][i] != o[c][i];
+  again &= L == L;
+  if (__syncthreads_or(bad || again)) {
+    if (__syncthreads_or(again)) attend(std::true_type{});
+    if (__syncthreads_or(bad)) L = __builtin_nanf("");  // a row outside the pool: no answer
   }
-  L += lane_xor32(L, lane);
-  if (__syncthreads_or(bad ? 1 : 0)) L = __builtin_nanf("");  // a row outside the pool: no answer
   const bool mine = r0 + wave * 32 + lo < rows_n;
   if (whole) {
     if (!mine) return;
@@ -450,7 +485,8 @@ __global__ __launch_bounds__(256) void extend_merge_kernel(ExtendArgs a) {
       ov[u] = *reinterpret_cast<const float4*>(a.part_o + (pr + min(p0 + u, parts - 1) * step) * kMfmaDim + d4);
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
-      const float wu = __shfl(w, p0 + u, 32);  // p0 + u < 32; 0 past the last part
+      const float wu = __shfl(w, p0 + u, 32);  // p0 + u < 32
+      if (p0 + u >= parts) break;  // block-uniform; a weight of 0 would make NaN of an infinite sum
       Os.x += wu * ov[u].x;
       Os.y += wu * ov[u].y;
       Os.z += wu * ov[u].z;

@@ -292,3 +292,33 @@ def test_derivatives_and_subclasses_go_through_torch():
         pass
 
     assert type(run(q.as_subclass(Seen))) is Seen
+
+
+@pytest.mark.parametrize("new,prefix,width", [([200, 40], [0, 30], None), ([6], [3000], 8192)])
+def test_infinite_values(new, prefix, width):
+    """An infinite value of an attended row makes the output infinite (also through K/V splits and
+    their merge), a NaN makes it NaN, and other channels stay as they are."""
+    be, q, k, v, batch, layer, slots = make(new, prefix, 4, 2, 19, width=width)
+    want = be.forward_extend(q, k, v, layer, batch).view(-1, 4, 128)
+    inf = float("inf")
+    pool, r2t = batch.token_to_kv_pool, batch.req_to_token_pool.req_to_token
+    at, ones = 0, torch.ones(4, device=DEV)
+    for i, (n, p) in enumerate(zip(new, prefix)):
+        rows = r2t[slots[i]].long()
+        old = sorted({0, p + n // 2})
+        for pos, c, val in ((0, 5, inf), (old[-1], 9, -inf), (old[-1], 11, float("nan"))):
+            if pos >= p:
+                v[at + pos - p, :, c] = val
+            else:
+                pool.v_all[0, rows[pos], :, c] = val
+        at += n
+    got = be.forward_extend(q, k, v, layer, batch).view(-1, 4, 128)
+    at = 0
+    for i, (n, p) in enumerate(zip(new, prefix)):
+        mid = n // 2  # the first of the request's tokens that attends the second position
+        assert torch.equal(got[at : at + n, :, 5].float(), inf * ones.expand(n, 4))
+        assert torch.equal(got[at + mid : at + n, :, 9].float(), -inf * ones.expand(n - mid, 4))
+        assert bool(got[at + mid : at + n, :, 11].isnan().all())
+        at += n
+    rest = [c for c in range(128) if c not in (5, 9, 11)]
+    assert torch.equal(got[..., rest], want[..., rest])
