@@ -32,30 +32,32 @@
 // Other shapes: four launches on one stream, each consuming the previous one's
 // output: score (all CUs) -> select + new-token store (one block per request)
 // -> chunk attention (MFMA) -> merge.
-#include <algorithm>
 #include <mutex>
 
 #include "qq_quest_dev.h"
+#include "qq_rules.h"
 
 namespace qq {
 namespace {
 
-constexpr int kDenseKV = 4;           // KV heads of the dense decode kernel (KV*D = 512)
 constexpr int kStepMaxG = 16;
 constexpr int kMaxSelFused = 64;
 constexpr int kStepMaxTopK = 4096;
 constexpr int kDenseWaves = 8;       // dense decode: 8-wave blocks (two waves per SIMD)
-constexpr int kDenseBlocks = 256;    // one per CU, at most: all resident
-constexpr int kDenseParts = kDenseBlocks / kDenseKV;  // parts of a (request, KV head), at most
-constexpr int kDenseWhole = 8;       // units of a pair that is not split
-constexpr int kDenseMinLen = 2;      // units of a part, at least
 constexpr int kDensePlanReqs = 4096; // requests whose units the plan keeps in LDS
-// The Quest step's attention (quest_attend_unit_kernel): up to kUnitParts blocks
-// per (request, KV head), merged in one pass; the selection of a 4-wave block
+// The selection of a 4-wave block of the Quest step's attention (quest_attend_unit_kernel)
 // holds up to 32 scores per thread (8192 pages; its LDS, 68 KiB, still lets two
 // blocks share a CU).
-constexpr int kUnitParts = 8;
 constexpr int kUnitMinWaves = 4;
+using rules::dense_part_begin;
+using rules::dense_parts;
+using rules::dense_units;
+using rules::kDenseKV;
+using rules::kDenseMinLen;
+using rules::kDenseParts;
+using rules::kUnitParts;
+using rules::unit_first;
+using rules::UnitShape;
 
 struct StepArgs {
   SelectArgs s;            // scoring, selection, positions, new token
@@ -346,17 +348,6 @@ struct DenseSmem {
 __device__ inline int dense_rows(const StepArgs& a, int b) {
   return (int)min(max(a.s.seq[b], (int64_t)0), (int64_t)a.s.top_k);
 }
-// A request without rows has one unit, which writes its zeros.
-__device__ inline int dense_units(int rows) { return max((rows + 63) / 64, 1); }
-
-// Parts of a pair for parts of `len` units.  A pair of up to a unit per wave stays
-// whole, which saves its merge (one request of 500 rows: 12.9 us against 15.3 in two
-// parts); longer ones may go down to two units a part (four of 1000 rows: 16.5 us, at
-// four units 17.4, at eight 19.6; one of 8000: 18.0, 17.8 and 19.9).
-__device__ inline int dense_parts(int units, int len) {
-  return units <= kDenseWhole ? 1 : (units + len - 1) / len;
-}
-
 // Sum of v over a 256-thread block (tmp: 4 ints).
 __device__ inline int block_sum_256(int v, int* tmp) {
 #pragma unroll
@@ -463,8 +454,8 @@ __global__ __launch_bounds__(256) void dense_store_plan_kernel(StepArgs a, Dense
       const int units = s_units[b];
       const int64_t req = a.s.rpi[b];
       it.bh = b * kDenseKV + h;
-      it.u0 = (int)(((int64_t)units * part) / parts);
-      it.u1 = (int)(((int64_t)units * (part + 1)) / parts);
+      it.u0 = dense_part_begin(units, part, parts);
+      it.u1 = dense_part_begin(units, part + 1, parts);
       it.part = part;
       it.parts = parts;
       it.rows = dense_rows(a, b);
@@ -724,7 +715,7 @@ __global__ __launch_bounds__(64 * W, 8 / W) void quest_attend_unit_kernel(StepAr
 #pragma unroll
   for (int e = 0; e < 8; ++e) o[e] = float4_t{0.f, 0.f, 0.f, 0.f};
   bool bad = false;
-  for (int u = wave * parts + part; u < units; u += stride_units) {  // wave-uniform
+  for (int u = unit_first(wave, part, parts); u < units; u += stride_units) {  // wave-uniform
     const int slot = u * P + lane;
     const int valid = min(n - u * P, P);  // real slots of this unit
     int64_t row = 0;
@@ -865,40 +856,8 @@ static bool fused_shape(int q_dtype, int kv_dtype, int new_dtype, int num_q_head
                                            top_k, max_pages);
 }
 
-// Launch shape of the unit attention: W waves per block, `parts` blocks per (request,
-// KV head); wave w of part p takes the units w * parts + p, + W * parts, ... one after
-// the other.  The grid is sized to one round of resident blocks, since each block pays
-// its own selection, row lookups and merge before and after its streaming (us per
-// layer-step, top_k 2048 at 4 KV heads unless said):
-//  * a unit per wave in 4-wave blocks that leave each CU at most one: those (batch 8:
-//    16.4, 18.2 in 8-wave blocks; batch 9, where they would be more than the CUs: 19.9
-//    against 18.7);
-//  * up to one pair per CU: 8-wave blocks (one per CU), parts = CUs / pairs, unless two
-//    4-wave blocks per CU, parts = 2 CUs / pairs, leave a wave fewer units in a row
-//    (batch 34: 42.3 in 4-wave blocks, three parts, against 47.6; batch 40: 45.5 and
-//    48.1, at top_k 4096 75.9 and 83.9; batch 48, where the rows are as long: 51.7
-//    and 50.5);
-//  * more pairs: 4-wave blocks, 3 parts up to 4/3 pairs per CU, then 2, past 8/5 1
-//    (batch 72: 74.3 in 3, 77.1 in 2; batch 84: 81.4 and 83.0; batch 96: 94.7 and 89.6;
-//    batch 104: 102.2 in 2, 96.3 in 1).
-// A second round of units in a part is dealt over all parts, not to the first ones
-// (batch 20, 32 units over 24 waves: 32.0 -> 28.5; choosing the order by whether there
-// is a second round costs batch 1 more, 0.04 us a layer, than the order does).
-struct UnitShape {
-  int W, parts;
-};
 static UnitShape unit_shape(int bs, int kv_heads, int top_k) {
-  const int64_t c = device_cu_count(), units = top_k / 64, pairs = (int64_t)bs * kv_heads;
-  const int cap8 = std::max(1, std::min(kUnitParts, ceil_div(units, 8)));
-  const int cap4 = std::max(1, std::min(kUnitParts, ceil_div(units, 4)));
-  if (units <= 4 * cap4 && pairs * cap4 <= c) return {4, cap4};
-  if (pairs <= c) {
-    const int p8 = (int)std::max<int64_t>(1, std::min<int64_t>(cap8, c / pairs));
-    const int p4 = (int)std::max<int64_t>(1, std::min<int64_t>(cap4, 2 * c / pairs));
-    if (ceil_div(units, 4 * p4) < ceil_div(units, 8 * p8)) return {4, p4};
-    return {8, p8};
-  }
-  return {4, std::min(cap4, 3 * pairs <= 4 * c ? 3 : 5 * pairs <= 8 * c ? 2 : 1)};
+  return rules::unit_shape(device_cu_count(), bs, kv_heads, top_k);
 }
 
 extern "C" int qq_quest_fused_step(int q_dtype, int kv_dtype, int new_dtype, int num_q_heads, int kv_heads,
@@ -961,12 +920,7 @@ int qq::attend_rows_fused(const void* q, int64_t q_bstride, int num_q_heads, con
   return QQ_OK;
 }
 
-// Dense decode: one block per CU, or as many as the table's width can use; at least
-// one per (request, KV head).
-static int64_t dense_blocks(int bs, int64_t max_rows) {
-  const int64_t pairs = (int64_t)bs * kDenseKV, units = pairs * ((max_rows + 63) / 64);
-  return std::max(pairs, std::min<int64_t>(std::min(device_cu_count(), kDenseBlocks), units));
-}
+static int64_t dense_blocks(int bs, int64_t max_rows) { return rules::dense_blocks(device_cu_count(), bs, max_rows); }
 
 extern "C" int64_t qq_dense_decode_workspace_bytes(int bs, int64_t max_rows, int num_q_heads, int kv_heads) {
   if (bs <= 0 || max_rows <= 0 || kv_heads <= 0 || num_q_heads <= 0) return 0;

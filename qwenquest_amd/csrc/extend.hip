@@ -34,6 +34,7 @@
 #include <type_traits>
 
 #include "qq_quest_dev.h"
+#include "qq_rules.h"
 
 namespace qq {
 namespace {
@@ -42,10 +43,14 @@ typedef float float16_t __attribute__((ext_vector_type(16)));
 typedef __attribute__((address_space(3))) short4_t lds_short4_t;
 
 constexpr int kExtWaves = 4;
-constexpr int kExtRows = 32 * kExtWaves;  // query rows per block
-constexpr int kExtTile = 64;              // tokens per K/V tile
-constexpr int kExtMinChunk = 4;           // K/V tiles per split, at least
-constexpr int kExtMaxSplits = 32;
+using rules::extend_request_tiles;
+using rules::extend_splits;
+using rules::extend_tiles;
+using rules::kExtMaxSplits;
+using rules::kExtRows;
+using rules::kExtTile;
+using rules::split_chunk;
+static_assert(kExtRows == 32 * kExtWaves && kExtMaxSplits <= 32, "a wave's rows; the merge's lanes");
 constexpr int kTileElems = kExtTile * kMfmaDim;
 constexpr int kPieces = 3;  // bf16 pieces of an fp32 weight
 
@@ -107,7 +112,7 @@ __device__ inline ExtendTile find_tile(const ExtendArgs& a, int t) {
     const int before = __shfl_up(sn, 1, 64);
     const int first = min(tok + (lane > 0 ? before : 0), a.n);
     n = min(n, a.n - first);
-    const int mine = (int)(((int64_t)n * a.G + kExtRows - 1) / kExtRows);
+    const int mine = extend_request_tiles(n, a.G);
     nt = mine;
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
@@ -153,13 +158,6 @@ __device__ inline void report_lengths(const ExtendArgs& a) {
   if (lane != 0) return;
   __hip_atomic_store(a.verdict + 1, total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   __hip_atomic_store(a.verdict, any ? 1 : 0, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-}
-
-// K/V tiles per split of a query tile that attends nt of them: equal parts, none
-// shorter than kExtMinChunk.
-__device__ inline int split_chunk(int nt, int splits) {
-  const int parts = max(min(splits, (nt + kExtMinChunk - 1) / kExtMinChunk), 1);
-  return max((nt + parts - 1) / parts, 1);
 }
 
 __device__ inline uint32_t pack_hi16(float even, float odd) {  // the high halves: truncation to bf16
@@ -498,22 +496,6 @@ __global__ __launch_bounds__(256) void extend_merge_kernel(ExtendArgs a) {
   uint16_t* op = a.out + ((int64_t)(et.q0 + tok) * a.H + h * a.G + r - tok * a.G) * kMfmaDim + d4;
   *reinterpret_cast<uint2*>(op) = make_uint2((uint32_t)f2bf(Os.x * inv) | ((uint32_t)f2bf(Os.y * inv) << 16),
                                              (uint32_t)f2bf(Os.z * inv) | ((uint32_t)f2bf(Os.w * inv) << 16));
-}
-
-// Query tiles of n tokens in bs requests, at most: every request's last tile may
-// be partial.
-int64_t extend_tiles(int64_t n, int bs, int G) { return n * G / kExtRows + bs; }
-
-// K/V splits: as many as give every CU a block when the query tiles do not, parts of
-// at least kExtMinChunk K/V tiles.  The merge costs a launch (6 us), so a grid that
-// covers half the chip stays whole: 600 new tokens (152 blocks) 30.5 us, in two
-// splits 34.6; 8 new tokens behind 8192 (4 blocks) in 32 splits 26.0 us, in 9 of 16
-// tiles 44.9; 64 behind 8192 (16 blocks) in 12 splits 42.2 us, in 25 52.9.  A minimum of 4
-// tiles against 8 and 16: 100 new behind 500, one KV head, 21 against 28 us.
-int extend_splits(int64_t tiles, int KV, int64_t max_rows) {
-  const int64_t by_grid = 256 / max(tiles * KV, (int64_t)1);
-  const int64_t by_rows = (max_rows + kExtTile * kExtMinChunk - 1) / (kExtTile * kExtMinChunk);
-  return (int)max((int64_t)1, min(min(by_grid, by_rows), (int64_t)kExtMaxSplits));
 }
 
 }  // namespace
