@@ -32,6 +32,7 @@
 // Other shapes: four launches on one stream, each consuming the previous one's
 // output: score (all CUs) -> select + new-token store (one block per request)
 // -> chunk attention (MFMA) -> merge.
+#include <algorithm>
 #include <mutex>
 
 #include "qq_quest_dev.h"
@@ -44,16 +45,20 @@ constexpr int kStepMaxG = 16;
 constexpr int kMaxSelFused = 64;
 constexpr int kStepMaxTopK = 4096;
 constexpr int kDenseWaves = 8;       // dense decode: 8-wave blocks (two waves per SIMD)
-constexpr int kDensePlanReqs = 4096; // requests whose units the plan keeps in LDS
+constexpr int kPlanReqs = 1024;      // requests whose words the dense plan keeps in LDS at once
 // The selection of a 4-wave block of the Quest step's attention (quest_attend_unit_kernel)
 // holds up to 32 scores per thread (8192 pages; its LDS, 68 KiB, still lets two
 // blocks share a CU).
 constexpr int kUnitMinWaves = 4;
+using rules::dense_all_whole;
+using rules::dense_candidate;
+using rules::dense_cost;
+using rules::dense_first;
 using rules::dense_part_begin;
 using rules::dense_parts;
+using rules::dense_range;
 using rules::dense_units;
 using rules::kDenseKV;
-using rules::kDenseMinLen;
 using rules::kDenseParts;
 using rules::kUnitParts;
 using rules::unit_first;
@@ -317,11 +322,10 @@ __device__ inline void finish_block(const StepArgs& a, int bh, int part, float M
 
 // ------------------------------------------------------------- dense decode
 // Every request attends its whole context (attention/dense.py:26-42).  A (request, KV
-// head) pair's 64-row units are split into equal parts, one to a block.  The parts are
-// as long as they have to be for all pairs' parts to fit the blocks that are resident
-// at once: one long request or many ragged ones keep the same number of CUs busy, and
-// the table's width costs nothing.  The lengths are on the device, so the division is
-// made there, by one more block of the launch that stores the new tokens (it hides
+// head) pair's 64-row units are split into equal parts, one to a block, of a length that
+// keeps the CUs alike busy: one long request, many ragged ones, or one long one among
+// many (dense_range and dense_cost in qq_rules.h).  The lengths are on the device, so the
+// division is made there, by one more block of the launch that stores the new tokens (it hides
 // behind that launch, and the attention's blocks each read one entry instead of the
 // batch's lengths).
 struct DenseItem {
@@ -330,7 +334,14 @@ struct DenseItem {
   int part, parts;  // of the pair; its parts are consecutive blocks
   int rows;         // context
   int req;          // table row, or -1: outside the table
-  int pad;
+  int queued;       // 0, or the entries of the plan, where there are more of them than blocks
+};
+
+// Where the plan has more entries than the grid has blocks, every block goes on with the
+// next one that no block has.
+struct DenseQueue {
+  uint32_t next;
+  uint32_t pad[7];
 };
 
 struct DenseSmem {
@@ -343,126 +354,206 @@ struct DenseSmem {
     } merge;
   };
   uint32_t last;
+  uint32_t next[2];  // the part after this one, in turn
 };
 
 __device__ inline int dense_rows(const StepArgs& a, int b) {
   return (int)min(max(a.s.seq[b], (int64_t)0), (int64_t)a.s.top_k);
 }
-// Sum of v over a 256-thread block (tmp: 4 ints).
-__device__ inline int block_sum_256(int v, int* tmp) {
-#pragma unroll
-  for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d, 64);
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) tmp[threadIdx.x >> 6] = v;
-  __syncthreads();
-  return tmp[0] + tmp[1] + tmp[2] + tmp[3];
+// dense_parts(units, len) with 1 / len at hand: the quotient by the inverse, then put right.
+__device__ inline int dense_parts_inv(int units, int len, float inv) {
+  const int x = units + len - 1;
+  int parts = (int)((float)x * inv);
+  const int rest = x - parts * len;
+  parts += rest >= len ? 1 : rest < 0 ? -1 : 0;
+  return units <= rules::kDenseWhole ? 1 : min(parts, kDenseParts);
 }
 
-// Block 0: the division of the batch into `blocks` parts; blocks 1 .. bs: the new
-// tokens (memory.py:114-120).  The part length is the smallest of 64 candidates,
-// between the one that would divide the batch without remainders and one that surely
-// fits, with which all parts fit; each lane tries one, the waves share the requests.
-// A batch of more requests than the LDS keeps gets one part per pair.
-__global__ __launch_bounds__(256) void dense_store_plan_kernel(StepArgs a, DenseItem* plan, int blocks) {
+// The division of a batch that one round of blocks takes (dense_one_round: at most 24
+// requests): a lane per request, every wave for itself, without LDS and barriers.  The
+// shortest of the lengths that fit is the cheapest.
+__device__ inline void plan_one_round(const StepArgs& a, DenseItem* plan, int fit, int round, int grid) {
+  const int bs = a.bs, tid = threadIdx.x, lane = tid & 63;
+  int rows = 0, units = 0, req = -1;
+  if (lane < bs) {
+    const int64_t r = a.s.rpi[lane];
+    rows = dense_rows(a, lane);
+    units = dense_units(rows);
+    req = r >= 0 && r < a.r2t_rows ? (int)r : -1;
+  }
+  int total = units, longest = max(units, 1);
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1) {
+    total += __shfl_xor(total, d, 64);
+    longest = max(longest, __shfl_xor(longest, d, 64));
+  }
+  int len = 1 << 30;  // nothing is split
+  if (fit > bs) {
+    const int cand = dense_candidate(dense_range(min(total, rules::kDenseMaxTotal), longest, bs, fit, round), lane);
+    const float inv = 1.0f / (float)cand;
+    int count = 0;
+    for (int b = 0; b < bs; ++b) count += dense_parts_inv(__builtin_amdgcn_readlane(units, b), cand, inv);
+    const uint64_t ok = __ballot(count <= fit);
+    if (ok) len = __builtin_amdgcn_readlane(cand, __builtin_ctzll(ok));
+  }
+  const int parts = lane < bs ? dense_parts(units, len) : 0;
+  int first = parts;  // parts (per KV head) up to this request's, then before it
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int y = __shfl_up(first, d, 64);
+    if (lane >= d) first += y;
+  }
+  const int all = __builtin_amdgcn_readlane(first, 63) * kDenseKV;
+  first -= parts;
+  for (int e0 = 0; e0 < grid; e0 += 256) {
+    const int e = e0 + tid;
+    // blocks of a request: its parts of KV head 0, then of head 1, ...
+    int b = -1;
+    for (int i = 0; i < bs; ++i) b += __builtin_amdgcn_readlane(first, i) * kDenseKV <= e ? 1 : 0;
+    const int p = __shfl(parts, b, 64), u = __shfl(units, b, 64);
+    const int at = e - __shfl(first, b, 64) * kDenseKV;
+    const int h = at / p, part = at - h * p;
+    const DenseItem it = {b * kDenseKV + h, dense_part_begin(u, part, p), dense_part_begin(u, part + 1, p), part,
+                          p, __shfl(rows, b, 64), __shfl(req, b, 64), 0};
+    if (e < grid) plan[e] = e < all ? it : DenseItem{-1, 0, 0, 0, 1, 0, -1, 0};
+  }
+}
+
+// Block 0: the division of the batch, `fit` parts per KV head at most; blocks 1 .. bs:
+// the new tokens (memory.py:114-120).  64 part lengths are tried, one per lane, the waves
+// sharing the requests (dense_range, dense_cost), and every entry finds its request.  The
+// requests' words are kept in LDS, kPlanReqs of them at a time.
+__global__ __launch_bounds__(256) void dense_store_plan_kernel(StepArgs a, DenseItem* plan, DenseQueue* queue, int fit,
+                                                               int round, int grid) {
   const int bs = a.bs, tid = threadIdx.x;
   if (blockIdx.x > 0) {
     store_new_token(a.s, blockIdx.x - 1);
     return;
   }
-  __shared__ uint16_t s_first[kDensePlanReqs + 1];  // parts (per KV head) before each request
-  __shared__ int s_units[kDensePlanReqs];
-  __shared__ int s_tmp[4], s_count[4][64], s_len;
-  const bool kept = bs <= kDensePlanReqs;
-  int sum = 0, most = 1;
-  for (int b = tid; kept && b < bs; b += 256) {
-    const int u = dense_units(dense_rows(a, b));
-    s_units[b] = u;
-    sum += u;
-    most = max(most, u);
-  }
-  const int wave = tid >> 6, lane = tid & 63;
-  const int fit = blocks / kDenseKV;  // parts per KV head that fit; at least bs
-  int len = 1 << 30;                  // units per part
-  if (kept && fit > bs) {
-    const int total = block_sum_256(sum, s_tmp);
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) most = max(most, __shfl_xor(most, d, 64));
-    __syncthreads();
-    if (lane == 0) s_tmp[wave] = most;
-    __syncthreads();
-    most = max(max(s_tmp[0], s_tmp[1]), max(s_tmp[2], s_tmp[3]));
-    const int lo = max((total + fit - 1) / fit, kDenseMinLen);
-    const int hi = max(lo, min(most, (total + fit - bs - 1) / (fit - bs)));  // sum of ceil(u / hi) <= total / hi + bs
-    const int cand = lo + (int)(((int64_t)(hi - lo) * lane) / 63);
-    int count = 0;
-    for (int b = wave; b < bs; b += 4) count += dense_parts(s_units[b], cand);
-    s_count[wave][lane] = count;
-    __syncthreads();
-    count = s_count[0][lane] + s_count[1][lane] + s_count[2][lane] + s_count[3][lane];
-    const uint64_t ok = __ballot(count <= fit);
-    len = __shfl(cand, ok ? __builtin_ctzll(ok) : 63, 64);
-  }
-  if (!kept || fit <= bs) {  // one part per pair
-    for (int e = tid; e < blocks; e += 256) {
-      DenseItem it = {-1, 0, 0, 0, 1, 0, -1, 0};
-      if (e < bs * kDenseKV) {
-        const int b = e / kDenseKV;
-        const int64_t req = a.s.rpi[b];
-        it.bh = e;
-        it.rows = dense_rows(a, b);
-        it.u1 = dense_units(it.rows);
-        it.req = req >= 0 && req < a.r2t_rows ? (int)req : -1;
-      }
-      plan[e] = it;
-    }
+  if (rules::dense_one_round(bs, round)) {
+    plan_one_round(a, plan, fit, round, grid);
     return;
   }
-  // parts before each request: a prefix sum, 256 requests at a time
-  int base = 0;
-  for (int b0 = 0; b0 < bs; b0 += 256) {
-    const int b = b0 + tid;
-    const int mine = b < bs ? dense_parts(s_units[b], len) : 0;
-    int x = mine;
+  if (tid == 0) queue->next = (uint32_t)grid;
+  __shared__ int s_first[kPlanReqs + 1];  // parts (per KV head) before each request
+  __shared__ int s_rows[kPlanReqs], s_req[kPlanReqs];
+  __shared__ int64_t s_sum[4];
+  __shared__ int s_tmp[4], s_count[4][64];
+  const int wave = tid >> 6, lane = tid & 63;
+  int64_t total = 0;
+  int longest = 1;
+  auto load_request = [&](int b) -> int {
+    const int64_t req = a.s.rpi[b];
+    const int rows = dense_rows(a, b);
+    s_rows[b & (kPlanReqs - 1)] = rows;
+    s_req[b & (kPlanReqs - 1)] = req >= 0 && req < a.r2t_rows ? (int)req : -1;
+    return rows;
+  };
+  for (int b = tid; b < bs; b += 256) {
+    const int u = dense_units(load_request(b));
+    total += u;
+    longest = max(longest, u);
+  }
+  // the words of requests c0 ... of a batch that LDS does not keep whole
+  auto load_requests = [&](int c0) {
+    if (bs <= kPlanReqs) return;
+    __syncthreads();
+    for (int b = c0 + tid; b < min(c0 + kPlanReqs, bs); b += 256) load_request(b);
+    __syncthreads();
+  };
 #pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const int y = __shfl_up(x, d, 64);
-      if (lane >= d) x += y;
-    }
-    __syncthreads();
-    if (lane == 63) s_tmp[wave] = x;
-    __syncthreads();
-    int before = base;
-    for (int w = 0; w < wave; ++w) before += s_tmp[w];
-    if (b < bs) s_first[b] = (uint16_t)(before + x - mine);
-    base += s_tmp[0] + s_tmp[1] + s_tmp[2] + s_tmp[3];
+  for (int d = 32; d >= 1; d >>= 1) {
+    total += __shfl_xor((long long)total, d, 64);
+    longest = max(longest, __shfl_xor(longest, d, 64));
   }
-  if (tid == 0) s_first[bs] = (uint16_t)base;
+  if (lane == 0) {
+    s_sum[wave] = total;
+    s_tmp[wave] = longest;
+  }
   __syncthreads();
-  for (int e = tid; e < blocks; e += 256) {
-    DenseItem it = {-1, 0, 0, 0, 1, 0, -1, 0};
-    // blocks of a request: its parts of KV head 0, then of head 1, ...
-    if (e < base * kDenseKV) {
-      int b = 0, b_end = bs;  // the last request whose first block is <= e
-      while (b_end - b > 1) {
-        const int mid = (b + b_end) >> 1;
-        if (s_first[mid] * kDenseKV <= e) b = mid;
-        else b_end = mid;
+  const int total32 = (int)min(s_sum[0] + s_sum[1] + s_sum[2] + s_sum[3], (int64_t)rules::kDenseMaxTotal);
+  longest = max(max(s_tmp[0], s_tmp[1]), max(s_tmp[2], s_tmp[3]));
+  if (fit <= bs || dense_all_whole(total32, longest, bs, round)) {
+    for (int c0 = 0; c0 < bs; c0 += kPlanReqs) {
+      load_requests(c0);
+      for (int e = c0 * kDenseKV + tid; e < min(c0 + kPlanReqs, bs) * kDenseKV; e += 256) {
+        const int r = e / kDenseKV - c0;
+        plan[e] = {e, 0, dense_units(s_rows[r]), 0, 1, s_rows[r], s_req[r], 0};
       }
-      const int parts = s_first[b + 1] - s_first[b];
-      const int at = e - s_first[b] * kDenseKV;
-      const int h = at / parts, part = at - h * parts;
-      const int units = s_units[b];
-      const int64_t req = a.s.rpi[b];
-      it.bh = b * kDenseKV + h;
-      it.u0 = dense_part_begin(units, part, parts);
-      it.u1 = dense_part_begin(units, part + 1, parts);
-      it.part = part;
-      it.parts = parts;
-      it.rows = dense_rows(a, b);
-      it.req = req >= 0 && req < a.r2t_rows ? (int)req : -1;
     }
-    plan[e] = it;
+    for (int e = bs * kDenseKV + tid; e < grid; e += 256) plan[e] = {-1, 0, 0, 0, 1, 0, -1, 0};
+    return;
   }
+  const int cand = dense_candidate(dense_range(total32, longest, bs, fit, round), lane);
+  const float inv = 1.0f / (float)cand;
+  int count = 0;
+  for (int c0 = 0; c0 < bs; c0 += kPlanReqs) {
+    load_requests(c0);
+#pragma unroll 4
+    for (int b = wave; b < min(kPlanReqs, bs - c0); b += 4)
+      count += dense_parts_inv(dense_units(s_rows[b]), cand, inv);
+  }
+  s_count[wave][lane] = count;
+  __syncthreads();
+  count = s_count[0][lane] + s_count[1][lane] + s_count[2][lane] + s_count[3][lane];
+  const float cost = dense_cost(total32, count, cand, fit, round);
+  float least_cost = cost;
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1) least_cost = fminf(least_cost, __shfl_xor(least_cost, d, 64));
+  const int best = __builtin_ctzll(__ballot(cost == least_cost));
+  const bool fits = least_cost < rules::kDenseNoFit;
+  const int len = fits ? __shfl(cand, best, 64) : 1 << 30;
+  const int parts_all = fits ? __shfl(count, best, 64) : bs;
+  const int classes = parts_all > round ? 2 : 1;
+  const int queued = parts_all * kDenseKV > grid ? parts_all * kDenseKV : 0;
+  int base = 0;  // parts so far
+  for (int cls = 0; cls < classes; ++cls)
+    for (int c0 = 0; c0 < bs; c0 += kPlanReqs) {
+      load_requests(c0);
+      const int n = min(kPlanReqs, bs - c0), base0 = base;
+      // parts before each request: a prefix sum, 256 requests at a time
+      for (int b0 = 0; b0 < n; b0 += 256) {
+        const int b = b0 + tid;
+        int mine = 0;
+        if (b < n) {
+          const int u = dense_units(s_rows[b]);
+          mine = dense_parts(u, len);
+          if (classes > 1 && dense_first(u, mine, len) != (cls == 0)) mine = 0;
+        }
+        int x = mine;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+          const int y = __shfl_up(x, d, 64);
+          if (lane >= d) x += y;
+        }
+        __syncthreads();
+        if (lane == 63) s_tmp[wave] = x;
+        __syncthreads();
+        int before = base;
+        for (int w = 0; w < wave; ++w) before += s_tmp[w];
+        if (b < n) s_first[b] = before + x - mine;
+        base += s_tmp[0] + s_tmp[1] + s_tmp[2] + s_tmp[3];
+      }
+      if (tid == 0) s_first[n] = base;
+      __syncthreads();
+      // blocks of a request: its parts of KV head 0, then of head 1, ...
+      for (int e = base0 * kDenseKV + tid; e < base * kDenseKV; e += 256) {
+        int b = 0, b_end = n;  // the last request whose first block is <= e
+        while (b_end - b > 1) {
+          const int mid = (b + b_end) >> 1;
+          if (s_first[mid] * kDenseKV <= e) b = mid;
+          else b_end = mid;
+        }
+        const int parts = s_first[b + 1] - s_first[b];
+        const int at = e - s_first[b] * kDenseKV;
+        const int h = at / parts, part = at - h * parts;
+        const int units = dense_units(s_rows[b]);
+        plan[e] = {(c0 + b) * kDenseKV + h, dense_part_begin(units, part, parts), dense_part_begin(units, part + 1, parts),
+                   part, parts, s_rows[b], s_req[b], queued};
+      }
+      __syncthreads();  // s_first is free
+    }
+  for (int e = base * kDenseKV + tid; e < grid; e += 256) plan[e] = {-1, 0, 0, 0, 1, 0, -1, 0};
 }
 
 // The parts of a pair added up by a whole block: the weights e^(m - max) of every
@@ -559,61 +650,91 @@ __device__ inline void merge_dense(const StepArgs& a, int bh, int64_t part0, int
 //
 // Bound: HBM.  Attention and store, per layer at 32 / 4 heads, against blocks of 4096
 // rows each, as many per pair as the table's width holds: one request of 8000 rows
-// 49 -> 18 us, of 100000 83 -> 52; 16 ragged requests of 2000 .. 65000 in a
+// 49 -> 17 us, of 100000 83 -> 52; 16 ragged requests of 2000 .. 65000 in a
 // 131072-wide table 480 -> 106 (4.6 TB/s); 16 of 131000 785 -> 745 (5.8 TB/s); 64 of
-// 3000 84 -> 76.  4-wave blocks, two per CU: 64 of 3000 87 us, one of 100000 63 (twice
+// 3000 84 -> 77.  4-wave blocks, two per CU: 64 of 3000 87 us, one of 100000 63 (twice
 // the parts to merge), one of 8000 16.9.
-__global__ __launch_bounds__(64 * kDenseWaves, 2) void dense_attend_kernel(StepArgs a, const DenseItem* plan) {
+// QUEUE: batches whose plan may have more parts than the grid has blocks.  Against one
+// round of parts as the limit (a pair per block from 64 requests on): 100000 rows and 63
+// x 2000 1175 -> 103 us, 2 x 100000 and 126 x 300 1171 -> 107, 8 x 30000 and 48 x 500
+// 207 -> 137, 70 x 10000 342 -> 311; 128 x 3000 143 -> 145, 64 x 3000 76.5 -> 77.  A
+// block per entry instead of the queue, 512 more of them, costs those 5 us.
+// A kernel's first argument, read anew from its argument block: kept in scalar registers
+// over a loop, the arguments would be spilt there.
+__device__ inline StepArgs reread_args(const StepArgs&) {
+  typedef const __attribute__((address_space(4))) char* arg_ptr_t;
+  arg_ptr_t p = (arg_ptr_t)__builtin_amdgcn_kernarg_segment_ptr();
+  __asm__ volatile("" : "+s"(p));
+  StepArgs a;
+  __builtin_memcpy(&a, (const void*)p, sizeof(a));
+  return a;
+}
+
+template <bool QUEUE>
+__global__ __launch_bounds__(64 * kDenseWaves, 2) void dense_attend_kernel(StepArgs args, const DenseItem* plan,
+                                                                        DenseQueue* queue) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   DenseSmem& sm = *reinterpret_cast<DenseSmem*>(smem_raw);
-  const SelectArgs& sa = a.s;
-  const DenseItem it = plan[blockIdx.x];
-  if (it.bh < 0) return;
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int lo = lane & 15, hi = lane >> 4;
-  const int G = a.G, n = it.rows;
-  const int b = it.bh / kDenseKV, h = it.bh - b * kDenseKV;
-  const int32_t* rt = a.r2t + (int64_t)max(it.req, 0) * a.r2t_stride;
-  // units with rows: a request without any has one unit and no rows
-  const int u_end = min(it.u1, (n + 63) / 64);
-  // lane l: the pool row of token l of a unit, as the table has it (row 0 past the
-  // context); looked at a unit later, so that it is loaded under the unit before
-  auto table_row = [&](int j) -> int {
-    const int slot = j * 64 + lane;
-    return (j < u_end && slot < n && it.req >= 0) ? rt[slot] : 0;
-  };
-  int row = table_row(it.u0 + wave);
-  bf16x8_t qb[4];
-  {
-    const uint16_t* qp = static_cast<const uint16_t*>(sa.q) + (int64_t)b * sa.q_bstride +
-                         (int64_t)(h * G + lo) * kMfmaDim + hi * 8;
+  for (int e = blockIdx.x, turn = 0;; turn ^= 1) {
+    const StepArgs a = QUEUE ? reread_args(args) : args;
+    const SelectArgs& sa = a.s;
+    const int G = a.G;
+    const DenseItem it = plan[e];
+    if (it.bh < 0) return;
+    uint32_t next = 0;
+    if (QUEUE && it.queued && tid == 0)
+      next = __hip_atomic_fetch_add(&queue->next, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const int n = it.rows;
+    const int b = it.bh / kDenseKV, h = it.bh - b * kDenseKV;
+    const int32_t* rt = a.r2t + (int64_t)max(it.req, 0) * a.r2t_stride;
+    // units with rows: a request without any has one unit and no rows
+    const int u_end = min(it.u1, (n + 63) / 64);
+    // lane l: the pool row of token l of a unit, as the table has it (row 0 past the
+    // context); looked at a unit later, so that it is loaded under the unit before
+    auto table_row = [&](int j) -> int {
+      const int slot = j * 64 + lane;
+      return (j < u_end && slot < n && it.req >= 0) ? rt[slot] : 0;
+    };
+    int row = table_row(it.u0 + wave);
+    bf16x8_t qb[4];
+    {
+      const uint16_t* qp = static_cast<const uint16_t*>(sa.q) + (int64_t)b * sa.q_bstride +
+                           (int64_t)(h * G + lo) * kMfmaDim + hi * 8;
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      if (lo < G) {
-        qb[ks] = *reinterpret_cast<const bf16x8_t*>(qp + ks * 32);
-      } else {
-        qb[ks] = __builtin_bit_cast(bf16x8_t, u32x4_t{0u, 0u, 0u, 0u});
+      for (int ks = 0; ks < 4; ++ks) {
+        if (lo < G) {
+          qb[ks] = *reinterpret_cast<const bf16x8_t*>(qp + ks * 32);
+        } else {
+          qb[ks] = __builtin_bit_cast(bf16x8_t, u32x4_t{0u, 0u, 0u, 0u});
+        }
       }
     }
-  }
-  const uint16_t* kb = a.k + h * kMfmaDim;
-  const uint16_t* vb = a.v + h * kMfmaDim;
-  float M = -INFINITY, L = 0.0f;
-  float4_t o[8];
+    const uint16_t* kb = a.k + h * kMfmaDim;
+    const uint16_t* vb = a.v + h * kMfmaDim;
+    float M = -INFINITY, L = 0.0f;
+    float4_t o[8];
 #pragma unroll
-  for (int e = 0; e < 8; ++e) o[e] = float4_t{0.f, 0.f, 0.f, 0.f};
-  // the row and the query are in; the compiler then knows that a unit's row, loaded
-  // under the unit before, needs no wait, which would be one for the next row too
-  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-  for (int j = it.u0 + wave; j < u_end; j += kDenseWaves) {
-    const int next = table_row(j + kDenseWaves);
-    attend_unit(row >= 0 && row < a.kv_rows ? row : 0, min(n - j * 64, 64), kb, vb, 9, qb, a.sl2, M, L, o);
-    row = next;
+    for (int e = 0; e < 8; ++e) o[e] = float4_t{0.f, 0.f, 0.f, 0.f};
+    // the row and the query are in; the compiler then knows that a unit's row, loaded
+    // under the unit before, needs no wait, which would be one for the next row too
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+    if (QUEUE && tid == 0) sm.next[turn] = next;  // read after this part's barriers
+    for (int j = it.u0 + wave; j < u_end; j += kDenseWaves) {
+      const int row_next = table_row(j + kDenseWaves);
+      attend_unit(row >= 0 && row < a.kv_rows ? row : 0, min(n - j * 64, 64), kb, vb, 9, qb, a.sl2, M, L, o);
+      row = row_next;
+    }
+    combine_block<kDenseWaves>(a, it.bh, it.parts == 1, e, M, L, o, false, sm.comb.m, sm.comb.l, sm.comb.o);
+    if (it.parts > 1 && last_part(a, it.bh, it.parts, &sm.last))
+      merge_dense(a, it.bh, (int64_t)e - it.part, it.parts, sm);
+    if (!QUEUE || !it.queued) return;
+    __syncthreads();  // this part's LDS is free
+    e = __builtin_amdgcn_readfirstlane((int)sm.next[turn]);
+    if (e >= it.queued) return;
   }
-  combine_block<kDenseWaves>(a, it.bh, it.parts == 1, blockIdx.x, M, L, o, false, sm.comb.m, sm.comb.l, sm.comb.o);
-  if (it.parts > 1 && last_part(a, it.bh, it.parts, &sm.last))
-    merge_dense(a, it.bh, (int64_t)blockIdx.x - it.part, it.parts, sm);
 }
 
 // ------------------------------------------------------- per-page-unit attention
@@ -770,11 +891,12 @@ static int device_cu_count() {
 
 // LDS of the dense attention kernel (above the 64 KiB default: opted in once per
 // device).
+template <bool QUEUE>
 static size_t dense_smem_bytes() {
   static bool opted[64] = {false};
   int dev = 0;
   if (hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < 64 && !opted[dev]) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&dense_attend_kernel),
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&dense_attend_kernel<QUEUE>),
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(DenseSmem));
     opted[dev] = true;
   }
@@ -920,12 +1042,15 @@ int qq::attend_rows_fused(const void* q, int64_t q_bstride, int num_q_heads, con
   return QQ_OK;
 }
 
-static int64_t dense_blocks(int bs, int64_t max_rows) { return rules::dense_blocks(device_cu_count(), bs, max_rows); }
+// Parts that the plan holds, at most.
+static int64_t dense_entries(int bs, int64_t max_rows) {
+  return rules::dense_fit(device_cu_count(), bs, max_rows) * kDenseKV;
+}
 
 extern "C" int64_t qq_dense_decode_workspace_bytes(int bs, int64_t max_rows, int num_q_heads, int kv_heads) {
   if (bs <= 0 || max_rows <= 0 || kv_heads <= 0 || num_q_heads <= 0) return 0;
-  // the division of the batch, then the parts' (m, l, o)
-  return dense_blocks(bs, max_rows) *
+  // the queue, the division of the batch, then the parts' (m, l, o)
+  return (int64_t)sizeof(DenseQueue) + dense_entries(bs, max_rows) *
          (int64_t)(sizeof(DenseItem) + (num_q_heads / kv_heads) * (kMfmaDim + 2) * sizeof(float));
 }
 
@@ -954,8 +1079,11 @@ extern "C" int qq_dense_forward_decode(const void* q, int q_dtype, int64_t q_bat
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int top_k = (int)req_to_token_stride;  // every context fits: seq_len <= the table's width
   const int G = num_q_heads / kv_heads;
-  const int64_t blocks = dense_blocks(bs, top_k);
-  QQ_REQUIRE(blocks < (int64_t)1 << 31 && req_to_token_rows < (int64_t)1 << 31, "%s: bad sizes", what);
+  const int64_t entries = dense_entries(bs, top_k);
+  const int round = rules::dense_round(device_cu_count());
+  // a block for every (request, KV head), or as many as are resident at once
+  const int64_t grid = std::min(entries, std::max<int64_t>((int64_t)bs * kDenseKV, round * kDenseKV));
+  QQ_REQUIRE(entries < (int64_t)1 << 31 && req_to_token_rows < (int64_t)1 << 31, "%s: bad sizes", what);
   StepArgs a{};
   a.s.q = q;
   a.s.q_dtype = QQ_DTYPE_BF16;
@@ -974,9 +1102,10 @@ extern "C" int qq_dense_forward_decode(const void* q, int q_dtype, int64_t q_bat
   a.r2t_rows = req_to_token_rows;
   a.sl2 = scale * kLog2e;
   a.out = static_cast<uint16_t*>(out);
-  DenseItem* plan = static_cast<DenseItem*>(workspace);
-  a.part_o = reinterpret_cast<float*>(plan + blocks);
-  a.part_ml = a.part_o + blocks * G * kMfmaDim;
+  DenseQueue* queue = static_cast<DenseQueue*>(workspace);
+  DenseItem* plan = reinterpret_cast<DenseItem*>(queue + 1);
+  a.part_o = reinterpret_cast<float*>(plan + entries);
+  a.part_ml = a.part_o + entries * G * kMfmaDim;
   a.sync = static_cast<uint32_t*>(sync);
   a.bs = bs;
   a.G = G;
@@ -1000,8 +1129,12 @@ extern "C" int qq_dense_forward_decode(const void* q, int q_dtype, int64_t q_bat
   a.s.v_pool = v_layer;
   a.s.pool_dtype = QQ_DTYPE_BF16;
   a.s.pool_rows = kv_rows;
-  dense_store_plan_kernel<<<store ? bs + 1 : 1, 256, 0, s>>>(a, plan, (int)blocks);
-  dense_attend_kernel<<<(int)blocks, 64 * kDenseWaves, dense_smem_bytes(), s>>>(a, plan);
+  dense_store_plan_kernel<<<store ? bs + 1 : 1, 256, 0, s>>>(a, plan, queue, (int)(entries / kDenseKV), round,
+                                                             (int)grid);
+  if (entries > grid)
+    dense_attend_kernel<true><<<(int)grid, 64 * kDenseWaves, dense_smem_bytes<true>(), s>>>(a, plan, queue);
+  else
+    dense_attend_kernel<false><<<(int)grid, 64 * kDenseWaves, dense_smem_bytes<false>(), s>>>(a, plan, queue);
   return check_launch(what);
 }
 

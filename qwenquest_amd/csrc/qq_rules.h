@@ -55,11 +55,13 @@ constexpr UnitShape unit_shape(int64_t cus, int64_t bs, int kv_heads, int top_k)
 constexpr int unit_first(int wave, int part, int parts) { return wave * parts + part; }
 
 // ------------------------------------------------------------- dense decode
-constexpr int kDenseKV = 4;                            // KV heads of the dense decode kernel (KV*D = 512)
-constexpr int kDenseBlocks = 256;                      // one per CU, at most: all resident
-constexpr int kDenseParts = kDenseBlocks / kDenseKV;   // parts of a (request, KV head), at most
-constexpr int kDenseWhole = 8;                         // units of a pair that is not split
-constexpr int kDenseMinLen = 2;                        // units of a part, at least
+// A (request, KV head) pair's 64-row units are split into equal parts, one to a block;
+// a CU holds one block.  Per KV head, `round` blocks are resident at once.
+constexpr int kDenseKV = 4;        // KV heads of the dense decode kernel (KV*D = 512)
+constexpr int kDenseBlocks = 256;  // blocks of a round, at most
+constexpr int kDenseParts = 64;    // parts of a pair, at most: the merge's table of weights
+constexpr int kDenseWhole = 8;     // units of a pair that is not split
+constexpr int kDenseMinLen = 2;    // units of a part, at least
 
 // Units of 64 rows; a request without rows has one, which writes its zeros.
 constexpr int dense_units(int rows) { return (int)most((rows + 63) / 64, 1); }
@@ -69,18 +71,81 @@ constexpr int dense_units(int rows) { return (int)most((rows + 63) / 64, 1); }
 // parts); longer ones may go down to two units a part (four of 1000 rows: 16.5 us, at
 // four units 17.4, at eight 19.6; one of 8000: 18.0, 17.8 and 19.9).
 constexpr int dense_parts(int units, int len) {
-  return units <= kDenseWhole ? 1 : (units + len - 1) / len;
+  return units <= kDenseWhole ? 1 : (int)least((units + len - 1) / len, kDenseParts);
 }
 
 // First unit of part `part` of `parts` of a pair: equal parts.
 constexpr int dense_part_begin(int units, int part, int parts) { return (int)((int64_t)units * part / parts); }
 
-// Blocks: one per CU, or as many as the table's width can use; at least one per
-// (request, KV head).
-constexpr int64_t dense_blocks(int64_t cus, int64_t bs, int64_t max_rows) {
-  const int64_t pairs = bs * kDenseKV, units = pairs * ((max_rows + 63) / 64);
-  return most(pairs, least(least(cus, kDenseBlocks), units));
+constexpr int dense_round(int64_t cus) { return (int)most(least(cus, kDenseBlocks) / kDenseKV, 1); }
+
+// Batches that one round of blocks always divides well enough: parts of `len` units fit
+// a round from len = total / (round - bs) on, and a CU alone reads 8/5 of its share of
+// the chip's rate (36 GB/s of 22.6), so that parts of up to 8/5 of the mean cost nothing:
+// up to 3/8 of the round's parts.
+constexpr bool dense_one_round(int64_t bs, int round) { return 8 * bs <= 3 * (int64_t)round; }
+
+// Parts per KV head that the grid holds (it is sized without the lengths, which are on
+// the device): one round, or for larger batches one part per request and two rounds'
+// more, with which any batch divides into parts of half the mean; no more than the
+// table's width can need.  An entry without work is a block that exits.
+constexpr int64_t dense_fit(int64_t cus, int64_t bs, int64_t max_rows) {
+  const int64_t units = most(ceil_of(max_rows, 64), 1), round = dense_round(cus);
+  if (units <= kDenseWhole) return bs;
+  if (dense_one_round(bs, (int)round)) return most(bs, least(round, bs * units));
+  return bs + least(2 * round, bs * (ceil_of(units, kDenseMinLen) - 1));
 }
+
+// The part lengths that are tried, 64 from lo to hi, for `total` units per KV head of
+// which one pair has `longest`; fit > bs.  (32-bit, as one block computes it before the
+// attention can start; a total above kDenseMaxTotal stands for more, and dense_cost then
+// finds the lengths that do not fit.)
+constexpr int kDenseMaxTotal = 1 << 24;
+struct DenseRange {
+  int lo, hi;
+};
+constexpr int ceil32(int a, int b) { return (a + b - 1) / b; }
+constexpr int least32(int a, int b) { return a < b ? a : b; }
+constexpr int most32(int a, int b) { return a > b ? a : b; }
+constexpr DenseRange dense_range(int total, int longest, int bs, int fit, int round) {
+  if (dense_one_round(bs, round)) {
+    const int lo = most32(ceil32(total, fit), kDenseMinLen);
+    return {lo, most32(lo, least32(longest, ceil32(total, fit - bs)))};  // sum of ceil(u / hi) <= fit
+  }
+  const int lo = most32(ceil32(total, fit - bs), kDenseMinLen);  // sum of ceil(u / lo) <= fit
+  int hi = least32(longest, 4 * ceil32(total, round));
+  if (bs < round) hi = least32(hi, ceil32(total, round - bs));  // fits one round
+  return {lo, most32(lo, hi)};
+}
+constexpr int dense_candidate(DenseRange r, int lane) { return r.lo + (r.hi - r.lo) * lane / 63; }
+
+// What a division into `count` parts of up to `len` units costs, in the time that the
+// chip at its full rate takes for one unit per block: the whole at that rate, or 5/8 of
+// the longest run of parts on a CU, which reads that much faster alone, and six units
+// (about 9 us) for the start and end of each block on it.  The first of the cheapest
+// lengths is taken; where none fits, no pair is split.  (It takes halves for 70 x 10000
+// rows, 311 us against 342 in whole pairs, and for 65 x 3000, 110 against 111.)
+constexpr float kDenseNoFit = 1e30f;
+constexpr float dense_run(int total, int count, int len, int round) {  // 5/8 of the longest run on a CU
+  const float rounds = (float)ceil32(count, round), even = rounds * (float)total / (float)count;
+  return 0.625f * (rounds > 1.0f && even > (float)len ? even : (float)len);
+}
+constexpr float dense_cost(int total, int count, int len, int fit, int round) {
+  if (count > fit) return kDenseNoFit;
+  const float run = dense_run(total, count, len, round), mean = (float)total / (float)round;
+  return (run > mean ? run : mean) + 6.0f * (float)ceil32(count, round);
+}
+
+// No pair is split where that cannot cost more than any division: short pairs, or a run
+// of whole ones that the chip's rate hides.  (The lengths are then not tried, which the
+// attention waits for: 3.5 us at 128 requests, 9 at 300.)
+constexpr bool dense_all_whole(int total, int longest, int bs, int round) {
+  return longest <= kDenseWhole || dense_run(total, bs, longest, round) <= (float)total / (float)round;
+}
+
+// Where the parts take more than one round, those longer than half the part length come
+// first, so that a round's end does not wait for a long one.
+constexpr bool dense_first(int units, int parts, int len) { return 2 * ((units + parts - 1) / parts) > len; }
 
 // ------------------------------------------------------------------ prefill
 constexpr int kExtRows = 128;      // query rows per block

@@ -1,6 +1,7 @@
-"""Dense decode's division of a batch into equal runs (reference
-``src/qwenquest/attention/dense.py:26-42``): runs that end inside a request, inside a KV head's
-rows or cover many requests, merges over one and several thread groups, against float64."""
+"""Dense decode's division of a batch into parts (reference
+``src/qwenquest/attention/dense.py:26-42``): (request, KV head) pairs whole and in up to 64 equal
+parts, one part per block and blocks that take several, merges over one and several thread groups,
+against float64."""
 
 from __future__ import annotations
 
@@ -18,15 +19,21 @@ class Layer:
 
 
 @pytest.mark.parametrize("heads,ctx,width", [
-    (32, [8000], 8064),  # one request over 125 blocks
+    (32, [8000], 8064),  # one request: 63 parts per KV head
     (16, [4097, 63], 4200),  # groups of 4: two thread groups merge
     (20, [2500, 1, 64, 65], 2600),  # groups of 5: threads past the merge's items
     (28, [700] * 3 + [3001], 3100),
     (4, [5000, 256], 5100),  # no grouping: eight thread groups merge
     (64, [3000, 17], 3100),  # groups of 16: two items per thread
     (8, [130, 0, 64], 200),  # a request without rows: zeros
-    (32, [1 + 37 * i for i in range(70)], 2700),  # more requests than lanes
+    (32, [1 + 37 * i for i in range(70)], 2700),  # more requests than a round has parts
     (32, [20000, 300, 9000], 131072),  # several units per wave; a table far wider than the contexts
+    (32, [9000] + [300] * 66, 9100),  # one long request among many: its parts go to blocks that are done
+    (20, [4000, 100] * 15, 4100),  # fewer requests than a round has parts, two rounds
+    (28, [1500] * 24 + [1600], 1700),  # 24 and 25 requests: the last batch of one round and the next
+    (28, [1500] * 24, 1700),
+    (8, [700, 0] * 40, 800),  # requests without rows among split ones
+    (4, [9000, 1, 5000, 0] + [5] * 1100, 9100),  # more requests than the plan keeps in LDS
 ])
 def test_dense_decode_matches_float64(heads, ctx, width):
     from qwenquest_amd.attention.dense import DenseBackend
