@@ -358,7 +358,8 @@ int qq_extend_verdict_wait(const int64_t* verdict, void* stream);
  * otherwise); seq_lens[i] <= req_to_token_stride.  sync as for
  * qq_quest_forward_decode (>= qq_quest_layer_step_sync_bytes(bs, 4), zeroed
  * once, left zeroed); workspace >= qq_dense_decode_workspace_bytes(bs,
- * req_to_token_stride, H, KV).  Two launches: the K/V store with the division of
+ * req_to_token_stride, H, KV), of any contents, this call's alone until its launches
+ * are done.  Two launches: the K/V store with the division of
  * the batch into parts that keep the chip evenly busy (on the device, from seq_lens),
  * then the attention over the parts, merged inside the launch. */
 int qq_dense_forward_decode(const void* q, int q_dtype, int64_t q_batch_stride, int num_q_heads,

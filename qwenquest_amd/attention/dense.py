@@ -32,10 +32,9 @@ class DenseBackend(AttentionBackend):
         super().__init__(req_to_token_pool, token_to_kv_pool)
         device = token_to_kv_pool.device
         lib = _lib.load()
-        # the attention's (request, KV head) counters: zeroed once, left zeroed by every call
+        # (request, KV head) counters, as the C entry asks for them
         sync_bytes = int(lib.qq_quest_layer_step_sync_bytes(req_to_token_pool.size, token_to_kv_pool.kv_heads))
         self._sync = torch.zeros(max(sync_bytes, 4), dtype=torch.uint8, device=device)
-        self._ws = torch.empty(0, dtype=torch.uint8, device=device)
         self._rows_ws = AttentionWorkspace(device)
 
     def _fast(self, q3: torch.Tensor) -> bool:
@@ -68,15 +67,16 @@ class DenseBackend(AttentionBackend):
         vn = v.reshape(bs, pool.kv_heads * dim).to(torch.bfloat16).contiguous()
         loc = batch.out_cache_loc.to(device=q3.device, dtype=torch.int64).contiguous()
         need = int(_lib.load().qq_dense_decode_workspace_bytes(bs, r2t.stride(0), heads, pool.kv_heads))
-        if self._ws.numel() < need:
-            self._ws = torch.empty(need, dtype=torch.uint8, device=q3.device)
+        # of this call alone: it holds the division of the batch, which a graph's replay or a call
+        # on another stream must not find replaced
+        ws = torch.empty(need, dtype=torch.uint8, device=q3.device)
         out = torch.empty((bs, heads * dim), dtype=q3.dtype, device=q3.device)
         _lib.call(
             "qq_dense_forward_decode", _lib.ptr(q3), _lib.dtype_code(q3.dtype), q3.stride(0), heads,
             _lib.ptr(kn), _lib.ptr(vn), _lib.dtype_code(kn.dtype), _lib.ptr(loc), _lib.ptr(k_buf),
             _lib.ptr(v_buf), _lib.dtype_code(k_buf.dtype), k_buf.shape[0], pool.kv_heads, dim, _lib.ptr(rpi),
             _lib.ptr(seq), bs, _lib.ptr(r2t), r2t.stride(0), r2t.shape[0], float(layer.scaling), _lib.ptr(out),
-            _lib.ptr(self._ws) if need else None, need, _lib.ptr(self._sync), self._sync.numel(),
+            _lib.ptr(ws), need, _lib.ptr(self._sync), self._sync.numel(),
             _lib.stream(q3.device),
         )
         return out

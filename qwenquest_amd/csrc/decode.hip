@@ -420,16 +420,20 @@ __device__ inline void plan_one_round(const StepArgs& a, DenseItem* plan, int fi
 }
 
 // Block 0: the division of the batch, `fit` parts per KV head at most; blocks 1 .. bs:
-// the new tokens (memory.py:114-120).  64 part lengths are tried, one per lane, the waves
+// the new tokens (memory.py:114-120), and the parts' counters.  64 part lengths are tried, one per lane, the waves
 // sharing the requests (dense_range, dense_cost), and every entry finds its request.  The
 // requests' words are kept in LDS, kPlanReqs of them at a time.
 __global__ __launch_bounds__(256) void dense_store_plan_kernel(StepArgs a, DenseItem* plan, DenseQueue* queue, int fit,
                                                                int round, int grid) {
   const int bs = a.bs, tid = threadIdx.x;
   if (blockIdx.x > 0) {
-    store_new_token(a.s, blockIdx.x - 1);
+    const int b = blockIdx.x - 1;
+    if (tid < kDenseKV) *attn_count(a, b * kDenseKV + tid) = 0u;
+    store_new_token(a.s, b);
     return;
   }
+  if (gridDim.x == 1)  // no blocks of new tokens
+    for (int i = tid; i < bs * kDenseKV; i += 256) *attn_count(a, i) = 0u;
   if (rules::dense_one_round(bs, round)) {
     plan_one_round(a, plan, fit, round, grid);
     return;
@@ -1049,8 +1053,8 @@ static int64_t dense_entries(int bs, int64_t max_rows) {
 
 extern "C" int64_t qq_dense_decode_workspace_bytes(int bs, int64_t max_rows, int num_q_heads, int kv_heads) {
   if (bs <= 0 || max_rows <= 0 || kv_heads <= 0 || num_q_heads <= 0) return 0;
-  // the queue, the division of the batch, then the parts' (m, l, o)
-  return (int64_t)sizeof(DenseQueue) + dense_entries(bs, max_rows) *
+  // the parts' counters, the queue, the division of the batch, then the parts' (m, l, o)
+  return qq_quest_layer_step_sync_bytes(bs, kDenseKV) + (int64_t)sizeof(DenseQueue) + dense_entries(bs, max_rows) *
          (int64_t)(sizeof(DenseItem) + (num_q_heads / kv_heads) * (kMfmaDim + 2) * sizeof(float));
 }
 
@@ -1102,11 +1106,13 @@ extern "C" int qq_dense_forward_decode(const void* q, int q_dtype, int64_t q_bat
   a.r2t_rows = req_to_token_rows;
   a.sl2 = scale * kLog2e;
   a.out = static_cast<uint16_t*>(out);
-  DenseQueue* queue = static_cast<DenseQueue*>(workspace);
+  // everything of the call lies in its workspace: calls on several streams share nothing
+  a.sync = static_cast<uint32_t*>(workspace);
+  DenseQueue* queue = reinterpret_cast<DenseQueue*>(static_cast<unsigned char*>(workspace) +
+                                                    qq_quest_layer_step_sync_bytes(bs, kDenseKV));
   DenseItem* plan = reinterpret_cast<DenseItem*>(queue + 1);
   a.part_o = reinterpret_cast<float*>(plan + entries);
   a.part_ml = a.part_o + entries * G * kMfmaDim;
-  a.sync = static_cast<uint32_t*>(sync);
   a.bs = bs;
   a.G = G;
   a.kv_shift = kv_shift_of(kDenseKV);

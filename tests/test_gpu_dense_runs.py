@@ -104,3 +104,73 @@ def test_columns_of_a_wider_table():
         batch = ForwardBatch(ForwardMode.DECODE, None, None, rpi, seq, loc, rtp, kvp, be)
         out.append(be.forward_decode(q, k, v, Layer(), batch))
     assert torch.equal(*out)
+
+
+def batch_of(ctx, width, size, seed):
+    from qwenquest_amd.attention.dense import DenseBackend
+    from qwenquest_amd.memory import MHATokenToKVPool, ReqToTokenPool
+
+    rtp = ReqToTokenPool(size, width, DEV)
+    kvp = MHATokenToKVPool(sum(ctx), 1, KV, D, torch.bfloat16, DEV)
+    gen = torch.Generator(device=DEV).manual_seed(seed)
+    kvp.k_all.normal_(generator=gen)
+    kvp.v_all.normal_(generator=gen)
+    at = 1
+    for i, n in enumerate(ctx):
+        rtp.req_to_token[i, :n] = torch.arange(at, at + n, dtype=torch.int32)
+        at += n
+    return rtp, kvp, DenseBackend(rtp, kvp), gen
+
+
+def decode_call(rtp, kvp, be, gen, rpi, ctx):
+    from qwenquest_amd.batch import ForwardBatch, ForwardMode
+
+    rpi, seq = torch.tensor(rpi, device=DEV), torch.tensor(ctx, device=DEV)
+    loc = rtp.req_to_token[rpi, seq - 1].long()
+    q = torch.empty((len(ctx), 32, D), device=DEV).normal_(generator=gen).to(torch.bfloat16)
+    k, v = kvp.k_all[0][loc].clone(), kvp.v_all[0][loc].clone()
+    batch = ForwardBatch(ForwardMode.DECODE, None, None, rpi, seq, loc, rtp, kvp, be)
+    return lambda: be.forward_decode(q, k, v, Layer(), batch)
+
+
+@pytest.mark.parametrize("first,rest", [([3000, 500], [4000] * 3), ([2500] + [300] * 30, [700] * 9)])
+def test_a_captured_call_keeps_its_workspace(first, rest):
+    """A graph captured with a small batch replays after a call with a larger one, and after other
+    tensors took the memory that is free by then."""
+    ctx = first + rest
+    rtp, kvp, be, gen = batch_of(ctx, 4096, len(ctx), 5)
+    small = decode_call(rtp, kvp, be, gen, list(range(len(first))), first)
+    large = decode_call(rtp, kvp, be, gen, list(range(len(ctx))), ctx)
+    want, all_want = small(), large()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = small()
+    for i in range(3):
+        assert torch.equal(large(), all_want)
+        junk = [torch.full((1 << n,), -7, dtype=torch.int32, device=DEV) for n in range(4, 22)]
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want), i
+        assert all(bool((x == -7).all()) for x in junk)
+    assert not be._sync.any()
+
+
+def test_calls_on_two_streams_share_nothing():
+    """Batches of one backend on two streams at once: each call's division, counters and partial
+    sums are its own."""
+    a, b = [4000, 900, 64], [100] * 40 + [3000]
+    rtp, kvp, be, gen = batch_of(a + b, 4096, len(a + b), 6)
+    calls = [decode_call(rtp, kvp, be, gen, list(range(len(a))), a),
+             decode_call(rtp, kvp, be, gen, list(range(len(a), len(a + b))), b)]
+    want = [c() for c in calls]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    got = [[], []]
+    for _ in range(20):
+        for i in (0, 1):
+            with torch.cuda.stream(streams[i]):
+                got[i].append(calls[i]())
+    torch.cuda.synchronize()
+    for i in (0, 1):
+        assert all(torch.equal(x, want[i]) for x in got[i])
