@@ -872,28 +872,22 @@ extern "C" int qq_quest_prefill_bounds(const void* k_base, int64_t k_layer_strid
   const int C = a.C;
   const bool wide = k_dtype == QQ_DTYPE_BF16 && C >= 8 && C <= 8 * kThreads && (C & (C - 1)) == 0 &&
                     k_layer_stride % 8 == 0 && reinterpret_cast<uintptr_t>(k_base) % 16 == 0;
-  if (!wide)
+  const bool per_wave = C == 128 || C == 256 || C == 512 || C == 1024;
+  // the waves' folds keep row numbers in 32 bits (past them the keys are 512 GiB at least)
+  if (!wide || (per_wave && k_rows > INT32_MAX))
     prefill_bounds_kernel<<<grid, kThreads, 0, s>>>(a);
-  else if (C == 512 && k_rows <= INT32_MAX)
+  else if (C == 512)
     prefill_bounds_wave_kernel<1, kWaveFoldBatch, kWavePages>
         <<<dim3(ceil_div(pages, kPfThreads / 64 * kWavePages), n_layers), kPfThreads, 0, s>>>(a);
-  else if (C == 1024 && k_rows <= INT32_MAX)
+  else if (C == 1024)
     prefill_bounds_wave_kernel<2, kWaveFoldBatch, kWavePages>
         <<<dim3(ceil_div(pages, kPfThreads / 64 * kWavePages), n_layers, 2), kPfThreads, 0, s>>>(a);
-  else if (C == 256 && k_rows <= INT32_MAX)
+  else if (C == 256)
     prefill_bounds_groups_kernel<32><<<dim3(ceil_div(pages, kPfThreads / 64), n_layers), kPfThreads, 0, s>>>(a);
-  else if (C == 128 && k_rows <= INT32_MAX)
+  else if (C == 128)
     prefill_bounds_groups_kernel<16><<<dim3(ceil_div(pages, kPfThreads / 64), n_layers), kPfThreads, 0, s>>>(a);
-  else if (C == 512)
-    prefill_bounds_wide_kernel<64><<<grid, kThreads, 0, s>>>(a);
-  else if (C == 1024)
-    prefill_bounds_wide_kernel<128><<<grid, kThreads, 0, s>>>(a);
   else if (C == 2048)
     prefill_bounds_wide_kernel<256><<<grid, kThreads, 0, s>>>(a);
-  else if (C == 256)
-    prefill_bounds_wide_kernel<32><<<grid, kThreads, 0, s>>>(a);
-  else if (C == 128)
-    prefill_bounds_wide_kernel<16><<<grid, kThreads, 0, s>>>(a);
   else if (C == 64)
     prefill_bounds_wide_kernel<8><<<grid, kThreads, 0, s>>>(a);
   else if (C == 32)

@@ -33,3 +33,17 @@ def test_prefill_bounds_match_the_per_element_fold(kv, page, n, kind):
         assert torch.equal(getattr(qb, name).view(torch.int16), getattr(qf, name).view(torch.int16)), name
     for name in ("running_token_count", "running_page_idx"):
         assert torch.equal(getattr(qb, name), getattr(qf, name)), name
+
+
+@pytest.mark.parametrize("kv", [1, 2, 4, 8])
+def test_row_counts_past_32_bits_take_the_general_fold(kv):
+    """A pool said to hold more than 2^31 rows (the indices are small): the same bounds."""
+    pool = rand_bf16((500, kv, 128), seed=kv).to(DEV)
+    idx = torch.randperm(500, generator=torch.Generator().manual_seed(kv))[:333].to(DEV)
+    got = []
+    for rows in (500, 1 << 32):
+        q, _ = new_quest(256, 64, 1, 1, 1024, kv, 128)
+        q._prefill(pool, 0, rows, 0, idx, 0, 1, True)
+        got.append([t.clone() for t in (q.page_k_bounds, q.running_k_min, q.running_k_max, q.running_page_idx)])
+    for a, b in zip(*got, strict=True):
+        assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
