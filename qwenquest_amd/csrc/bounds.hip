@@ -259,20 +259,50 @@ __device__ inline uint32_t u16x2_min(uint32_t a, uint32_t b) {
 __device__ inline uint32_t u16x2_max(uint32_t a, uint32_t b) {
   return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2_t, a), __builtin_bit_cast(u16x2_t, b)));
 }
-// A fold's result as keys is exact unless one of its extremes is a NaN or a zero.  A NaN
-// among the values shows in them: its key lies above +inf's (0xFF80) or below -inf's
-// (0x007F).  A zero that is neither the minimum nor the maximum leaves no trace, so only
-// an extreme that is a zero (0x7FFF, 0x8000) needs the order of the values.
-__device__ inline bool keys_need_order(const uint32_t (&kmn)[4], const uint32_t (&kmx)[4]) {
-  uint32_t nan = 0xFFFFFFFFu, zero = 0xFFFFFFFFu;
+// A fold's result as keys is exact unless a NaN is among the values, or zeros of both
+// signs are and an extreme is a zero: the first of them is the result then.  A NaN shows
+// in the extremes: its key lies above +inf's (0xFF80) or below -inf's (0x007F).  So may
+// zeros of both signs: the minimum is -0 (0x7FFF) and the maximum not below +0 (0x8000),
+// or the maximum is +0 and the minimum not above -0.
+__device__ inline bool keys_have_nan(const uint32_t (&kmn)[4], const uint32_t (&kmx)[4]) {
+  uint32_t nan = 0xFFFFFFFFu;
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
-    const u16x2_t mn = __builtin_bit_cast(u16x2_t, kmn[q]), mx = __builtin_bit_cast(u16x2_t, kmx[q]);
+    const u16x2_t mx = __builtin_bit_cast(u16x2_t, kmx[q]);
     nan = u16x2_min(nan, u16x2_min(kmn[q], __builtin_bit_cast(uint32_t, mx - (u16x2_t){0xFF81, 0xFF81})));
-    zero = u16x2_min(zero, u16x2_min(__builtin_bit_cast(uint32_t, mn - (u16x2_t){0x7FFF, 0x7FFF}),
-                                     __builtin_bit_cast(uint32_t, mx - (u16x2_t){0x7FFF, 0x7FFF})));
   }
-  return min(nan & 0xFFFFu, nan >> 16) <= 0x7Eu || min(zero & 0xFFFFu, zero >> 16) <= 1u;
+  return min(nan & 0xFFFFu, nan >> 16) <= 0x7Eu;
+}
+__device__ inline bool keys_have_two_zeros(const uint32_t (&kmn)[4], const uint32_t (&kmx)[4]) {
+  uint32_t zeros = 0xFFFFFFFFu;  // a zero half where they may be two
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    zeros = u16x2_min(zeros, u16x2_min((kmx[q] ^ 0x80008000u) | (kmn[q] & 0x80008000u),
+                                       (kmn[q] ^ 0x7FFF7FFFu) | (~kmx[q] & 0x80008000u)));
+  return (zeros & 0xFFFFu) == 0 || (zeros >> 16) == 0;
+}
+
+// 0xFFFF for a value (half of w) that is not a zero, else 0.
+__device__ inline uint32_t nonzero_halves(uint32_t w) {
+  const uint32_t one = u16x2_min(w & 0x7FFF7FFFu, 0x00010001u);
+  return __builtin_bit_cast(uint32_t, (u16x2_t){0, 0} - __builtin_bit_cast(u16x2_t, one));
+}
+// The first zero of each channel, over rows taken last to first: in `first`, where there
+// is one.
+__device__ inline void first_zero(uint32_t (&first)[4], const uint4& v) {
+  const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const uint32_t nz = nonzero_halves(w[q]);
+    first[q] = (first[q] & nz) | (w[q] & ~nz);
+  }
+}
+// The folded extreme `k` (keys, no NaN): a zero is the one that was the extreme before the
+// batch (`before`), else the batch's first.
+__device__ inline uint32_t zero_in_order(uint32_t k, uint32_t before, uint32_t first) {
+  const uint32_t v = bf16x2_unkey(k), o = bf16x2_unkey(before);
+  const uint32_t vnz = nonzero_halves(v), onz = nonzero_halves(o);
+  return bf16x2_key((v & vnz) | (((o & ~onz) | (first & onz)) & ~vnz));
 }
 
 // The wide fold for C = 512 SL (KV*D = 4 x 128 and 8 x 128, bf16): one wave per PPW
@@ -282,13 +312,16 @@ __device__ inline bool keys_need_order(const uint32_t (&kmn)[4], const uint32_t 
 // with one load (lane r: row r of a 64-row chunk; the first chunk of every page of the
 // wave is loaded up front) and reach the row loads through readlane, and the rows fold
 // in order in batches of B loads in flight, as unsigned min / max of monotone 16-bit keys
-// (two channels per instruction); a batch after which an extreme is a NaN or a zero is
-// folded again from the state before it, element by element with torch.minimum / maximum
-// semantics, so ties and NaNs resolve as in a sequential fold.  (Looking for NaNs and
-// zeros in every element instead cost as much as the fold, and one zero in a page - one
-// in a million of normally distributed keys - sent it through the slow fold, 20 us of a
-// wave: 64 rows of 24 layers at KV*D = 512 32 -> 10 us, 16384 rows of 48 layers 173 ->
-// 159 (5.2 TB/s); at KV*D = 1024, against a block per page, 374 -> 317.)  A row outside the buffer is not folded (its load
+// (two channels per instruction); zeros of both signs in the place of an extreme are
+// resolved by their order (first_zero), and a batch with a NaN is folded again from the
+// state before it, element by element with torch.minimum / maximum semantics, so ties and
+// NaNs resolve as in a sequential fold.  (Looking for NaNs and zeros in every element instead cost as much as the fold, and one
+// zero in a page - one in a million of normally distributed keys - sent it through the
+// slow fold, 20 us of a wave: 64 rows of 24 layers at KV*D = 512 32 -> 10 us, 16384 rows
+// of 48 layers 173 -> 159 (5.2 TB/s); at KV*D = 1024, against a block per page, 374 ->
+// 317.  16384 rows of 24 layers in which every batch has zeros as extremes, of one sign 80
+// and 156 us at KV*D = 512 and 1024, as without them, of both signs 90 and 166; folded
+// element by element, as with a NaN, 146 and 360; a block per page 186 at 1024.)  A row outside the buffer is not folded (its load
 // reads row 0).
 template <int SL, int B, int PPW>
 __global__ __launch_bounds__(kPfThreads) void prefill_bounds_wave_kernel(PrefillArgs a) {
@@ -357,14 +390,26 @@ __global__ __launch_bounds__(kPfThreads) void prefill_bounds_wave_kernel(Prefill
             nmx[q] = u16x2_max(nmx[q], kw);
           }
         }
-        if (!__builtin_amdgcn_ballot_w64(keys_need_order(nmn, nmx))) {
+        const bool nan = __builtin_amdgcn_ballot_w64(keys_have_nan(nmn, nmx));  // wave-uniform
+        if (!nan && __builtin_amdgcn_ballot_w64(keys_have_two_zeros(nmn, nmx))) {
+          uint32_t first[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+          for (int i = B - 1; i >= 0; --i)
+            if (ok[i]) first_zero(first, v[i]);
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            nmn[q] = zero_in_order(nmn[q], kmn[q], first[q]);
+            nmx[q] = zero_in_order(nmx[q], kmx[q], first[q]);
+          }
+        }
+        if (!nan) {
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
             kmn[q] = nmn[q];
             kmx[q] = nmx[q];
           }
         } else {
-          // NaNs or zeros: torch.minimum / maximum element by element, in row order
+          // NaNs: torch.minimum / maximum element by element, in row order
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
             const uint32_t bmn = bf16x2_unkey(kmn[q]), bmx = bf16x2_unkey(kmx[q]);
@@ -425,12 +470,14 @@ __global__ __launch_bounds__(kPfThreads) void prefill_bounds_wave_kernel(Prefill
 // of one layer, no LDS and no barrier.  A load instruction reads one row in each of the
 // wave's 64 / L lane groups; group g takes the g-th run of consecutive rows of a chunk of
 // 16 rows per group, all of its loads in flight at once.  The chunk folds as keys, whatever the
-// order; where that does not do (keys_need_order) element by element in each group, and
-// the groups' results fold in group order, which is the rows' order.
+// order; zeros of both signs are then resolved, and with a NaN the chunk is folded element
+// by element, in each group and then over the groups in their order, which is the rows'.
 //
 // Bound: HBM.  16384 rows over 48 layers, against a block per page that folds every
 // element by itself: KV*D = 256 121 -> 76 us (5.4 TB/s), 128 94 -> 36 (5.8 TB/s); 32-row
-// runs at KV*D = 256 take 256 VGPRs and 81 us.
+// runs at KV*D = 256 take 256 VGPRs and 81 us.  Over 24 layers 34 and 20 us, with zeros of
+// both signs as extremes 52 and 31, with a NaN in every chunk 105 and 63, a block per page
+// 57 and 52 whatever the values.
 template <int L>
 __global__ __launch_bounds__(kPfThreads) void prefill_bounds_groups_kernel(PrefillArgs a) {
   constexpr int C = 8 * L, GR = 64 / L, B = 16, CH = B * GR;
@@ -510,7 +557,33 @@ __global__ __launch_bounds__(kPfThreads) void prefill_bounds_groups_kernel(Prefi
         nmx[q] = u16x2_max(nmx[q], (uint32_t)__shfl_xor((int)nmx[q], d, 64));
       }
     }
-    if (!__builtin_amdgcn_ballot_w64(keys_need_order(nmn, nmx))) {
+    const bool nan = __builtin_amdgcn_ballot_w64(keys_have_nan(nmn, nmx));  // wave-uniform
+    if (!nan && __builtin_amdgcn_ballot_w64(keys_have_two_zeros(nmn, nmx))) {
+      uint32_t first[4] = {0u, 0u, 0u, 0u}, none[4];  // this group's rows; none: 0xFFFF without a zero
+#pragma unroll
+      for (int q = 0; q < 4; ++q) none[q] = 0xFFFFFFFFu;
+#pragma unroll
+      for (int i = B - 1; i >= 0; --i) {
+        if (r[i] < 0) continue;
+        first_zero(first, v[i]);
+        const uint32_t w[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
+#pragma unroll
+        for (int q = 0; q < 4; ++q) none[q] &= nonzero_halves(w[q]);
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        uint32_t f = 0u;
+#pragma unroll
+        for (int g = GR - 1; g >= 0; --g) {
+          const uint32_t fg = (uint32_t)__shfl((int)first[q], g * L + sub, 64);
+          const uint32_t ng = (uint32_t)__shfl((int)none[q], g * L + sub, 64);
+          f = (f & ng) | (fg & ~ng);
+        }
+        nmn[q] = zero_in_order(nmn[q], kmn[q], f);
+        nmx[q] = zero_in_order(nmx[q], kmx[q], f);
+      }
+    }
+    if (!nan) {
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         kmn[q] = nmn[q];

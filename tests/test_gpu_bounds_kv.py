@@ -1,4 +1,4 @@
-"""Prefill page bounds at KV*D = 128, 256 and 1024 (1, 2 and 8 KV heads x 128): the wave-per-page
+"""Prefill page bounds at KV*D = 128, 256, 512 and 1024 (1, 2, 4 and 8 KV heads x 128): the wave-per-page
 folds against the per-element fold of the same keys as fp32 (reference quest.py:231-280)."""
 
 from __future__ import annotations
@@ -11,9 +11,9 @@ from tests.test_gpu_quest import DEV, new_quest, rand_bf16
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("kv", [1, 2, 8])
+@pytest.mark.parametrize("kv", [1, 2, 4, 8])
 @pytest.mark.parametrize("page,n", [(64, 0), (64, 1), (64, 63), (64, 777), (16, 100), (32, 65), (128, 333), (200, 777)])
-@pytest.mark.parametrize("kind", ["plain", "special", "bad_rows"])
+@pytest.mark.parametrize("kind", ["plain", "special", "bad_rows", "zeros"])
 def test_prefill_bounds_match_the_per_element_fold(kv, page, n, kind):
     pool = rand_bf16((1100, kv, 128), seed=n + page)
     gen = torch.Generator().manual_seed(kv)
@@ -21,6 +21,20 @@ def test_prefill_bounds_match_the_per_element_fold(kv, page, n, kind):
         bits = pool.view(torch.int16).view(-1)
         for val in (0x7FC0, 0x0000, -0x8000, 0x7F80, 0xFF80 - 65536):
             bits[torch.randint(0, bits.numel(), (60 * kv,), generator=gen)] = val
+    if kind == "zeros":  # by channel: all of one zero, clamped at one, with a few of the other, NaNs
+        x = pool.view(1100, kv * 128)
+        zero, neg = torch.zeros((), dtype=x.dtype), -torch.zeros((), dtype=x.dtype)
+        for c in range(kv * 128):
+            z, other = (zero, neg) if c % 2 else (neg, zero)
+            how = (c // 2) % 8
+            if how == 1:
+                x[:, c] = z
+            elif how in (2, 3, 4):
+                x[:, c] = torch.where((x[:, c] < 0) if how == 2 else (x[:, c] > 0), z, x[:, c])
+            if how in (1, 3) and c % 5 == 0:
+                x[torch.randint(0, 1100, (9,), generator=gen), c] = other
+            if how == 4 and c % 31 == 0:
+                x[torch.randint(0, 1100, (2,), generator=gen), c] = float("nan")
     idx = torch.randperm(1100, generator=gen)[:n].to(torch.int32 if page != 128 else torch.int64)
     if kind == "bad_rows" and n > 3:
         idx[[0, n // 2, n - 1]] = torch.tensor([-1, 5000, 1100], dtype=idx.dtype)
