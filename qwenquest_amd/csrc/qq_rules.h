@@ -30,7 +30,8 @@ constexpr int kUnitParts = 8;  // blocks per (request, KV head), at most: merged
 //    and 50.5);
 //  * more pairs: 4-wave blocks, 3 parts up to 4/3 pairs per CU, then 2, past 8/5 1
 //    (batch 72: 74.3 in 3, 77.1 in 2; batch 84: 81.4 and 83.0; batch 96: 94.7 and 89.6;
-//    batch 104: 102.2 in 2, 96.3 in 1).
+//    batch 104: 102.2 in 2, 96.3 in 1), but no part that leaves the longest wave as many
+//    units (top_k 1024, 2 units a wave in 2 parts and in 3: batch 84 51.4 us in 3, 49.8 in 2).
 // A second round of units in a part is dealt over all parts, not to the first ones
 // (batch 20, 32 units over 24 waves: 32.0 -> 28.5; choosing the order by whether there
 // is a second round costs batch 1 more, 0.04 us a layer, than the order does).
@@ -48,7 +49,8 @@ constexpr UnitShape unit_shape(int64_t cus, int64_t bs, int kv_heads, int top_k)
     if (ceil_of(units, 4 * p4) < ceil_of(units, 8 * p8)) return {4, (int)p4};
     return {8, (int)p8};
   }
-  return {4, (int)least(cap4, 3 * pairs <= 4 * cus ? 3 : 5 * pairs <= 8 * cus ? 2 : 1)};
+  const int64_t parts = least(cap4, 3 * pairs <= 4 * cus ? 3 : 5 * pairs <= 8 * cus ? 2 : 1);
+  return {4, (int)ceil_of(units, 4 * ceil_of(units, 4 * parts))};
 }
 
 // The units of wave `wave` of part `part`: this one, + W * parts, ...

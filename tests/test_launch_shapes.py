@@ -87,6 +87,8 @@ def test_every_unit_belongs_to_one_wave(rules, kv, top_k):
             for wave in range(W):
                 taken += range(rules.unit_first(wave, part, parts), units, parts * W)
         assert sorted(taken) == list(range(units))
+        if bs * kv > CUS:  # a part fewer gives a wave more units
+            assert parts == 1 or ceil_div(units, W * (parts - 1)) > ceil_div(units, W * parts)
         if bs * kv <= CUS:  # one round of resident blocks
             assert bs * kv * parts <= (2 * CUS if W == 4 else CUS)
 
