@@ -338,9 +338,9 @@ int64_t qq_extend_attention_workspace_bytes(int64_t n, int bs, int num_q_heads, 
 /* qq_extend_attention that also reports whether it answers the batch as base.py:65-93's loop
  * does: verdict[0] becomes 0 when every request index lies in its table (from either end) and
  * every request with new tokens has a context and a prefix of no negative length, else 1;
- * verdict[1] is the requests' new tokens.  verdict is pinned host memory of two words (the
- * device writes it as the launch begins; the call sets it to -1 first), to be kept until
- * qq_extend_verdict_wait, on the same stream, has returned.  Not for a captured call. */
+ * verdict[1] is the requests' new tokens.  verdict is two words of pinned host memory, which
+ * the device writes as the launch begins: the call returns when it has (on failure the
+ * words may be written until the stream is done).  Not for a captured call. */
 int qq_extend_attention_checked(const void* q, int num_q_heads, const void* k_layer, const void* v_layer,
                                 int64_t kv_rows, int kv_heads, int head_dim, const int32_t* req_to_token,
                                 int64_t req_to_token_stride, int64_t req_to_token_rows,
@@ -348,7 +348,6 @@ int qq_extend_attention_checked(const void* q, int num_q_heads, const void* k_la
                                 const int64_t* prefix_lens, const int64_t* extend_lens, int bs, int64_t n,
                                 float scale, void* out, void* workspace, int64_t workspace_bytes,
                                 int64_t* verdict, void* stream);
-int qq_extend_verdict_wait(const int64_t* verdict, void* stream);
 
 /* Replaces DenseBackend.forward_decode (src/qwenquest/attention/dense.py:26-42) for
  * one layer: the new tokens' K/V (k_new/v_new [bs, KV, D]; NULL: none) go to rows

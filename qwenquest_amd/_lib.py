@@ -99,7 +99,6 @@ SIGNATURES: dict[str, tuple] = {
         _I,
         [_P, _I, _P, _P, _L, _I, _I, _P, _L, _L, _P, _P, _P, _P, _I, _L, _F, _P, _P, _L, _P, _P],
     ),
-    "qq_extend_verdict_wait": (_I, [_P, _P]),
     "qq_extend_attention_workspace_bytes": (_L, [_L, _I, _I, _I, _L]),
     "qq_kv_scatter": (_I, [_P, _P, _I, _L, _P, _P, _I, _P, _I, _L, _P]),
     "qq_hisparse_swap_in": (
@@ -180,4 +179,6 @@ def dtype_code(dt: torch.dtype) -> int:
 
 
 def stream(device: torch.device | None = None) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    index = device.index if device is not None else None
+    # the handle alone: a Stream object for it costs a call 2 us
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)

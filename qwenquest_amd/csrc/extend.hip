@@ -503,6 +503,22 @@ __global__ __launch_bounds__(256) void extend_merge_kernel(ExtendArgs a) {
 
 using namespace qq;
 
+// Waits for a launch's verdict: it reports as it begins; a stream that is done, or in
+// error, has nothing to wait for.
+static int wait_verdict(const int64_t* verdict, hipStream_t s, const char* what) {
+  for (;;) {
+    for (int spin = 0; spin < 4096; ++spin) {
+      if (__atomic_load_n(verdict, __ATOMIC_ACQUIRE) >= 0) return QQ_OK;
+      __builtin_ia32_pause();
+    }
+    const hipError_t e = hipStreamQuery(s);
+    if (e == hipErrorNotReady) continue;
+    if (e == hipSuccess && __atomic_load_n(verdict, __ATOMIC_ACQUIRE) >= 0) return QQ_OK;
+    set_error(QQ_EHIP, "%s: no verdict: %s", what, hipGetErrorString(e));
+    return QQ_EHIP;
+  }
+}
+
 extern "C" int64_t qq_extend_attention_workspace_bytes(int64_t n, int bs, int num_q_heads, int kv_heads,
                                                        int64_t max_rows) {
   if (n <= 0 || bs <= 0 || kv_heads <= 0 || num_q_heads < kv_heads) return 0;
@@ -520,23 +536,6 @@ extern "C" int qq_extend_attention(const void* q, int num_q_heads, const void* k
   return qq_extend_attention_checked(q, num_q_heads, k_layer, v_layer, kv_rows, kv_heads, head_dim, req_to_token,
                                      req_to_token_stride, req_to_token_rows, req_pool_indices, seq_lens, prefix_lens,
                                      extend_lens, bs, n, scale, out, workspace, workspace_bytes, nullptr, stream);
-}
-
-extern "C" int qq_extend_verdict_wait(const int64_t* verdict, void* stream) {
-  const char* what = "qq_extend_verdict_wait";
-  QQ_REQUIRE(verdict, "%s: null pointer", what);
-  for (;;) {
-    for (int spin = 0; spin < 4096; ++spin) {
-      if (__atomic_load_n(verdict, __ATOMIC_ACQUIRE) >= 0) return QQ_OK;
-      __builtin_ia32_pause();
-    }
-    // the launch reports as it begins; a stream that is done, or in error, has nothing to wait for
-    const hipError_t e = hipStreamQuery(static_cast<hipStream_t>(stream));
-    if (e == hipErrorNotReady) continue;
-    if (e == hipSuccess && __atomic_load_n(verdict, __ATOMIC_ACQUIRE) >= 0) return QQ_OK;
-    set_error(QQ_EHIP, "%s: no verdict: %s", what, hipGetErrorString(e));
-    return QQ_EHIP;
-  }
 }
 
 extern "C" int qq_extend_attention_checked(const void* q, int num_q_heads, const void* k_layer, const void* v_layer,
@@ -595,5 +594,6 @@ extern "C" int qq_extend_attention_checked(const void* q, int num_q_heads, const
   extend_kernel<<<(int)grid, 64 * kExtWaves, kSmem, s>>>(a);
   if (a.splits > 1)
     extend_merge_kernel<<<dim3(a.tiles, kv_heads, kExtRows / 8), 256, 0, s>>>(a);
-  return check_launch(what);
+  const int st = check_launch(what);
+  return st == QQ_OK && verdict ? wait_verdict(verdict, s, what) : st;
 }
