@@ -323,8 +323,9 @@ int qq_quest_layer_step_fused(int q_dtype, int kv_dtype, int new_dtype, int num_
  * 0 .. seq_lens[i]) -> out [n, H*128] bf16.  The lengths are read on the device only.
  * bf16, head_dim 128, H divisible by KV, scale > 0 (QQ_EINVAL otherwise); scores,
  * weights and sums in fp32.  A negative request index or pool row counts from its
- * table's end; a request whose index or a row of which lies outside its table gets NaN,
- * as do rows of q past the requests' tokens.  workspace >=
+ * table's end.  NaN: a request whose index lies outside the table, the query tiles (128 rows
+ * of one KV head's query heads) that attend a row outside the pool, and rows of q past the
+ * requests' tokens.  workspace >=
  * qq_extend_attention_workspace_bytes(n, bs, H, KV, req_to_token_stride): (m, l, o)
  * partials, when few query rows meet a wide table. */
 int qq_extend_attention(const void* q, int num_q_heads, const void* k_layer, const void* v_layer,

@@ -315,14 +315,16 @@ __device__ inline uint32_t zero_in_order(uint32_t k, uint32_t before, uint32_t f
 // (two channels per instruction); zeros of both signs in the place of an extreme are
 // resolved by their order (first_zero), and a batch with a NaN is folded again from the
 // state before it, element by element with torch.minimum / maximum semantics, so ties and
-// NaNs resolve as in a sequential fold.  (Looking for NaNs and zeros in every element instead cost as much as the fold, and one
+// NaNs resolve as in a sequential fold.  A row outside the buffer is not folded (its load
+// reads row 0).
+//
+// Looking for NaNs and zeros in every element instead cost as much as the fold, and one
 // zero in a page - one in a million of normally distributed keys - sent it through the
 // slow fold, 20 us of a wave: 64 rows of 24 layers at KV*D = 512 32 -> 10 us, 16384 rows
-// of 48 layers 173 -> 159 (5.2 TB/s); at KV*D = 1024, against a block per page, 374 ->
-// 317.  16384 rows of 24 layers in which every batch has zeros as extremes, of one sign 80
-// and 156 us at KV*D = 512 and 1024, as without them, of both signs 90 and 166; folded
-// element by element, as with a NaN, 146 and 360; a block per page 186 at 1024.)  A row outside the buffer is not folded (its load
-// reads row 0).
+// of 48 layers 173 -> 157 (5.3 TB/s); at KV*D = 1024, against a block per page, 374 ->
+// 317.  16384 rows of 24 layers in which every batch has zeros as extremes, of one sign: 80
+// and 156 us at KV*D = 512 and 1024, as without them; of both signs 90 and 166; folded
+// element by element, as with a NaN, 189 and 361; a block per page 186 at 1024.
 template <int SL, int B, int PPW>
 __global__ __launch_bounds__(kPfThreads) void prefill_bounds_wave_kernel(PrefillArgs a) {
   constexpr int C = 512 * SL;

@@ -744,7 +744,7 @@ __global__ __launch_bounds__(64 * kDenseWaves, 2) void dense_attend_kernel(StepA
 // ------------------------------------------------------- per-page-unit attention
 // The Quest step's attention (after the score launch; and over given rows for
 // quest_hisparse, so that both compute the same partials in the same order):
-// one 4-wave block per (request, KV head, part), blockIdx = (request, KV head) *
+// one block of W waves per (request, KV head, part), blockIdx = (request, KV head) *
 // parts + part.  The layout's slots come in units of 64 (a selected page, or the
 // recent window, or 64 slots of the dense layout); wave w of part p takes units
 // w*parts + p, w*parts + p + W*parts, ...  (unit_shape).  Per unit a

@@ -23,13 +23,13 @@
 // the other's MFMAs.
 //
 // Bound: the matrix cores.  8192 new tokens behind 8192 cached ones, 32 / 4 heads:
-// 27.5 ms with scaled_dot_product_attention in float32 over gathered rows, 2.8 ms
-// here; with the three value products that is 1180 TFLOP/s of bf16 MFMA, where a
-// library product of 8192^3 reaches 1234 on the card.  (Two pieces per weight take
+// 27.5 ms with scaled_dot_product_attention in float32 over gathered rows, 2.7 to 2.8
+// ms here; with the three value products that is 1180 to 1220 TFLOP/s of bf16 MFMA,
+// where a library product of 8192^3 reaches 1234 on the card.  (Two pieces per weight take
 // 2.2 ms, with an error against float64 that is larger in the fifth digit: the third
 // piece is the weight bits that the general path keeps.)
-// 600 new tokens, where a chain of ten K/V tiles per block is what counts: 25 us of
-// 430.  The products are ordered so that neighbours have different accumulators
+// 600 new tokens, where a chain of ten K/V tiles per block is what counts: 26 us in the
+// kernel, 30 us a call, 430 before.  The products are ordered so that neighbours have different accumulators
 // (2.83 -> 2.78 ms).
 #include <type_traits>
 
@@ -254,7 +254,7 @@ __global__ __launch_bounds__(64 * kExtWaves, 2) void extend_kernel(ExtendArgs a)
   auto load_rows = [&](int j) {
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      rows[i] = rt[min(j * kExtTile + wave * 16 + i * 4 + (lane >> 4), kv_len - 1)];
+      rows[i] = rt[min(j * kExtTile + wave * 16 + i * 4 + (lane >> 4), lim_blk - 1)];  // none past the block's limit
   };
   auto load_tile = [&](int buf) {
     // this wave's 16 tokens of the buffer's K tile (bytes)

@@ -164,9 +164,9 @@ constexpr int extend_request_tiles(int64_t n, int G) { return (int)((n * G + kEx
 
 // K/V splits: as many as give every CU a block when the query tiles do not, one for
 // every kExtMinChunk K/V tiles at most.  The merge costs a launch (6 us), so a grid that
-// covers half the chip stays whole: 600 new tokens (152 blocks) 30.5 us, in two
-// splits 34.6; 8 new tokens behind 8192 (4 blocks) in 32 splits 26.0 us, in 9 of 16
-// tiles 44.9; 64 behind 8192 (16 blocks) in 12 splits 42.2 us, in 25 52.9.  A minimum of 4
+// covers half the chip stays whole.  Us a call: 600 new tokens (152 blocks) 30.5, in two
+// splits 34.6; 8 new tokens behind 8192 (4 blocks) in 32 splits 26.0, in 9 of 16
+// tiles 44.9; 64 behind 8192 (16 blocks) in 12 splits 42.2, in 25 52.9.  A minimum of 4
 // tiles against 8 and 16: 100 new behind 500, one KV head, 21 against 28 us.
 constexpr int extend_splits(int64_t tiles, int KV, int64_t max_rows) {
   const int64_t by_grid = 256 / most(tiles * KV, 1);

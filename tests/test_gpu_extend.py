@@ -322,3 +322,49 @@ def test_infinite_values(new, prefix, width):
         at += n
     rest = [c for c in range(128) if c not in (5, 9, 11)]
     assert torch.equal(got[..., rest], want[..., rest])
+
+
+def test_a_row_outside_the_pool_in_the_new_tokens():
+    """Every token that attends the row gets NaN, and tokens before it keep their answer up to the
+    tile of 128 query rows that holds it."""
+    H, KV, n, at = 32, 4, 600, 300
+    be, q, k, v, batch, layer, slots = make([n, 20], [0, 9], H, KV, 23)
+    want = be.forward_extend(q, k, v, layer, batch)
+    batch.req_to_token_pool.req_to_token[slots[0], at] = 1 << 20
+    got = launch(be, q, batch, layer)
+    tile = 128 // (H // KV)  # tokens of a tile
+    first = at // tile * tile
+    assert torch.equal(got[:first], want[:first]) and torch.equal(got[n:], want[n:])
+    assert bool(got[at:n].isnan().all())
+
+
+def test_threads_on_their_own_streams():
+    """Calls of several threads, some of them refused, each with its own verdict."""
+    import threading
+
+    cases = [make([50 + 30 * i], [10 * i], 8, 2, 30 + i) for i in range(3)]
+    want = [be.forward_extend(q, k, v, layer, batch) for be, q, k, v, batch, layer, _ in cases]
+    torch.cuda.synchronize()
+    wrong = []
+
+    def work(i):
+        be, q, k, v, batch, layer, slots = cases[i]
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for _ in range(30):
+                if not torch.equal(be.forward_extend(q, k, v, layer, batch), want[i]):
+                    wrong.append(i)
+                good, batch.req_pool_indices = batch.req_pool_indices, torch.full((1,), 9, device=DEV)
+                try:
+                    be.forward_extend(q, k, v, layer, batch)
+                    wrong.append(i)
+                except IndexError:
+                    pass
+                batch.req_pool_indices = good
+            torch.cuda.current_stream().synchronize()
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(3)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
