@@ -132,7 +132,7 @@ __device__ inline void attend_unit(int r32, int valid, const uint16_t* kb, const
   mx = fmaxf(mx, lane_xor32(mx, lane));
   const float Mn = fmaxf(M, mx);
   const float alpha = M == -INFINITY ? 0.0f : exp2f(M - Mn);  // rescale of the running sums
-  const float Mb = Mn == -INFINITY ? 0.0f : Mn;  // every score so far -inf: weights of 0, not of NaN
+  const float Mb = fmaxf(Mn, -3.402823466e38f);  // every score so far -inf: weights of 0, not of NaN
   float sum = 0.0f;
   short4_t pa[4];
 #pragma unroll
