@@ -337,11 +337,11 @@ int qq_extend_attention(const void* q, int num_q_heads, const void* k_layer, con
 int64_t qq_extend_attention_workspace_bytes(int64_t n, int bs, int num_q_heads, int kv_heads,
                                             int64_t max_rows);
 /* qq_extend_attention that also reports whether it answers the batch as base.py:65-93's loop
- * does: verdict[0] becomes 0 when every request index lies in its table (from either end) and
- * every request with new tokens has a context and a prefix of no negative length, else 1;
- * verdict[1] is the requests' new tokens.  verdict is two words of pinned host memory, which
- * the device writes as the launch begins: the call returns when it has (on failure the
- * words may be written until the stream is done).  Not for a captured call. */
+ * does: *verdict becomes twice the requests' new tokens when every request index lies in its
+ * table (from either end) and every request with new tokens has a context and a prefix of no
+ * negative length, else 1.  verdict is a word of pinned host memory, which the device writes as
+ * the launch begins: the call returns when it has (on failure the word may be written until
+ * the stream is done).  Not for a captured call. */
 int qq_extend_attention_checked(const void* q, int num_q_heads, const void* k_layer, const void* v_layer,
                                 int64_t kv_rows, int kv_heads, int head_dim, const int32_t* req_to_token,
                                 int64_t req_to_token_stride, int64_t req_to_token_rows,

@@ -105,7 +105,7 @@ def extend_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, prefix_l
 
 # Pinned words for the verdicts of checked prefill launches, as many as calls were ever in
 # flight at once (one per thread): each is taken for one call and is back when the call has read
-# it.  After an error the device may still write its words: they are not used again.
+# it.  After an error the device may still write its word: it is not used again.
 _verdicts: list = []
 
 
@@ -117,7 +117,7 @@ def _extend_launch(
     lens: tuple[torch.Tensor, ...],
     scaling: float,
     checked: bool,
-) -> tuple[torch.Tensor, list[int] | None]:
+) -> tuple[torch.Tensor, int | None]:
     """qq_extend_attention; the output, and the verdict on the lengths if asked for."""
     n, heads, dim = q.shape
     kv, bs, dev = k_buf.shape[1], int(lens[0].shape[0]), q.device
@@ -145,9 +145,9 @@ def _extend_launch(
     try:
         verdict = _verdicts.pop()
     except IndexError:
-        verdict = torch.empty(2, dtype=torch.int64, pin_memory=True).numpy()
+        verdict = torch.empty(1, dtype=torch.int64, pin_memory=True).numpy()
     _lib.call("qq_extend_attention_checked", *args, verdict.ctypes.data, stream)
-    found = verdict.tolist()
+    found = int(verdict[0])
     _verdicts.append(verdict)
     return out, found
 
@@ -191,7 +191,7 @@ def extend_attention_batch_checked(
     without a verdict; by a launch of its own 40, with an event 43, by a copy of the lengths 52)."""
     lens = (req_pool_indices, seq_lens, prefix_lens, extend_lens)
     out, verdict = _extend_launch(q, k_buf, v_buf, req_to_token, lens, scaling, True)
-    irregular, total = verdict
-    if irregular:
+    if verdict == 1:
         return None
-    return out if total >= out.shape[0] else out[:total]
+    tokens = verdict // 2
+    return out if tokens >= out.shape[0] else out[:tokens]

@@ -141,8 +141,8 @@ __device__ inline ExtendTile find_tile(const ExtendArgs& a, int t) {
   return {-1, 0, tok, 0, t - tile, -1, 0, 0};
 }
 
-// qq_extend_attention_checked's verdict, by one wave: host memory, so the words go out at
-// system scope, the one that the host waits for last.
+// qq_extend_attention_checked's verdict, by one wave: one word of host memory, stored at
+// system scope (nothing else is handed over with it, so no cache is written back).
 __device__ inline void report_lengths(const ExtendArgs& a) {
   const int lane = threadIdx.x & 63;
   int64_t total = 0;
@@ -155,9 +155,8 @@ __device__ inline void report_lengths(const ExtendArgs& a) {
 #pragma unroll
   for (int d = 32; d >= 1; d >>= 1) total += __shfl_xor((long long)total, d, 64);
   const bool any = __any(irregular);
-  if (lane != 0) return;
-  __hip_atomic_store(a.verdict + 1, total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-  __hip_atomic_store(a.verdict, any ? 1 : 0, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  if (lane == 0)
+    __hip_atomic_store(a.verdict, any ? 1 : total * 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 __device__ inline uint32_t pack_hi16(float even, float odd) {  // the high halves: truncation to bf16
@@ -554,7 +553,7 @@ extern "C" int qq_extend_attention_checked(const void* q, int num_q_heads, const
                  req_to_token_stride < (int64_t)1 << 30 && kv_rows > 0 &&
                  req_to_token_rows < (int64_t)1 << 31,
              "%s: bad sizes", what);
-  if (verdict) verdict[0] = verdict[1] = bs == 0 || n == 0 ? 0 : -1;
+  if (verdict) *verdict = bs == 0 || n == 0 ? 0 : -1;
   if (bs == 0 || n == 0) return QQ_OK;
   QQ_REQUIRE(q && k_layer && v_layer && req_to_token && req_pool_indices && seq_lens && prefix_lens &&
                  extend_lens && out, "%s: null pointer", what);
