@@ -186,7 +186,7 @@ def extend_attention_batch_checked(
     """``extend_attention_batch`` outside a graph capture: the requests' rows only, and None for a
     batch that the loop treats in another way (or refuses).
 
-    The launch judges the lengths as it begins and the host waits for that, not for its end: the
+    The launch looks at the lengths as it begins and the host waits for that, not for its end: the
     device is not left idle, and no copy, event or launch is queued (600 new tokens 30 us, 29
     without a verdict; by a launch of its own 40, with an event 43, by a copy of the lengths 52)."""
     lens = (req_pool_indices, seq_lens, prefix_lens, extend_lens)
